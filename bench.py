@@ -451,6 +451,11 @@ def roofline(workload: str, plan: dict, n: int, m: int, kernel_s: float, npdu: b
                exchanges_per_launch=exchanges, exchange_floor_us=round(floor_us, 4),
                us_per_exchange=round(kernel_s * 1e6 / exchanges, 4),
                floor_probe={"grid": grid, "words": words, "threads": 1024})
+    if kind == "rounds":
+        out["note"] = ("threshold rounds: one exchange settles many picks, and a round's own work (the "
+                       "update, sorting the candidates, deciding the picks) takes longer than the "
+                       "exchange that the floor counts")
+        out["picks_per_exchange"] = round(m / exchanges, 1)
     if kind in ("spruned", "spair"):
         out["note"] = ("the floor is the exchange alone; a streamed round also waits for the memory "
                        "round trip of its listed blocks (a paired round for two: the update's, then "
@@ -698,7 +703,7 @@ def run_sweep(args) -> dict:
         d_pts = D.DeviceArray.from_numpy(np.ascontiguousarray(pc.T))
         d_start = D.DeviceArray.from_numpy(np.zeros(1, np.uint64))
         d_out = D.DeviceArray((m,), np.uint64)
-        plan = D.plan_info(n, 3, n_samples=m)
+        plan = D.call_info(n, 3, n_samples=m)
         for _ in range(2):
             D.fps_sampling_device(d_pts, n, 3, m, d_start, 1, d_out)
         D.synchronize()
@@ -818,7 +823,7 @@ def main() -> int:
     elif kdline:
         import fpsample_amd as F
 
-        plan = dict(D.plan_info(n, 3, tie=D.TIE_LOWEST, n_samples=m), tie="lowest",
+        plan = dict(D.call_info(n, 3, tie=D.TIE_LOWEST, n_samples=m), tie="lowest",
                     h=wl["h"])
         host_out = [None]
 
@@ -829,7 +834,7 @@ def main() -> int:
         d_pts = D.DeviceArray.from_numpy(soa)
         if args.autotune == "on":
             D.autotune(d_pts, 1, n, n, 3, passes=m)  # untimed: picks the plan for this cloud
-        plan = D.plan_info(n, 3, n_samples=m)
+        plan = D.call_info(n, 3, n_samples=m)
 
         def step():
             D.fps_sampling_device(d_pts, n, 3, m, d_start, 1, d_out)

@@ -1,0 +1,45 @@
+// fps_rounds.hpp -- host-visible description of the threshold-round FPS kernel.
+#pragma once
+#include <hip/hip_runtime.h>
+#include <stddef.h>
+#include <stdint.h>
+
+#include "fps_kernels.hpp"
+
+namespace fpsx {
+
+struct RoundsParams {
+  FpsParams fps;       // the cloud (original order), picks, exchange area, status, dmin
+  const float *pos;    // coordinate j of position p at pos[p * pos_sp + j * pos_ld]
+  uint64_t pos_sp;
+  uint64_t pos_ld;
+  const uint32_t *perm;  // original index of every position; null: the identity
+  uint32_t nblocks;      // blocks of 64 * P consecutive positions
+  uint32_t cap_wg;       // candidates one workgroup may publish per round
+  uint32_t target;       // candidates aimed at per round
+};
+
+constexpr int kRoundsThreads = 1024;
+constexpr uint32_t kRoundsCap = 256;       // candidates of one round
+constexpr uint32_t kRoundsTarget = 160;    // candidates aimed at
+constexpr uint32_t kRoundsMaxGrid = 256;
+constexpr uint32_t kRoundsHeadWords = 3;   // count, high and low half of the best key
+constexpr uint32_t kRoundsReplicas = 4;    // copies of the headers
+// Candidates one workgroup may publish: the area stays small enough to clear.
+inline uint32_t rounds_cap_wg(uint32_t grid) {
+  return grid <= 8 ? kRoundsCap : grid <= 64 ? 64 : 32;
+}
+// Exchange words of a grid: two buffers of headers and candidates.
+inline size_t rounds_xchg_words(uint32_t grid, uint32_t dim) {
+  if (grid <= 1) return 1;
+  return (size_t)2 * ((size_t)kRoundsReplicas * kRoundsHeadWords * kRoundsMaxGrid +
+                      (size_t)(2 + dim) * grid * rounds_cap_wg(grid));
+}
+// Dynamic LDS of a workgroup holding nbl blocks: box and best key of each.
+inline size_t rounds_shmem(uint32_t dim, uint32_t nbl) {
+  return (size_t)nbl * (2 * dim * sizeof(float) + sizeof(uint64_t));
+}
+
+const KernelEntry *rounds_table(size_t *count);
+
+}  // namespace fpsx

@@ -24,6 +24,7 @@
 #include "fps_kernels.hpp"
 #include "fps_npdu.hpp"
 #include "fps_pruned.hpp"
+#include "fps_rounds.hpp"
 #include "fpsx.h"
 #include "fpsx_internal.hpp"
 #include "kdline.hpp"
@@ -398,6 +399,65 @@ int plan(Ctx &c, size_t n, size_t dim, int tie, size_t m, Plan &p) {
   return plan_stream(c, n, dim, tie, 1024, 0, false, p);
 }
 
+// Threshold-round plan.  FPSX_ROUNDS="P:G[:target[:order]]" overrides: points per lane,
+// workgroups (0: the rules below), candidates aimed at per round, spatial order (0 or 1).
+//   P: a workgroup's 16 waves take a block of 64 * P points each.  Small blocks have tight
+//   boxes and spread a pick's work; large ones need fewer box tests.  Kernel ms at 64
+//   workgroups (gauss1m: 128): uniform 50 K / 4096 picks 0.83 at P = 1, 0.87 at 4, 1.09 at 8
+//   (its 98 blocks fill 6 workgroups); uniform 100 K / 50 K picks 4.53, 4.52 and 5.58;
+//   gauss1m / 16384 picks 2.74 at 4, 2.67 at 8.
+//   G: gauss1m 3.58, 2.94, 2.67 and 2.80 ms at 32, 64, 128 and 256; the 16.7 M-point lattice
+//   7.45, 5.41 and 4.48 ms at 64, 128 and 256 (early rounds sweep the whole cloud).
+static int plan_rounds(Ctx &c, size_t n, size_t dim, int tie, Plan &p) {
+  int P = 0, G = 0, target = 0, order = -1;
+  if (const char *env = std::getenv("FPSX_ROUNDS"))
+    if (*env) std::sscanf(env, "%d:%d:%d:%d", &P, &G, &target, &order);
+  if (P <= 0) P = n <= 65536 ? 1 : n <= 524288 ? 4 : 8;
+  size_t cnt;
+  const KernelEntry *t = rounds_table(&cnt);
+  const KernelEntry *k = nullptr;
+  for (size_t i = 0; i < cnt; ++i)
+    if (t[i].dim == (int)dim && t[i].tie == tie && t[i].ppt == P) k = &t[i];
+  if (!k) return fail(FPSX_EINVAL, "no threshold-round kernel for dim " + std::to_string(dim) +
+                                       " with " + std::to_string(P) + " points per lane");
+  const size_t nblocks = (n + 64 * (size_t)P - 1) / (64 * (size_t)P);
+  size_t g = G > 0 ? (size_t)G : n <= 524288 ? 64 : n <= ((size_t)1 << 22) ? 128 : 256;
+  g = std::min<size_t>(std::min<size_t>(g, nblocks), kRoundsMaxGrid);
+  const size_t nbl = (nblocks + g - 1) / g;
+  const size_t shmem = rounds_shmem((uint32_t)dim, (uint32_t)nbl);
+  if (shmem > 96 * 1024) return fail(FPSX_ETOOBIG, "threshold rounds: too many blocks per workgroup");
+  if (g > (size_t)c.max_blocks(k, shmem))
+    return fail(FPSX_ETOOBIG, "threshold rounds: grid exceeds co-residency");
+  p.kind = PlanKind::Rounds;
+  p.k = k;
+  p.block = kRoundsThreads;
+  p.grid = (uint32_t)g;
+  p.chunk = (uint32_t)(nbl * 64 * P);
+  p.shmem = shmem;
+  p.target = target > 0 ? std::min<uint32_t>((uint32_t)target, kRoundsCap) : kRoundsTarget;
+  p.order = order >= 0 ? order != 0 : n > 4096;
+  return FPSX_OK;
+}
+
+static bool env_set(const char *name) {
+  const char *v = std::getenv(name);
+  return v && *v && std::strcmp(v, "0") != 0;
+}
+
+// Threshold rounds from 4096 points (1024 points, 256 picks: 274 us a call against 232 us by
+// the one-workgroup pass kernel; 4096 points, 1024 picks: 469 against 881 us), unless a pass
+// plan is asked for by name or by the tuner.
+int plan_call(Ctx &c, size_t n, size_t dim, int tie, size_t m, Plan &p) {
+  const bool passes = env_set("FPSX_PLAN") || env_set("FPSX_NO_PAIR") || env_set("FPSX_NO_PRUNE") ||
+                      env_set("FPSX_NO_ROUNDS") ||
+                      c.tuned.find(std::make_tuple(n, dim, tie)) != c.tuned.end();
+  if (!passes && (env_set("FPSX_ROUNDS") || (n >= 4096 && m >= 64)) &&
+      plan_rounds(c, n, dim, tie, p) == FPSX_OK)
+    return FPSX_OK;
+  t_err.clear();
+  return plan(c, n, dim, tie, m, p);
+}
+
 static const KernelEntry *find_npdu(int dim, int B, int ppt) {
   size_t cnt;
   const KernelEntry *t = npdu_table(&cnt);
@@ -553,13 +613,15 @@ int plan_npdu(Ctx &c, size_t n, size_t dim, Plan &p) {
 }
 
 // Candidate plans the tuner times for a cloud of n points and m samples:
-// the planner's own choice, every feasible resident shape of this dimension,
+// the planner's own choice, the threshold rounds, every feasible resident shape of this dimension,
 // for 3-D clouds every feasible pruned and paired shape and the streaming
 // pruned plan, and the streaming kernel at two block sizes.
 static std::vector<Plan> candidates(Ctx &c, size_t n, size_t dim, int tie, size_t m) {
   std::vector<Plan> out;
   Plan q;
   if (plan(c, n, dim, tie, m, q) == FPSX_OK) out.push_back(q);
+  if (plan_rounds(c, n, dim, tie, q) == FPSX_OK) out.push_back(q);
+  q = Plan();
   size_t cnt;
   const KernelEntry *t = resident_table(&cnt);
   for (size_t i = 0; i < cnt; ++i) {
@@ -607,7 +669,7 @@ static std::vector<Plan> candidates(Ctx &c, size_t n, size_t dim, int tie, size_
 static int common_params(Ctx &c, const float *d_pts, size_t sp, size_t ld, size_t n, size_t dim,
                          size_t m, const uint64_t *d_starts, size_t n_starts, uint64_t *d_out,
                          float *d_out_pts, float init, uint32_t chunk, hipStream_t st,
-                         FpsParams &a) {
+                         FpsParams &a, size_t words = 0) {
   // Exchange tuning knobs (read per launch so a tuner can vary them).
   const char *rep_env = std::getenv("FPSX_XCHG_REPLICAS");
   const char *bo_env = std::getenv("FPSX_XCHG_BACKOFF");
@@ -617,7 +679,7 @@ static int common_params(Ctx &c, const float *d_pts, size_t sp, size_t ld, size_
   c.backoff = bo_env ? std::atoi(bo_env) : 0;
   if (c.backoff < 0) c.backoff = 0;
   const uint32_t reps = (uint32_t)c.replicas;
-  const size_t xwords = xchg_words(reps);
+  const size_t xwords = words ? words : xchg_words(reps);
   HIP_TRY(c.xchg.reserve(xwords * sizeof(uint64_t)));
   HIP_TRY(c.status.reserve(sizeof(uint64_t)));
   HIP_TRY(launch_fill_u64((uint64_t *)c.xchg.p, xwords, 0, st));
@@ -690,8 +752,41 @@ int launch_fps(Ctx &c, const Plan &p, const float *d_pts, size_t sp, size_t ld, 
   }
   FpsParams a;
   rc = common_params(c, d_pts, sp, ld, n, dim, m, d_starts, n_starts, d_out, d_out_pts, init,
-                     p.chunk, st, a);
+                     p.chunk, st, a,
+                     p.kind == PlanKind::Rounds ? rounds_xchg_words(p.grid, (uint32_t)dim) : 0);
   if (rc) return rc;
+  RoundsParams ra;
+  if (p.kind == PlanKind::Rounds) {
+    HIP_TRY(c.dmin.reserve(n * sizeof(float)));
+    a.dmin = (float *)c.dmin.p;
+    const uint32_t block = (uint32_t)(64 * p.k->ppt);
+    ra.fps = a;
+    ra.pos = d_pts;
+    ra.pos_sp = sp;
+    ra.pos_ld = ld;
+    ra.perm = nullptr;
+    ra.nblocks = (uint32_t)((n + block - 1) / block);
+    ra.cap_wg = rounds_cap_wg(p.grid);
+    ra.target = p.target;
+    if (p.order) {
+      HIP_TRY(c.sorted.reserve(n * 3 * sizeof(float)));
+      HIP_TRY(c.perm.reserve(n * sizeof(uint32_t)));
+      if (!c.spatial) c.spatial = new_spatial_scratch();
+      rc = spatial_order(d_pts, sp, ld, (uint32_t)n, block, (float *)c.sorted.p,
+                         (uint32_t *)c.perm.p, *c.spatial, st);
+      if (rc) return rc;
+      ra.pos = (const float *)c.sorted.p;
+      ra.pos_sp = 1;
+      ra.pos_ld = n;
+      ra.perm = (const uint32_t *)c.perm.p;
+    }
+    rc = dispatch(c, p, &ra, st);
+    if (rc) return rc;
+    c.last_plan = p;
+    c.last_m = m;
+    c.last_starts = n_starts;
+    return scratch_release(c, st);
+  }
   if (p.kind == PlanKind::Stream) {
     HIP_TRY(c.dmin.reserve(n * sizeof(float)));
     a.dmin = (float *)c.dmin.p;
@@ -790,7 +885,7 @@ int fps_host(const float *points, size_t n, size_t dim, int layout, size_t m,
   Ctx &c = *cp;
   std::lock_guard<std::mutex> lk(c.mu);
   Plan p;
-  rc = plan(c, n, dim, tie, m, p);
+  rc = plan_call(c, n, dim, tie, m, p);
   if (rc) return rc;
   hipStream_t st = c.stream;
   rc = scratch_acquire(c, st);
@@ -877,7 +972,7 @@ FPSX_EXPORT int fpsx_fps_sampling_device_strided(const float *d_points, size_t s
   Ctx &c = *cp;
   std::lock_guard<std::mutex> lk(c.mu);
   Plan p;
-  rc = plan(c, n_points, dim, tie, n_samples, p);
+  rc = plan_call(c, n_points, dim, tie, n_samples, p);
   if (rc) return rc;
   hipStream_t st = stream ? (hipStream_t)stream : c.stream;
   return launch_fps(c, p, d_points, stride_point, stride_dim, n_points, dim, n_samples, d_start,
@@ -995,7 +1090,7 @@ FPSX_EXPORT int fpsx_launch_exchanges(void *stream, uint64_t *exchanges) {
   const bool paired_npdu = c.last_plan.kind == PlanKind::Npdu && c.last_plan.k >= npdu_pair &&
                            c.last_plan.k < npdu_pair + npdu_pairs;
   if (c.last_plan.kind != PlanKind::Pair && c.last_plan.kind != PlanKind::StreamPair &&
-      !paired_npdu) {
+      c.last_plan.kind != PlanKind::Rounds && !paired_npdu) {
     // One exchange per pick after the forced prefix.
     *exchanges = c.last_m > c.last_starts ? c.last_m - c.last_starts : 0;
     return FPSX_OK;
@@ -1033,8 +1128,8 @@ FPSX_EXPORT int fpsx_device_status(void *stream) {
   return status_code(*c.host_status);
 }
 
-FPSX_EXPORT int fpsx_plan_info(size_t n_points, size_t dim, int tie, size_t n_samples, int *kind,
-                               int *block, int *ppt, int *grid, int *chunk) {
+static int report_plan(bool call, size_t n_points, size_t dim, int tie, size_t n_samples, int *kind,
+                       int *block, int *ppt, int *grid, int *chunk) {
   t_err.clear();
   Ctx *cp = nullptr;
   int rc = get_ctx(&cp);
@@ -1042,7 +1137,8 @@ FPSX_EXPORT int fpsx_plan_info(size_t n_points, size_t dim, int tie, size_t n_sa
   Ctx &c = *cp;
   std::lock_guard<std::mutex> lk(c.mu);
   Plan p;
-  rc = plan(c, n_points, dim, tie, n_samples, p);
+  rc = call ? plan_call(c, n_points, dim, tie, n_samples, p)
+            : plan(c, n_points, dim, tie, n_samples, p);
   if (rc) return rc;
   if (kind) *kind = (int)p.kind;
   if (block) *block = (int)p.block;
@@ -1050,6 +1146,16 @@ FPSX_EXPORT int fpsx_plan_info(size_t n_points, size_t dim, int tie, size_t n_sa
   if (grid) *grid = (int)p.grid;
   if (chunk) *chunk = (int)p.chunk;
   return FPSX_OK;
+}
+
+FPSX_EXPORT int fpsx_plan_info(size_t n_points, size_t dim, int tie, size_t n_samples, int *kind,
+                               int *block, int *ppt, int *grid, int *chunk) {
+  return report_plan(false, n_points, dim, tie, n_samples, kind, block, ppt, grid, chunk);
+}
+
+FPSX_EXPORT int fpsx_call_info(size_t n_points, size_t dim, int tie, size_t n_samples, int *kind,
+                               int *block, int *ppt, int *grid, int *chunk) {
+  return report_plan(true, n_points, dim, tie, n_samples, kind, block, ppt, grid, chunk);
 }
 
 FPSX_EXPORT int fpsx_autotune(const float *d_points, size_t stride_point, size_t stride_dim,

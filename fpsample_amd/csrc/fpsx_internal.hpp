@@ -28,7 +28,8 @@ struct DevBuf {
 };
 
 enum class PlanKind : int {
-  Resident = 0, Stream = 1, Pruned = 2, Npdu = 3, StreamPruned = 4, Pair = 5, StreamPair = 6
+  Resident = 0, Stream = 1, Pruned = 2, Npdu = 3, StreamPruned = 4, Pair = 5, StreamPair = 6,
+  Rounds = 7
 };
 
 struct Plan {
@@ -38,6 +39,8 @@ struct Plan {
   uint32_t grid = 0;
   uint32_t chunk = 0;  // points per workgroup
   size_t shmem = 0;    // dynamic LDS bytes
+  uint32_t target = 0;   // threshold rounds: candidates aimed at per round
+  bool order = false;    // threshold rounds: points in spatial order
 };
 
 // One per device, created on first use and kept until the process ends.
@@ -149,6 +152,8 @@ int fail(int code, const std::string &msg);
 int get_ctx(Ctx **out);
 // Kernel and grid for a cloud of n points of dimension dim and m samples.
 int plan(Ctx &c, size_t n, size_t dim, int tie, size_t m, Plan &p);
+// What a call runs: the threshold rounds where they serve, else plan()'s pass kernel.
+int plan_call(Ctx &c, size_t n, size_t dim, int tie, size_t m, Plan &p);
 // Enqueue one FPS run on device data: coordinate j of point i at
 // d_pts[i*sp + j*ld].  d_out_pts (may be null) receives the picks' coordinates.
 int launch_fps(Ctx &c, const Plan &p, const float *d_pts, size_t sp, size_t ld, size_t n,

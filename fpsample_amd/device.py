@@ -82,6 +82,7 @@ def lib() -> ctypes.CDLL:
         L.fpsx_timing_read.argtypes = [ctypes.POINTER(ctypes.c_double), ctypes.POINTER(ctypes.c_int)]
         ip = ctypes.POINTER(ctypes.c_int)
         L.fpsx_plan_info.argtypes = [sz, sz, ctypes.c_int, sz, ip, ip, ip, ip, ip]
+        L.fpsx_call_info.argtypes = [sz, sz, ctypes.c_int, sz, ip, ip, ip, ip, ip]
         L.fpsx_fps_npdu_sampling_device.argtypes = [vp, sz, sz, sz, sz, sz, sz, vp, vp, vp, vp]
         L.fpsx_fps_npdu_sampling_device.restype = ctypes.c_int
         L.fpsx_npdu_plan_info.argtypes = [sz, sz, ip, ip, ip, ip]
@@ -411,11 +412,21 @@ def timing_read():
     return ms.value, n.value
 
 
-def plan_info(n_points: int, dim: int, tie: int = TIE_HIGHEST, n_samples: int = 0) -> dict:
-    """The launch the planner picks (n_samples 0: as for a short run)."""
+_KINDS = ("resident", "stream", "pruned", "npdu", "spruned", "pair", "spair", "rounds")
+
+
+def _info(entry, name: str, n_points: int, dim: int, tie: int, n_samples: int) -> dict:
     v = [ctypes.c_int() for _ in range(5)]
-    _raise(lib().fpsx_plan_info(n_points, dim, tie, n_samples, *[ctypes.byref(x) for x in v]),
-           "fpsx_plan_info")
+    _raise(entry(n_points, dim, tie, n_samples, *[ctypes.byref(x) for x in v]), name)
     kind, block, ppt, grid, chunk = (x.value for x in v)
-    return dict(kind=("resident", "stream", "pruned", "npdu", "spruned", "pair", "spair")[kind], block=block, ppt=ppt, grid=grid,
-                chunk=chunk)
+    return dict(kind=_KINDS[kind], block=block, ppt=ppt, grid=grid, chunk=chunk)
+
+
+def plan_info(n_points: int, dim: int, tie: int = TIE_HIGHEST, n_samples: int = 0) -> dict:
+    """The pass kernel the planner picks (n_samples 0: as for a short run)."""
+    return _info(lib().fpsx_plan_info, "fpsx_plan_info", n_points, dim, tie, n_samples)
+
+
+def call_info(n_points: int, dim: int, tie: int = TIE_HIGHEST, n_samples: int = 0) -> dict:
+    """What a call of that size runs: threshold rounds, or plan_info's kernel."""
+    return _info(lib().fpsx_call_info, "fpsx_call_info", n_points, dim, tie, n_samples)

@@ -71,8 +71,9 @@ int fpsx_device_status(void *stream);
 void *fpsx_stream(void);
 
 /*
- * The launch the planner picks for a cloud of n_points x dim and n_samples
- * picks under `tie`: kind 0 = register-resident, 1 = HBM-streaming,
+ * The pass kernel the planner picks for a cloud of n_points x dim and n_samples
+ * picks under `tie` (what a call runs when it does not take the threshold
+ * rounds, see fpsx_call_info): kind 0 = register-resident, 1 = HBM-streaming,
  * 2 = register-resident with spatial order and per-wave pruning,
  * 4 = HBM-streaming with spatial order and per-block pruning,
  * 5 = kind 2 settling up to two picks per cross-workgroup exchange (2..256
@@ -91,6 +92,19 @@ void *fpsx_stream(void);
  * kinds 5 and 6.
  */
 int fpsx_plan_info(size_t n_points, size_t dim, int tie, size_t n_samples, int *kind, int *block,
+                   int *ppt, int *grid, int *chunk);
+
+/*
+ * What a call of that size runs: kind 7 = threshold rounds (many picks per
+ * exchange; threads per workgroup, points per lane of a block, workgroups,
+ * points per workgroup), else as fpsx_plan_info.  The rounds give way to the
+ * pass kernels under FPSX_PLAN, FPSX_NO_PAIR=1, FPSX_NO_PRUNE=1,
+ * FPSX_NO_ROUNDS=1, or a tuned plan that is a pass kernel; FPSX_ROUNDS=
+ * "P:G[:target[:order]]" sets their shape (points per lane, workgroups,
+ * candidates aimed at per round, spatial order 0 or 1) and takes them at any
+ * size.  The picks are the same either way.
+ */
+int fpsx_call_info(size_t n_points, size_t dim, int tie, size_t n_samples, int *kind, int *block,
                    int *ppt, int *grid, int *chunk);
 
 /*
@@ -125,7 +139,7 @@ int fpsx_exchange_timeout(double seconds);
  * rounds, one barrier each), one per pick after the forced prefix for the
  * one-pick kernels, counted by the kernel for the paired kinds and the paired
  * windowed-update kernel (up to two picks per exchange; kind 5 also exchanges
- * workgroup boxes once).  Measurement aid; no counterpart in the reference.
+ * workgroup boxes once) and, as rounds, for kind 7.  Measurement aid; no counterpart in the reference.
  */
 int fpsx_launch_exchanges(void *stream, uint64_t *exchanges);
 

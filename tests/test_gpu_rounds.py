@@ -1,0 +1,93 @@
+"""GPU tests of the threshold rounds: every pick against the oracle at the sizes where the
+blocks, the candidate lists and the bound can go wrong.  Picks are indices: they are equal."""
+import os
+
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def log(msg):
+    print(msg, flush=True)
+
+
+@pytest.fixture
+def rounds_env(monkeypatch):
+    def set_(value):
+        monkeypatch.setenv("FPSX_ROUNDS", value)
+    return set_
+
+
+def run(pc, m, starts, lowest=False):
+    """(picks, their coordinates) by the device entry, row-major points in place."""
+    from fpsample_amd import device as D
+
+    n, d = pc.shape
+    st = np.atleast_1d(np.asarray(starts, np.uint64))
+    rows, ds = D.DeviceArray.from_numpy(pc), D.DeviceArray.from_numpy(st)
+    out, pts = D.DeviceArray((m,), np.uint64), D.DeviceArray((m, d), np.float32)
+    tie = D.TIE_LOWEST if lowest else D.TIE_HIGHEST
+    init = float(np.finfo(np.float32).max) if lowest else float("inf")
+    assert D.call_info(n, d, tie=tie, n_samples=m)["kind"] == "rounds"
+    D.fps_sampling_device_strided(rows, d, 1, n, d, m, ds, st.size, out, pts, tie=tie, init=init)
+    D.device_status()
+    return out.numpy(), pts.numpy()
+
+
+def check(pc, m, starts, name):
+    log(f"rounds {name} n={len(pc)} d={pc.shape[1]} m={m} env={os.environ.get('FPSX_ROUNDS')}")
+    got, pts = run(pc, m, starts)
+    want = O.fps(pc, m, starts)
+    np.testing.assert_array_equal(got, want, err_msg=name)
+    np.testing.assert_array_equal(pts, pc[want.astype(np.int64)], err_msg=name + " coordinates")
+    if np.size(starts) == 1:
+        got, _ = run(pc, m, starts, lowest=True)
+        want = O.fps_ex(pc, m, int(starts), lowest=True, init=float(np.finfo(np.float32).max))
+        np.testing.assert_array_equal(got, want, err_msg=name + " lowest")
+
+
+# Points per lane : workgroups, with and without spatial order.
+SHAPES = ["1:1", "1:3", "1:64:160:1", "1:200", "4:5", "4:64:256:0", "8:2:1", "8:16"]
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+def test_rounds_block_edges(gpu, rounds_env, shape):
+    # Around whole blocks of 64, 256 and 512 points and the smallest clouds.
+    rounds_env(shape)
+    rng = np.random.default_rng(60)
+    for n, m in ((1, 1), (2, 2), (63, 63), (64, 40), (65, 65), (257, 100), (511, 300), (513, 513),
+                 (4097, 700)):
+        check(rng.random((n, 3)).astype(np.float32), m, int(rng.integers(n)), "edge")
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+def test_rounds_ties_special_values_and_prefixes(gpu, rounds_env, shape):
+    # Far more equal distances than a round's candidates, duplicates to the last pick (the
+    # best key stays), NaN and infinite coordinates, squares that overflow, and forced
+    # prefixes below, at and beyond the 256 picks a round can hold.
+    rounds_env(shape)
+    rng = np.random.default_rng(61)
+    check(rng.integers(0, 24, (9000, 3)).astype(np.float32), 3000, 5, "lattice")
+    check(np.repeat(rng.integers(0, 5, (700, 3)), 3, axis=0).astype(np.float32), 2100, 7, "dups")
+    check(np.ones((3000, 3), np.float32), 400, 11, "same")
+    sp = (rng.random((5000, 3)) * 4e19).astype(np.float32)
+    sp[9] = np.inf
+    sp[10, 1] = -np.inf
+    check(sp, 500, 0, "overflow")
+    sp[[5, 700, 4000]] = np.nan
+    check(sp, 500, 0, "nan")
+    check((rng.random((5000, 3)) * 1e-21).astype(np.float32), 500, 3, "denormal")
+    pc = rng.random((6000, 3)).astype(np.float32)
+    for count in (2, 255, 256, 257, 700):
+        check(pc, 700, [int(v) for v in rng.integers(0, 6000, count)], f"prefix {count}")
+
+
+def test_rounds_planner_sizes(gpu):
+    # The planner's own shapes on both sides of each of its lines.
+    rng = np.random.default_rng(62)
+    for n, m in ((4096, 64), (65536, 1500), (65537, 1500), (524288, 600), (524289, 600),
+                 ((1 << 22) + 1, 100)):
+        check(rng.random((n, 3)).astype(np.float32), m, int(rng.integers(n)), "planner")
