@@ -19,7 +19,14 @@
 // Keys are total (the index breaks ties), so steps below one value work through any number
 // of equal distances.
 //
-// A cloud of 2^20 clustered points settles about 130 picks per round of 256 candidates.
+// What bounds it: a round's serial chain, not bytes (2^20 clustered points, 16384 picks, 128
+// workgroups: 224 rounds of 9.5 us).  Of a round (100 K points, 64 workgroups, 363 rounds of
+// 9.5 us): update 2.2 us with the wait for the slowest wave, exchange 2.9, sorting 1.4, rows
+// 1.9 (the vector ALUs are busy throughout: 10 instructions for 64 pairs), settling 0.4, the
+// bound and the picks 1.1.  Settling the candidates one by one instead took 450 ns a pick.
+// A block per wave in registers, the candidates loaded beside the headers and the best 256
+// taken from up to 512 brought gauss1m from 2.67 to 2.13 ms, 100 K / 50 K picks from 4.52 to
+// 3.44 ms.
 #include "fps_rounds.hpp"
 
 #include "fps_device.hpp"
@@ -75,54 +82,60 @@ __device__ __forceinline__ uint64_t uniform_u64(uint64_t v) {
 
 }  // namespace
 
+// One record of a candidate's coordinates in LDS, read 16 bytes at a time.
+template <int D>
+struct alignas(16) Rec {
+  float c[(D + 3) / 4 * 4];
+};
+
 template <int D, int P, int TIE>
 __global__ void __launch_bounds__(kRoundsThreads) fps_rounds(RoundsParams a) {
   constexpr int W = kRoundsThreads / 64;
-  constexpr int CAP = (int)kRoundsCap;
-  constexpr int CH = CAP / 64;  // front waves
+  constexpr int CAP = (int)kRoundsCap;        // candidates the front decides on
+  constexpr int LIST = (int)kRoundsList;      // candidates that may come in
+  constexpr int CH = CAP / 64;
   constexpr uint32_t NWC = 2 + D;
   extern __shared__ uint64_t s_dyn[];  // best key of every block, then the boxes
 
-  __shared__ uint64_t s_lk[CAP];      // this workgroup's candidates
-  __shared__ float s_lc[D][CAP];
-  __shared__ uint64_t s_ck[CAP];      // all candidates as they came
-  __shared__ float s_cc[D][CAP];
-  __shared__ uint64_t s_sk[CAP];      // sorted
-  __shared__ float s_sc[D][CAP];
-  __shared__ uint32_t s_rank[CAP];
-  __shared__ uint32_t s_src[CAP];
-  __shared__ float s_pk[D][CAP];      // picks of the round
+  __shared__ alignas(16) uint64_t s_ck[LIST];  // candidates as they came
+  __shared__ Rec<D> s_cc[LIST];
+  __shared__ Rec<D> s_pk[CAP];        // picks of the round
   __shared__ uint32_t s_pt[CAP];      // their tie words
-  __shared__ uint32_t s_cnt[2];     // candidates of this workgroup, by round parity
-  __shared__ uint64_t s_wmax[W];
-  __shared__ uint64_t s_wu[W];
-  __shared__ uint32_t s_wtot[W];
-  __shared__ uint32_t s_ok;
+  __shared__ uint32_t s_rank[LIST];
+  __shared__ uint64_t s_sk[CAP];      // sorted candidates
+  __shared__ Rec<D> s_sc[CAP];
   __shared__ uint16_t s_low[CAP / 32][CAP][2];  // rows: which earlier candidates lower this one
+  __shared__ uint64_t s_lk[CAP];  // this workgroup's candidates
+  __shared__ Rec<D> s_lc[CAP];
+  __shared__ uint32_t s_cnt[2];  // candidates of this workgroup, by round parity
+  __shared__ uint32_t s_sum[2];  // candidates of the grid, by round parity
+  __shared__ uint32_t s_at[2];   // candidates taken in, by round parity
+  __shared__ uint64_t s_wmax[W];
   __shared__ uint64_t s_acc[CH];
   __shared__ uint64_t s_te;    // the bound that the round's picks exceed
   __shared__ uint32_t s_stop;  // first pick that does not lower itself
   __shared__ uint32_t s_np;
   __shared__ uint32_t s_stuck;
+  __shared__ uint32_t s_ok;
 
   const FpsParams &f = a.fps;
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
+  int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const uint32_t G = gridDim.x;
-  const uint32_t g = blockIdx.x;
+  uint32_t g = blockIdx.x;
   const uint32_t nbl = (a.nblocks - g + G - 1) / G;  // this workgroup's blocks: g, g + G, ...
+  const bool resident = nbl <= (uint32_t)W;          // a block per wave stays in registers
   uint64_t *s_bkey = s_dyn;
   float *s_box = (float *)(s_dyn + nbl);  // [2 * D][nbl]
 
   if (tid == 0) {
-    s_cnt[0] = 0;
-    s_cnt[1] = 0;
+    s_cnt[0] = s_cnt[1] = 0;
+    s_sum[0] = s_sum[1] = 0;
+    s_at[0] = s_at[1] = 0;
     s_stuck = 0;
     s_ok = 1;
   }
 
-  // Start: the forced picks, in pieces of CAP.
   uint32_t s = 0;        // picks recorded
   uint32_t np = 0;       // picks of the last round, in s_pk
   bool first = true;
@@ -131,11 +144,16 @@ __global__ void __launch_bounds__(kRoundsThreads) fps_rounds(RoundsParams a) {
   uint64_t step = (uint64_t)1 << 51;  // a sixteenth of a binade
   uint32_t e = 0;        // rounds
   uint32_t idle = 0;     // rounds since the last pick
+  float x[P][D], dm[P];  // the block in hand
+  uint32_t id[P];
 
   for (;;) {
-    // ---- forced picks -------------------------------------------------------
-    const bool forced = s < f.n_starts;
-    if (forced) {
+    // Rewritten each round: addresses formed from them would otherwise be kept in registers
+    // over the whole loop, beside the block.
+    asm volatile("" : "+v"(tid), "+s"(g));
+    const int lane = tid & 63;
+    // ---- forced picks, in pieces of CAP -------------------------------------
+    if (s < f.n_starts) {
       np = min(f.n_starts - s, (uint32_t)CAP);
       if ((uint32_t)tid < np) {
         uint64_t idx = f.starts[s + tid];
@@ -144,7 +162,7 @@ __global__ void __launch_bounds__(kRoundsThreads) fps_rounds(RoundsParams a) {
           idx = 0;
         }
 #pragma unroll
-        for (int j = 0; j < D; ++j) s_pk[j][tid] = f.pts[(size_t)idx * f.sp + (size_t)j * f.ld];
+        for (int j = 0; j < D; ++j) s_pk[tid].c[j] = f.pts[(size_t)idx * f.sp + (size_t)j * f.ld];
         s_pt[tid] = tie_of<TIE>((uint32_t)idx);
       }
       lds_barrier();
@@ -155,12 +173,12 @@ __global__ void __launch_bounds__(kRoundsThreads) fps_rounds(RoundsParams a) {
         f.out[s + tid] = tie_of<TIE>(s_pt[tid]);
         if (f.out_pts != nullptr) {
 #pragma unroll
-          for (int j = 0; j < D; ++j) f.out_pts[(size_t)(s + tid) * D + j] = s_pk[j][tid];
+          for (int j = 0; j < D; ++j) f.out_pts[(size_t)(s + tid) * D + j] = s_pk[tid].c[j];
         }
       }
+      if (tid == 0) f.status[1] = e;
     }
     s += np;
-    if (g == 0 && tid == 0) f.status[1] = e;
     if (s >= f.m) return;
     if (s_stuck) {
       // The last pick left its own key unchanged, so it stays the best for good.
@@ -170,7 +188,7 @@ __global__ void __launch_bounds__(kRoundsThreads) fps_rounds(RoundsParams a) {
           f.out[q] = tie_of<TIE>(t);
           if (f.out_pts != nullptr) {
 #pragma unroll
-            for (int j = 0; j < D; ++j) f.out_pts[(size_t)q * D + j] = s_pk[j][np - 1];
+            for (int j = 0; j < D; ++j) f.out_pts[(size_t)q * D + j] = s_pk[np - 1].c[j];
           }
         }
       }
@@ -209,32 +227,32 @@ __global__ void __launch_bounds__(kRoundsThreads) fps_rounds(RoundsParams a) {
 #pragma unroll
         for (int c = 0; c < CH; ++c) {
           if ((uint32_t)c < nch) {
+            const Rec<D> r = s_pk[c * 64 + lane];
             float p[D];
 #pragma unroll
-            for (int j = 0; j < D; ++j) p[j] = s_pk[j][c * 64 + lane];
-            const bool h = (uint32_t)(c * 64 + lane) < np && box_bound<D>(p, lo, hi) < bmax;
-            hit[c] = __ballot(h);
+            for (int j = 0; j < D; ++j) p[j] = r.c[j];
+            hit[c] = __ballot((uint32_t)(c * 64 + lane) < np && box_bound<D>(p, lo, hi) < bmax);
             any = any || hit[c] != 0;
           }
         }
       }
       if (any || bkey > Tg) {
-        float x[P][D], dm[P];
-        uint32_t id[P];
+        if (first || !resident) {
 #pragma unroll
-        for (int k = 0; k < P; ++k) {
-          const uint32_t p = base + (uint32_t)(k * 64 + lane);
-          const uint32_t pc = min(p, f.n - 1);
+          for (int k = 0; k < P; ++k) {
+            const uint32_t p = base + (uint32_t)(k * 64 + lane);
+            const uint32_t pc = min(p, f.n - 1);
 #pragma unroll
-          for (int j = 0; j < D; ++j)
-            x[k][j] = a.pos[(size_t)pc * a.pos_sp + (size_t)j * a.pos_ld];
-          id[k] = a.perm ? a.perm[pc] : pc;
-          dm[k] = first ? f.init : f.dmin[pc];
-        }
-        if (base + 64 * P > f.n) {
+            for (int j = 0; j < D; ++j)
+              x[k][j] = a.pos[(size_t)pc * a.pos_sp + (size_t)j * a.pos_ld];
+            id[k] = a.perm ? a.perm[pc] : pc;
+            dm[k] = first ? f.init : f.dmin[pc];
+          }
+          if (base + 64 * P > f.n) {
 #pragma unroll
-          for (int k = 0; k < P; ++k)
-            if (base + (uint32_t)(k * 64 + lane) >= f.n) dm[k] = -1.0f;
+            for (int k = 0; k < P; ++k)
+              if (base + (uint32_t)(k * 64 + lane) >= f.n) dm[k] = -1.0f;
+          }
         }
         if (first) {
           // Bounding box (clamped padding repeats the last point).
@@ -259,24 +277,24 @@ __global__ void __launch_bounds__(kRoundsThreads) fps_rounds(RoundsParams a) {
           for (int c = 0; c < CH; ++c) {
             uint64_t mm = hit[c];
             if (mm) {
-              float q[D];
-#pragma unroll
-              for (int j = 0; j < D; ++j) q[j] = s_pk[j][c * 64 + lane];
+              const Rec<D> r = s_pk[c * 64 + lane];
               do {
                 const int l = __ffsll((unsigned long long)mm) - 1;
                 mm &= mm - 1;
                 float p[D];
 #pragma unroll
-                for (int j = 0; j < D; ++j) p[j] = readlane_f(q[j], l);
+                for (int j = 0; j < D; ++j) p[j] = readlane_f(r.c[j], l);
 #pragma unroll
                 for (int k = 0; k < P; ++k) dm[k] = min_keep(sqdist<D>(x[k], p), dm[k]);
               } while (mm);
             }
           }
+          if (!resident) {
 #pragma unroll
-          for (int k = 0; k < P; ++k) {
-            const uint32_t p = base + (uint32_t)(k * 64 + lane);
-            if (p < f.n) f.dmin[p] = dm[k];
+            for (int k = 0; k < P; ++k) {
+              const uint32_t p = base + (uint32_t)(k * 64 + lane);
+              if (p < f.n) f.dmin[p] = dm[k];
+            }
           }
           // The block's best key.
           int bv = INT_MIN;
@@ -311,8 +329,10 @@ __global__ void __launch_bounds__(kRoundsThreads) fps_rounds(RoundsParams a) {
             const uint32_t q = at + lanes_below(m[k]);
             if (((m[k] >> lane) & 1) && q < (uint32_t)CAP) {
               s_lk[q] = make_key(__float_as_int(dm[k]), tie_of<TIE>(id[k]));
+              Rec<D> r;
 #pragma unroll
-              for (int j = 0; j < D; ++j) s_lc[j][q] = x[k][j];
+              for (int j = 0; j < D; ++j) r.c[j] = x[k][j];
+              s_lc[q] = r;
             }
             at += (uint32_t)__popcll(m[k]);
           }
@@ -326,77 +346,120 @@ __global__ void __launch_bounds__(kRoundsThreads) fps_rounds(RoundsParams a) {
       continue;
     }
     if (lane == 0) s_wmax[wave] = wmax;
+    if (tid < LIST) {
+      s_ck[tid] = 0;
+      s_rank[tid] = 0;
+    }
+    if (tid == 0) {
+      s_te = Tg;
+      s_stop = ~0u;
+    }
     lds_barrier();
     ++e;
-    uint32_t C = s_cnt[e & 1];
+    const uint32_t par = e & 1u;
+    const uint32_t own = s_cnt[par];
     uint64_t U = wave_max_u64(lane < W ? s_wmax[lane] : 0ull);  // this workgroup's best key
 
     // ---- 2. exchange --------------------------------------------------------
-    bool over;
+    // L lanes read one workgroup's header and its first L candidates at once, so most
+    // candidates are here as soon as their header is; those beyond L follow.
+    uint32_t C = own;
     if (G > 1) {
       const uint32_t capw = a.cap_wg;
-      over = C > capw;
       const size_t head = (size_t)kRoundsReplicas * kRoundsHeadWords * kRoundsMaxGrid;
-      const size_t cands = (size_t)NWC * G * capw;
-      uint64_t *buf = f.xchg + (size_t)(e & 1u) * (head + cands);
-      uint64_t *cbuf = buf + head;
       const size_t cp = (size_t)G * capw;  // pitch of one word's array
+      uint64_t *buf = f.xchg + (size_t)par * (head + NWC * cp);
+      uint64_t *cbuf = buf + head;
       if (wave == 0) {
         if (lane < (int)(kRoundsReplicas * kRoundsHeadWords)) {
           const uint32_t rep = (uint32_t)lane / kRoundsHeadWords;
           const uint32_t k = (uint32_t)lane - rep * kRoundsHeadWords;
-          const uint32_t v = k == 0 ? (C | (over ? 0x80000000u : 0u))
-                                    : (k == 1 ? (uint32_t)(U >> 32) : (uint32_t)U);
+          const uint32_t v = k == 0 ? own : (k == 1 ? (uint32_t)(U >> 32) : (uint32_t)U);
           xchg_store(buf + ((size_t)rep * kRoundsHeadWords + k) * kRoundsMaxGrid + g,
                      ((uint64_t)v << 32) | e);
         }
-      } else if (!over) {
-        for (uint32_t q = (uint32_t)tid - 64; q < C; q += kRoundsThreads - 64) {
+      } else if (own <= capw) {
+        for (uint32_t q = (uint32_t)tid - 64; q < own; q += kRoundsThreads - 64) {
           const uint64_t k = s_lk[q];
+          const Rec<D> r = s_lc[q];
           uint64_t *w = cbuf + (size_t)g * capw + q;
           xchg_store(w, (k & 0xffffffff00000000ull) | e);
           xchg_store(w + cp, (k << 32) | e);
 #pragma unroll
           for (int j = 0; j < D; ++j)
             xchg_store(w + (size_t)(2 + j) * cp,
-                       ((uint64_t)(uint32_t)__float_as_int(s_lc[j][q]) << 32) | e);
+                       ((uint64_t)(uint32_t)__float_as_int(r.c[j]) << 32) | e);
         }
       }
-      const uint32_t PW = (G + 63u) >> 6;
-      uint32_t cq = 0;
-      uint32_t incl = 0;
-      if ((uint32_t)wave < PW) {
-        const uint32_t q = (uint32_t)tid;
-        const uint64_t *h = buf + (size_t)(g % kRoundsReplicas) * kRoundsHeadWords * kRoundsMaxGrid + q;
-        uint64_t w0 = 0, w1 = 0, w2 = 0;
-        bool ok = true;
-        if (q < G) {
+      const uint32_t L = G <= 128 ? 8 : 4;
+      const uint32_t q = (uint32_t)tid / L;
+      const uint32_t l = (uint32_t)tid & (L - 1);
+      uint64_t w1 = 0, w2 = 0;
+      if ((uint32_t)wave * 64 < G * L) {
+        const uint64_t *h =
+            buf + (size_t)(g % kRoundsReplicas) * kRoundsHeadWords * kRoundsMaxGrid + q;
+        const uint64_t *w = cbuf + (size_t)q * capw;
+        uint32_t cq = 0;
+        uint64_t v[NWC];
+        const bool mine = q < G;
+        bool here = false;  // candidate l of workgroup q is there
+        if (mine) {
           const uint64_t deadline = now_ticks() + f.spin_ticks;
           for (;;) {
-            w0 = xchg_load(h);
+            const uint64_t w0 = xchg_load(h);
             w1 = xchg_load(h + kRoundsMaxGrid);
             w2 = xchg_load(h + 2 * kRoundsMaxGrid);
-            if ((uint32_t)w0 == e && (uint32_t)w1 == e && (uint32_t)w2 == e) break;
+#pragma unroll
+            for (uint32_t k = 0; k < NWC; ++k) v[k] = xchg_load(w + l + k * cp);
+            bool all = true;
+#pragma unroll
+            for (uint32_t k = 0; k < NWC; ++k) all = all && (uint32_t)v[k] == e;
+            cq = (uint32_t)(w0 >> 32);
+            here = l < cq && cq <= capw;
+            if ((uint32_t)w0 == e && (uint32_t)w1 == e && (uint32_t)w2 == e && (all || !here)) break;
             if (now_ticks() > deadline) {
-              ok = false;
+              s_ok = 0;
+              cq = 0;
+              here = false;
               break;
             }
           }
         }
-        const bool wave_ok = __ballot(!ok) == 0;
-        cq = (uint32_t)(w0 >> 32);
-        const bool ov = __ballot((cq & 0x80000000u) != 0) != 0;
-        cq &= 0x7fffffffu;
-        incl = wave_scan_add(cq);
-        const uint64_t u = wave_max_u64((w1 & 0xffffffff00000000ull) | (w2 >> 32));
-        if (lane == 63) {
-          s_wtot[wave] = (incl & 0x7fffffffu) | (ov ? 0x80000000u : 0u);
-          s_wu[wave] = u;
-          if (!wave_ok) s_ok = 0;
-        }
-        if (PW == 1 && !ov) {
-          const uint32_t off = incl - cq;
-          for (uint32_t i = 0; i < cq && off + i < (uint32_t)CAP; ++i) s_src[off + i] = q * capw + i;
+        const uint32_t sum =
+            (uint32_t)__builtin_amdgcn_readlane((int)wave_scan_add(l == 0 ? cq : 0u), 63);
+        if (lane == 0 && sum) atomicAdd(&s_sum[par], sum);
+        uint32_t i = l;
+        for (;;) {
+          const uint64_t m = __ballot(here);
+          if (!m) break;
+          uint32_t at = 0;
+          if (lane == 0) at = atomicAdd(&s_at[par], (uint32_t)__popcll(m));
+          at = (uint32_t)__builtin_amdgcn_readfirstlane((int)at) + lanes_below(m);
+          if (here && at < (uint32_t)LIST) {
+            s_ck[at] = (v[0] & 0xffffffff00000000ull) | (v[1] >> 32);
+            Rec<D> r;
+#pragma unroll
+            for (int j = 0; j < D; ++j) r.c[j] = __int_as_float((int)(v[2 + j] >> 32));
+            s_cc[at] = r;
+          }
+          i += L;
+          here = here && i < cq;
+          if (here) {
+            const uint64_t deadline = now_ticks() + f.spin_ticks;
+            for (;;) {
+              bool all = true;
+#pragma unroll
+              for (uint32_t k = 0; k < NWC; ++k) v[k] = xchg_load(w + i + k * cp);
+#pragma unroll
+              for (uint32_t k = 0; k < NWC; ++k) all = all && (uint32_t)v[k] == e;
+              if (all) break;
+              if (now_ticks() > deadline) {
+                s_ok = 0;
+                here = false;
+                break;
+              }
+            }
+          }
         }
       }
       lds_barrier();
@@ -404,67 +467,33 @@ __global__ void __launch_bounds__(kRoundsThreads) fps_rounds(RoundsParams a) {
         if (tid == 0) atomicOr(f.status, kStatusTimeout);
         return;
       }
-      C = 0;
-      over = false;
-      U = 0;
-      uint32_t before = 0;
-      for (uint32_t w = 0; w < PW; ++w) {
-        const uint32_t t = s_wtot[w];
-        if (w < (uint32_t)wave) before += t & 0x7fffffffu;
-        C += t & 0x7fffffffu;
-        over = over || (t & 0x80000000u);
-        U = s_wu[w] > U ? s_wu[w] : U;
-      }
-      over = over || C > (uint32_t)CAP;
-      if (PW > 1 && !over) {
-        if ((uint32_t)wave < PW) {
-          const uint32_t off = before + incl - cq;
-          for (uint32_t i = 0; i < cq; ++i) s_src[off + i] = (uint32_t)tid * capw + i;
-        }
+      C = s_sum[par];
+      const uint32_t got = s_at[par];
+      if (got != C || C > (uint32_t)LIST) C = max(C, (uint32_t)LIST + 1);  // some did not fit
+      if (C == 0) {
+        // Nobody has a candidate: the best key of all is the exact bound.
+        const uint64_t u = wave_max_u64((w1 & 0xffffffff00000000ull) | (w2 >> 32));
+        if (lane == 0) s_wmax[wave] = (uint32_t)wave * 64 < G * L ? u : 0ull;
         lds_barrier();
-      }
-      if (!over && (uint32_t)tid < C) {
-        const uint64_t *w = cbuf + s_src[tid];
-        uint64_t v[NWC];
-        const uint64_t deadline = now_ticks() + f.spin_ticks;
-        for (;;) {
-          bool all = true;
-#pragma unroll
-          for (uint32_t k = 0; k < NWC; ++k) v[k] = xchg_load(w + k * cp);
-#pragma unroll
-          for (uint32_t k = 0; k < NWC; ++k) all = all && (uint32_t)v[k] == e;
-          if (all) break;
-          if (now_ticks() > deadline) {
-            s_ok = 0;
-            break;
-          }
-        }
-        s_ck[tid] = (v[0] & 0xffffffff00000000ull) | (v[1] >> 32);
-#pragma unroll
-        for (int j = 0; j < D; ++j) s_cc[j][tid] = __int_as_float((int)(v[2 + j] >> 32));
+        U = wave_max_u64(lane < W ? s_wmax[lane] : 0ull);
       }
     } else {
-      over = C > (uint32_t)CAP;
-      if (!over && (uint32_t)tid < C) {
+      if ((uint32_t)tid < own && tid < CAP) {
         s_ck[tid] = s_lk[tid];
-#pragma unroll
-        for (int j = 0; j < D; ++j) s_cc[j][tid] = s_lc[j][tid];
+        s_cc[tid] = s_lc[tid];
       }
+      if (own > (uint32_t)CAP) C = max(own, (uint32_t)LIST + 1);
+      lds_barrier();
     }
-    if (tid < CAP) s_rank[tid] = 0;
-    if (tid == 0) {
-      s_cnt[(e + 1) & 1] = 0;  // read by everybody before this round's first barrier
-      s_te = Tg;
-      s_stop = ~0u;
-    }
-    lds_barrier();
-    if (!s_ok) {
-      if (tid == 0) atomicOr(f.status, kStatusTimeout);
-      return;
+    if (tid == 0) {  // the other parity's counters: everybody has read them
+      s_np = 0;
+      s_cnt[par ^ 1] = 0;
+      s_sum[par ^ 1] = 0;
+      s_at[par ^ 1] = 0;
     }
     U = uniform_u64(U);
     C = (uint32_t)__builtin_amdgcn_readfirstlane((int)C);
-    if (over || C == 0) {
+    if (C > (uint32_t)LIST || C == 0) {
       // No picks: a smaller step, or the exact bound and a larger one.  From an exact bound
       // every step has a candidate, and halving ends at the best point alone, so a pick
       // comes within some 64 rounds; the count only guards the loop's end.
@@ -473,39 +502,50 @@ __global__ void __launch_bounds__(kRoundsThreads) fps_rounds(RoundsParams a) {
         if (tid == 0) atomicOr(f.status, kStatusTimeout);
         return;
       }
-      if (over) {
-        const double r = sqrt((double)a.target / (double)(C > 2 * a.target ? C : 2 * a.target));
-        const uint64_t ns = (uint64_t)((double)step * r);
+      if (C) {
+        const uint64_t ns = (uint64_t)((double)step * sqrt((double)a.target / (double)C));
         step = ns < 1 ? 1 : ns;
       } else {
         T = U;
         if (Tg != ~0ull) step = step < ((uint64_t)1 << 60) ? step << 1 : step;
       }
       Tg = T > step ? T - step : 0;
+      lds_barrier();
       continue;
     }
 
     // ---- 3. front -----------------------------------------------------------
-    const uint32_t nc = (C + 63u) >> 6;
-    for (uint32_t job = wave; job < nc * nc; job += W) {
-      const uint32_t ic = job % nc, jc = job / nc;
-      const uint32_t i = ic * 64 + lane;
-      const uint64_t ki = i < C ? s_ck[i] : ~0ull;
-      const uint32_t jl = jc * 64 + lane;
-      const uint64_t kj = jl < C ? s_ck[jl] : 0ull;
-      const int jn = (int)min(64u, C - jc * 64);
-      uint32_t r = 0;
-      for (int l = 0; l < jn; ++l) r += readlane_u64(kj, l) > ki ? 1u : 0u;
-      if (i < C) atomicAdd(&s_rank[i], r);
+    // Order of the candidates: how many keys exceed one's own, 16 at a time.
+    {
+      const uint32_t nc = (C + 63u) >> 6;
+      const uint32_t nj = (C + 15u) >> 4;
+      for (uint32_t job = wave; job < nc * nj; job += W) {
+        const uint32_t jc = job / nc, ic = job - jc * nc;
+        const uint32_t i = ic * 64 + lane;
+        const uint64_t ki = s_ck[i];
+        const uint64_t *kj = s_ck + jc * 16;
+        uint32_t r = 0;
+#pragma unroll 1
+        for (int h = 0; h < 16; h += 8) {
+#pragma unroll
+          for (int l = 0; l < 8; ++l) r += kj[h + l] > ki ? 1u : 0u;
+        }
+        if (i < C && r) atomicAdd(&s_rank[i], r);
+      }
     }
     lds_barrier();
     if ((uint32_t)tid < C) {
       const uint32_t r = s_rank[tid];
-      s_sk[r] = s_ck[tid];
-#pragma unroll
-      for (int j = 0; j < D; ++j) s_sc[j][r] = s_cc[j][tid];
+      if (r < (uint32_t)CAP) {
+        s_sk[r] = s_ck[tid];
+        s_sc[r] = s_cc[tid];
+      } else if (r == (uint32_t)CAP) {
+        s_te = s_ck[tid];  // the first one that the front does not see is the bound
+      }
     }
     lds_barrier();
+    const uint32_t F = min(C, (uint32_t)CAP);
+    const uint32_t nc = (F + 63u) >> 6;
     // Which earlier candidates lower a candidate: bit j of candidate i's row, j < i, for the
     // sorted candidates.  A job is 64 candidates against 16 earlier ones.
     for (uint32_t job = wave, c = 0; c < nc;) {
@@ -515,22 +555,24 @@ __global__ void __launch_bounds__(kRoundsThreads) fps_rounds(RoundsParams a) {
         continue;
       }
       const uint32_t j0 = job * 16;
-      if (j0 < C) {
+      if (j0 < F) {
         const uint32_t i = c * 64 + lane;
         const float v = __int_as_float((int)(uint32_t)(s_sk[i] >> 32) - 1);
-        float x[D], q[D];
+        const Rec<D> ri = s_sc[i];
+        float xi[D];
 #pragma unroll
-        for (int j = 0; j < D; ++j) {
-          x[j] = s_sc[j][i];
-          q[j] = s_sc[j][j0 + (lane & 15)];
-        }
+        for (int j = 0; j < D; ++j) xi[j] = ri.c[j];
         uint32_t bits = 0;
+#pragma unroll 1
+        for (int h = 12; h >= 0; h -= 4) {
 #pragma unroll
-        for (int l = 15; l >= 0; --l) {
-          float p[D];
+          for (int l = 3; l >= 0; --l) {
+            const Rec<D> rj = s_sc[j0 + h + l];
+            float p[D];
 #pragma unroll
-          for (int j = 0; j < D; ++j) p[j] = readlane_f(q[j], l);
-          bits = bits + bits + (sqdist<D>(x, p) < v ? 1u : 0u);
+            for (int j = 0; j < D; ++j) p[j] = rj.c[j];
+            bits = bits + bits + (sqdist<D>(xi, p) < v ? 1u : 0u);
+          }
         }
         s_low[job >> 1][i][job & 1] = (uint16_t)bits;
       }
@@ -539,31 +581,30 @@ __global__ void __launch_bounds__(kRoundsThreads) fps_rounds(RoundsParams a) {
     lds_barrier();
     // The picks, were no candidate only partly lowered: each candidate that no earlier pick
     // lowers, settled in a few steps per 64 candidates rather than one by one.
+    const uint32_t *rows = (const uint32_t *)&s_low[0][0][0];
     if (wave == 0) {
       uint64_t low[CH][CH];
 #pragma unroll
       for (int c = 0; c < CH; ++c)
 #pragma unroll
-        for (int w = 0; w <= c; ++w) {
-          const uint32_t *r = (const uint32_t *)&s_low[0][0][0];
-          low[c][w] = ((uint64_t)r[(2 * w + 1) * CAP + c * 64 + lane] << 32) |
-                      r[2 * w * CAP + c * 64 + lane];
-        }
+        for (int w = 0; w <= c; ++w)
+          low[c][w] = ((uint64_t)rows[(2 * w + 1) * CAP + c * 64 + lane] << 32) |
+                      rows[2 * w * CAP + c * 64 + lane];
       uint64_t acc[CH];
 #pragma unroll
       for (int c = 0; c < CH; ++c) {
         acc[c] = 0;
         if ((uint32_t)c < nc) {
-          uint64_t hitc = 0;
+          uint64_t before = 0;
 #pragma unroll
-          for (int w = 0; w < c; ++w) hitc |= low[c][w] & acc[w];
-          const uint64_t own = low[c][c] & (((uint64_t)1 << lane) - 1);
-          uint64_t open = __ballot((uint32_t)(c * 64 + lane) < C && hitc == 0);
+          for (int w = 0; w < c; ++w) before |= low[c][w] & acc[w];
+          const uint64_t same = low[c][c] & (((uint64_t)1 << lane) - 1);
+          uint64_t open = __ballot((uint32_t)(c * 64 + lane) < F && before == 0);
           while (open) {
-            const uint64_t free = __ballot((own & open) == 0) & open;
+            const uint64_t free = __ballot((same & open) == 0) & open;
             acc[c] |= free;
             open &= ~free;
-            open &= ~__ballot((own & free) != 0);
+            open &= ~__ballot((same & free) != 0);
           }
         }
         if (lane == 0) s_acc[c] = acc[c];
@@ -572,59 +613,58 @@ __global__ void __launch_bounds__(kRoundsThreads) fps_rounds(RoundsParams a) {
     lds_barrier();
     // A candidate whose first lowering pick leaves its key above the bound raises the bound
     // to that key; a pick that does not lower itself ends the round.
+    uint64_t key = 0;
+    uint64_t taken = 0;
+    Rec<D> ri;
     if ((uint32_t)wave < nc) {
       const uint32_t i = (uint32_t)tid;
-      const uint64_t key = s_sk[i];
+      key = s_sk[i];
+      ri = s_sc[i];
       const float v = __int_as_float((int)(uint32_t)(key >> 32) - 1);
-      float x[D];
+      float xi[D];
 #pragma unroll
-      for (int j = 0; j < D; ++j) x[j] = s_sc[j][i];
-      const uint64_t mine = uniform_u64(s_acc[wave]);
-      const bool taken = (mine >> lane) & 1;
+      for (int j = 0; j < D; ++j) xi[j] = ri.c[j];
+      taken = uniform_u64(s_acc[wave]);
+      const bool mine = (taken >> lane) & 1;
       int by = -1;
 #pragma unroll
       for (int w = CH - 1; w >= 0; --w) {
         if (w <= wave) {
-          const uint32_t *r = (const uint32_t *)&s_low[0][0][0];
-          uint64_t k = ((uint64_t)r[(2 * w + 1) * CAP + i] << 32) | r[2 * w * CAP + i];
+          uint64_t k = ((uint64_t)rows[(2 * w + 1) * CAP + i] << 32) | rows[2 * w * CAP + i];
           if (w == wave) k &= ((uint64_t)1 << lane) - 1;
           k &= s_acc[w];
           if (k) by = w * 64 + __ffsll((unsigned long long)k) - 1;
         }
       }
-      if (i < C && !taken && by >= 0) {
+      if (i < F && !mine && by >= 0) {
+        const Rec<D> rb = s_sc[by];
         float p[D];
 #pragma unroll
-        for (int j = 0; j < D; ++j) p[j] = s_sc[j][by];
-        const uint64_t nk = make_key(__float_as_int(sqdist<D>(x, p)), (uint32_t)key);
+        for (int j = 0; j < D; ++j) p[j] = rb.c[j];
+        const uint64_t nk = make_key(__float_as_int(sqdist<D>(xi, p)), (uint32_t)key);
         if (nk > Tg) atomicMax((unsigned long long *)&s_te, (unsigned long long)nk);
       }
-      if (i < C && taken && !(sqdist<D>(x, x) < v)) atomicMin(&s_stop, i);
+      if (i < F && mine && !(sqdist<D>(xi, xi) < v)) atomicMin(&s_stop, i);
     }
     lds_barrier();
     T = uniform_u64(s_te);
-    const uint32_t stop = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_stop);
     if ((uint32_t)wave < nc) {
+      const uint32_t stop = s_stop;
+      // Keys fall along the chunks: a chunk with picks has those before it whole.
       uint32_t at = 0;
-      uint64_t mine = 0;
-      for (uint32_t c = 0; c < nc; ++c) {
-        const uint32_t i = c * 64 + lane;
-        const uint64_t m =
-            __ballot(i < C && s_sk[i] > T && i <= stop) & uniform_u64(s_acc[c]);
-        if (c < (uint32_t)wave) at += (uint32_t)__popcll(m);
-        if (c == (uint32_t)wave) mine = m;
-      }
+      for (int w = 0; w < wave; ++w) at += (uint32_t)__popcll(s_acc[w]);
+      taken &= __ballot(key > T && (uint32_t)tid <= stop);
+      at = (uint32_t)__builtin_amdgcn_readfirstlane((int)at);
       const uint32_t room = f.m - s;
-      const uint32_t q = at + lanes_below(mine);
-      if (((mine >> lane) & 1) && q < room) {
-        s_pt[q] = (uint32_t)s_sk[tid];
-#pragma unroll
-        for (int j = 0; j < D; ++j) s_pk[j][q] = s_sc[j][tid];
-      }
-      if ((uint32_t)wave == nc - 1 && lane == 0) {
-        const uint32_t all = at + (uint32_t)__popcll(mine);
-        s_np = all < room ? all : room;
-        if (stop < C && s_sk[stop] > T) s_stuck = 1;
+      if (taken) {
+        const uint32_t q = at + lanes_below(taken);
+        if (((taken >> lane) & 1) && q < room) {
+          s_pt[q] = (uint32_t)key;
+          s_pk[q] = ri;
+        }
+        if (lane == 0) atomicMax(&s_np, min(at + (uint32_t)__popcll(taken), room));
+        if (stop - (uint32_t)wave * 64 < 64u && ((taken >> (stop & 63u)) & 1) && lane == 0)
+          s_stuck = 1;
       }
     }
     lds_barrier();

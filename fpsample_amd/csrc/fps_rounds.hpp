@@ -20,8 +20,8 @@ struct RoundsParams {
 };
 
 constexpr int kRoundsThreads = 1024;
-constexpr uint32_t kRoundsCap = 256;       // candidates of one round
-constexpr uint32_t kRoundsTarget = 160;    // candidates aimed at
+constexpr uint32_t kRoundsCap = 256;       // candidates a round decides on
+constexpr uint32_t kRoundsList = 512;      // candidates that may come in: the best kRoundsCap count
 constexpr uint32_t kRoundsMaxGrid = 256;
 constexpr uint32_t kRoundsHeadWords = 3;   // count, high and low half of the best key
 constexpr uint32_t kRoundsReplicas = 4;    // copies of the headers

@@ -401,14 +401,18 @@ int plan(Ctx &c, size_t n, size_t dim, int tie, size_t m, Plan &p) {
 
 // Threshold-round plan.  FPSX_ROUNDS="P:G[:target[:order]]" overrides: points per lane,
 // workgroups (0: the rules below), candidates aimed at per round, spatial order (0 or 1).
-//   P: a workgroup's 16 waves take a block of 64 * P points each.  Small blocks have tight
-//   boxes and spread a pick's work; large ones need fewer box tests.  Kernel ms at 64
-//   workgroups (gauss1m: 128): uniform 50 K / 4096 picks 0.83 at P = 1, 0.87 at 4, 1.09 at 8
-//   (its 98 blocks fill 6 workgroups); uniform 100 K / 50 K picks 4.53, 4.52 and 5.58;
-//   gauss1m / 16384 picks 2.74 at 4, 2.67 at 8.
-//   G: gauss1m 3.58, 2.94, 2.67 and 2.80 ms at 32, 64, 128 and 256; the 16.7 M-point lattice
-//   7.45, 5.41 and 4.48 ms at 64, 128 and 256 (early rounds sweep the whole cloud).
-static int plan_rounds(Ctx &c, size_t n, size_t dim, int tie, Plan &p) {
+//   P: a workgroup's 16 waves take a block of 64 * P points each, kept in registers while
+//   there is one block per wave.  Small blocks have tight boxes and spread a pick's work;
+//   large ones need fewer box tests.  Kernel ms: uniform 50 K points / 4096 picks at 64
+//   workgroups 0.66 at P = 1, 0.68 at 4 (32 workgroups); uniform 100 K / 50 K picks 3.68 and
+//   3.44 (64), 4.23 at 8 (13); gauss1m / 16384 picks 2.13 at 4 (256), 2.13 at 8 (128).
+//   G: gauss1m 2.53, 2.13 and 2.20 ms at 64, 128 and 256 (P = 8); the 16.7 M-point lattice
+//   4.94 and 4.09 ms at 128 and 256 (early rounds sweep the whole cloud).
+//   target: a round costs about 6 us and 20 ns a candidate, so long runs take more per round:
+//   100 K / 50 K picks 4.05, 3.58, 3.39, 3.23 and 3.20 ms at 128, 160, 192, 224 and 256;
+//   gauss1m 2.13 and 2.08 at 160 and 224; 50 K / 4096 picks 0.69, 0.66, 0.69 and 0.72 at 128,
+//   160, 192 and 224; 4096 / 1024 picks 0.32, 0.33, 0.35 and 0.36 at 96, 128, 160 and 192.
+static int plan_rounds(Ctx &c, size_t n, size_t dim, int tie, size_t m, Plan &p) {
   int P = 0, G = 0, target = 0, order = -1;
   if (const char *env = std::getenv("FPSX_ROUNDS"))
     if (*env) std::sscanf(env, "%d:%d:%d:%d", &P, &G, &target, &order);
@@ -434,7 +438,9 @@ static int plan_rounds(Ctx &c, size_t n, size_t dim, int tie, Plan &p) {
   p.grid = (uint32_t)g;
   p.chunk = (uint32_t)(nbl * 64 * P);
   p.shmem = shmem;
-  p.target = target > 0 ? std::min<uint32_t>((uint32_t)target, kRoundsCap) : kRoundsTarget;
+  p.target = target > 0 ? std::min<uint32_t>((uint32_t)target, kRoundsCap)
+             : m >= 16384 ? 224
+                          : (uint32_t)std::min<size_t>(160, std::max<size_t>(64, m / 8));
   p.order = order >= 0 ? order != 0 : n > 4096;
   return FPSX_OK;
 }
@@ -452,7 +458,7 @@ int plan_call(Ctx &c, size_t n, size_t dim, int tie, size_t m, Plan &p) {
                       env_set("FPSX_NO_ROUNDS") ||
                       c.tuned.find(std::make_tuple(n, dim, tie)) != c.tuned.end();
   if (!passes && (env_set("FPSX_ROUNDS") || (n >= 4096 && m >= 64)) &&
-      plan_rounds(c, n, dim, tie, p) == FPSX_OK)
+      plan_rounds(c, n, dim, tie, m, p) == FPSX_OK)
     return FPSX_OK;
   t_err.clear();
   return plan(c, n, dim, tie, m, p);
@@ -620,7 +626,7 @@ static std::vector<Plan> candidates(Ctx &c, size_t n, size_t dim, int tie, size_
   std::vector<Plan> out;
   Plan q;
   if (plan(c, n, dim, tie, m, q) == FPSX_OK) out.push_back(q);
-  if (plan_rounds(c, n, dim, tie, q) == FPSX_OK) out.push_back(q);
+  if (plan_rounds(c, n, dim, tie, m, q) == FPSX_OK) out.push_back(q);
   q = Plan();
   size_t cnt;
   const KernelEntry *t = resident_table(&cnt);
