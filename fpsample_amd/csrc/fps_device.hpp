@@ -80,6 +80,20 @@ __device__ __forceinline__ float readlane_f(float v, int lane) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
 }
 
+// Inclusive prefix sum over the wave.
+__device__ __forceinline__ uint32_t wave_scan_add(uint32_t v) {
+  int x = (int)v;
+#define STEP(ctrl, rm) x += __builtin_amdgcn_update_dpp(0, x, ctrl, rm, 0xf, false)
+  STEP(0x111, 0xf);  // row_shr:1
+  STEP(0x112, 0xf);  // row_shr:2
+  STEP(0x114, 0xf);  // row_shr:4
+  STEP(0x118, 0xf);  // row_shr:8
+  STEP(0x142, 0xa);  // row_bcast:15
+  STEP(0x143, 0xc);  // row_bcast:31
+#undef STEP
+  return (uint32_t)x;
+}
+
 // True when candidate (v, i) beats (bv, bi) under the tie rule.
 template <int TIE>
 __device__ __forceinline__ bool beats(int v, uint32_t i, int bv, uint32_t bi) {

@@ -51,20 +51,6 @@ __device__ __forceinline__ uint64_t wave_max_u64(uint64_t k) {
   return ((uint64_t)hi << 32) | lo;
 }
 
-// Inclusive prefix sum over the wave.
-__device__ __forceinline__ uint32_t wave_scan_add(uint32_t v) {
-  int x = (int)v;
-#define STEP(ctrl, rm) x += __builtin_amdgcn_update_dpp(0, x, ctrl, rm, 0xf, false)
-  STEP(0x111, 0xf);  // row_shr:1
-  STEP(0x112, 0xf);  // row_shr:2
-  STEP(0x114, 0xf);  // row_shr:4
-  STEP(0x118, 0xf);  // row_shr:8
-  STEP(0x142, 0xa);  // row_bcast:15
-  STEP(0x143, 0xc);  // row_bcast:31
-#undef STEP
-  return (uint32_t)x;
-}
-
 __device__ __forceinline__ uint32_t lanes_below(uint64_t mask) {
   return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32),
                                    __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
@@ -242,10 +228,18 @@ __global__ void __launch_bounds__(kRoundsThreads) fps_rounds(RoundsParams a) {
           for (int k = 0; k < P; ++k) {
             const uint32_t p = base + (uint32_t)(k * 64 + lane);
             const uint32_t pc = min(p, f.n - 1);
+            if (a.rec) {
+              const float4 r = a.rec[pc];
+              const float r3[3] = {r.x, r.y, r.z};
 #pragma unroll
-            for (int j = 0; j < D; ++j)
-              x[k][j] = a.pos[(size_t)pc * a.pos_sp + (size_t)j * a.pos_ld];
-            id[k] = a.perm ? a.perm[pc] : pc;
+              for (int j = 0; j < D; ++j)
+                x[k][j] = j < 3 ? r3[j < 3 ? j : 0] : a.rest[(size_t)(j - 3) * f.n + pc];
+              id[k] = (uint32_t)__float_as_int(r.w);
+            } else {
+#pragma unroll
+              for (int j = 0; j < D; ++j) x[k][j] = f.pts[(size_t)pc * f.sp + (size_t)j * f.ld];
+              id[k] = pc;
+            }
             dm[k] = first ? f.init : f.dmin[pc];
           }
           if (base + 64 * P > f.n) {
@@ -685,7 +679,11 @@ __global__ void __launch_bounds__(kRoundsThreads) fps_rounds(RoundsParams a) {
   {D, kRoundsThreads, P, kTieHighest, (const void *)fps_rounds<D, P, kTieHighest>},      \
       {D, kRoundsThreads, P, kTieLowest, (const void *)fps_rounds<D, P, kTieLowest>}
 
-static const KernelEntry kRounds[] = {ROUNDS(3, 1), ROUNDS(3, 4), ROUNDS(3, 8)};
+static const KernelEntry kRounds[] = {
+    ROUNDS(1, 4), ROUNDS(2, 1), ROUNDS(2, 4), ROUNDS(2, 8), ROUNDS(3, 1), ROUNDS(3, 4),
+    ROUNDS(3, 8), ROUNDS(4, 1), ROUNDS(4, 4), ROUNDS(5, 1), ROUNDS(5, 4), ROUNDS(6, 1),
+    ROUNDS(6, 4), ROUNDS(7, 1), ROUNDS(7, 4), ROUNDS(8, 1), ROUNDS(8, 4),
+};
 
 const KernelEntry *rounds_table(size_t *count) {
   *count = sizeof(kRounds) / sizeof(kRounds[0]);

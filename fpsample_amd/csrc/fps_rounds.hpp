@@ -10,10 +10,10 @@ namespace fpsx {
 
 struct RoundsParams {
   FpsParams fps;       // the cloud (original order), picks, exchange area, status, dmin
-  const float *pos;    // coordinate j of position p at pos[p * pos_sp + j * pos_ld]
-  uint64_t pos_sp;
-  uint64_t pos_ld;
-  const uint32_t *perm;  // original index of every position; null: the identity
+  // The points in spatial order: {x, y, z, original index} of every position, and coordinate
+  // j >= 3 at rest[(j - 3) * n + position].  Null: positions are indices, points as in fps.
+  const float4 *rec;
+  const float *rest;
   uint32_t nblocks;      // blocks of 64 * P consecutive positions
   uint32_t cap_wg;       // candidates one workgroup may publish per round
   uint32_t target;       // candidates aimed at per round
@@ -41,5 +41,13 @@ inline size_t rounds_shmem(uint32_t dim, uint32_t nbl) {
 }
 
 const KernelEntry *rounds_table(size_t *count);
+
+// Enqueues the spatial order of a cloud (fps_rounds_order.hip): rec holds n records, rest
+// (dim - 3) * n floats beyond three dimensions.  Returns a FPSX_* code.
+struct RoundsOrderScratch;
+RoundsOrderScratch *new_rounds_order_scratch();
+void delete_rounds_order_scratch(RoundsOrderScratch *s);
+int rounds_order(const float *pts, uint64_t sp, uint64_t ld, uint32_t n, uint32_t dim, float4 *rec,
+                 float *rest, RoundsOrderScratch &scratch, hipStream_t st);
 
 }  // namespace fpsx

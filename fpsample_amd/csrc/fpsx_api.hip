@@ -406,17 +406,25 @@ int plan(Ctx &c, size_t n, size_t dim, int tie, size_t m, Plan &p) {
 //   large ones need fewer box tests.  Kernel ms: uniform 50 K points / 4096 picks at 64
 //   workgroups 0.66 at P = 1, 0.68 at 4 (32 workgroups); uniform 100 K / 50 K picks 3.68 and
 //   3.44 (64), 4.23 at 8 (13); gauss1m / 16384 picks 2.13 at 4 (256), 2.13 at 8 (128).
-//   G: gauss1m 2.53, 2.13 and 2.20 ms at 64, 128 and 256 (P = 8); the 16.7 M-point lattice
-//   4.94 and 4.09 ms at 128 and 256 (early rounds sweep the whole cloud).
+//   G: enough for one block per wave (2^20 8-D points / 256 picks 1.28 ms at 128 workgroups
+//   with two blocks per wave, 0.52 at 256 with one).  Few where the exchange is what counts:
+//   1024 points / 256 picks 151, 172 and 167 us a call at 1, 8 and 16 workgroups; 4096 / 512
+//   473, 265, 236 and 243 at 1, 8, 16 and 32; 8192 / 2048 528, 464, 460 and 466 at 8, 16, 32
+//   and 64; gauss1m 2.53, 2.13 and 2.20 ms at 64, 128 and 256; the 16.7 M-point lattice 4.94
+//   and 4.09 ms at 128 and 256 (early rounds sweep the whole cloud).
 //   target: a round costs about 6 us and 20 ns a candidate, so long runs take more per round:
 //   100 K / 50 K picks 4.05, 3.58, 3.39, 3.23 and 3.20 ms at 128, 160, 192, 224 and 256;
 //   gauss1m 2.13 and 2.08 at 160 and 224; 50 K / 4096 picks 0.69, 0.66, 0.69 and 0.72 at 128,
 //   160, 192 and 224; 4096 / 1024 picks 0.32, 0.33, 0.35 and 0.36 at 96, 128, 160 and 192.
+//   order: its launches cost 23 us up to 8192 points, 50 to 80 up to 2^20, and save updates
+//   once most picks reach few blocks.  Call with and without it, us: 2048 / 512 picks 219 and
+//   214; 4096 / 1024 327 and 352; 8192 / 2048 460 and 533; 65536 / 256 367 and 334; 50 K /
+//   4096 716 and 1008; 2^20 / 256 777 and 712; gauss1m / 16384 2160 and 7746.
 static int plan_rounds(Ctx &c, size_t n, size_t dim, int tie, size_t m, Plan &p) {
   int P = 0, G = 0, target = 0, order = -1;
   if (const char *env = std::getenv("FPSX_ROUNDS"))
     if (*env) std::sscanf(env, "%d:%d:%d:%d", &P, &G, &target, &order);
-  if (P <= 0) P = n <= 65536 ? 1 : n <= 524288 ? 4 : 8;
+  if (P <= 0) P = n <= 65536 && dim != 1 ? 1 : n <= 524288 || dim == 1 || dim > 3 ? 4 : 8;
   size_t cnt;
   const KernelEntry *t = rounds_table(&cnt);
   const KernelEntry *k = nullptr;
@@ -425,7 +433,9 @@ static int plan_rounds(Ctx &c, size_t n, size_t dim, int tie, size_t m, Plan &p)
   if (!k) return fail(FPSX_EINVAL, "no threshold-round kernel for dim " + std::to_string(dim) +
                                        " with " + std::to_string(P) + " points per lane");
   const size_t nblocks = (n + 64 * (size_t)P - 1) / (64 * (size_t)P);
-  size_t g = G > 0 ? (size_t)G : n <= 524288 ? 64 : n <= ((size_t)1 << 22) ? 128 : 256;
+  size_t g = G > 0 ? (size_t)G : n <= 1024 ? 1 : n <= 4096 ? 16 : n <= 16384 ? 32
+             : n <= 524288 ? 64 : n <= ((size_t)1 << 22) ? 128 : 256;
+  if (G <= 0 && n > 1024) g = std::max<size_t>(g, (nblocks + 15) / 16);
   g = std::min<size_t>(std::min<size_t>(g, nblocks), kRoundsMaxGrid);
   const size_t nbl = (nblocks + g - 1) / g;
   const size_t shmem = rounds_shmem((uint32_t)dim, (uint32_t)nbl);
@@ -441,7 +451,8 @@ static int plan_rounds(Ctx &c, size_t n, size_t dim, int tie, size_t m, Plan &p)
   p.target = target > 0 ? std::min<uint32_t>((uint32_t)target, kRoundsCap)
              : m >= 16384 ? 224
                           : (uint32_t)std::min<size_t>(160, std::max<size_t>(64, m / 8));
-  p.order = order >= 0 ? order != 0 : n > 4096;
+  p.order = order >= 0 ? order != 0
+                       : m >= 512 && (double)n * (double)m >= (n <= 8192 ? 1.5e5 : 6e5) * (double)g;
   return FPSX_OK;
 }
 
@@ -450,14 +461,19 @@ static bool env_set(const char *name) {
   return v && *v && std::strcmp(v, "0") != 0;
 }
 
-// Threshold rounds from 4096 points (1024 points, 256 picks: 274 us a call against 232 us by
-// the one-workgroup pass kernel; 4096 points, 1024 picks: 469 against 881 us), unless a pass
-// plan is asked for by name or by the tuner.
+// Threshold rounds from 512 points and 192 picks (64 beyond three dimensions), unless a pass
+// plan is asked for by name or by the tuner: the first picks come one or two a round, at 5 to
+// 10 us, where a pass takes 0.6 to 3 us.  Passes against rounds, us a call: 512 points / 128
+// picks 88 and 85, 1024 / 128 96 and 121, 1024 / 256 181 and 151, 4096 / 128 122 and 136,
+// 4096 / 512 452 and 236, 65536 / 64 146 and 214, 65536 / 256 555 and 334, 2^20 / 256 847
+// and 686; eight dimensions, 4096 / 64 106 and 120, 65536 / 64 207 and 165, 2^20 / 64 456
+// and 251.
 int plan_call(Ctx &c, size_t n, size_t dim, int tie, size_t m, Plan &p) {
   const bool passes = env_set("FPSX_PLAN") || env_set("FPSX_NO_PAIR") || env_set("FPSX_NO_PRUNE") ||
                       env_set("FPSX_NO_ROUNDS") ||
                       c.tuned.find(std::make_tuple(n, dim, tie)) != c.tuned.end();
-  if (!passes && (env_set("FPSX_ROUNDS") || (n >= 4096 && m >= 64)) &&
+  const bool serves = n >= 512 && m >= (dim <= 3 ? 192u : 64u);
+  if (!passes && (env_set("FPSX_ROUNDS") || serves) &&
       plan_rounds(c, n, dim, tie, m, p) == FPSX_OK)
     return FPSX_OK;
   t_err.clear();
@@ -767,24 +783,20 @@ int launch_fps(Ctx &c, const Plan &p, const float *d_pts, size_t sp, size_t ld, 
     a.dmin = (float *)c.dmin.p;
     const uint32_t block = (uint32_t)(64 * p.k->ppt);
     ra.fps = a;
-    ra.pos = d_pts;
-    ra.pos_sp = sp;
-    ra.pos_ld = ld;
-    ra.perm = nullptr;
+    ra.rec = nullptr;
+    ra.rest = nullptr;
     ra.nblocks = (uint32_t)((n + block - 1) / block);
     ra.cap_wg = rounds_cap_wg(p.grid);
     ra.target = p.target;
     if (p.order) {
-      HIP_TRY(c.sorted.reserve(n * 3 * sizeof(float)));
-      HIP_TRY(c.perm.reserve(n * sizeof(uint32_t)));
-      if (!c.spatial) c.spatial = new_spatial_scratch();
-      rc = spatial_order(d_pts, sp, ld, (uint32_t)n, block, (float *)c.sorted.p,
-                         (uint32_t *)c.perm.p, *c.spatial, st);
+      HIP_TRY(c.rec.reserve(n * sizeof(float4)));
+      if (dim > 3) HIP_TRY(c.rest.reserve(n * (dim - 3) * sizeof(float)));
+      if (!c.order) c.order = new_rounds_order_scratch();
+      rc = rounds_order(d_pts, sp, ld, (uint32_t)n, (uint32_t)dim, (float4 *)c.rec.p,
+                        (float *)c.rest.p, *c.order, st);
       if (rc) return rc;
-      ra.pos = (const float *)c.sorted.p;
-      ra.pos_sp = 1;
-      ra.pos_ld = n;
-      ra.perm = (const uint32_t *)c.perm.p;
+      ra.rec = (const float4 *)c.rec.p;
+      ra.rest = (const float *)c.rest.p;
     }
     rc = dispatch(c, p, &ra, st);
     if (rc) return rc;

@@ -56,6 +56,8 @@ struct Ctx {
   std::mutex mu;
   DevBuf pts, rows, starts, out, xchg, status, dmin, sorted, perm;
   struct SpatialScratch *spatial = nullptr;
+  DevBuf rec, rest;  // threshold rounds: the points in spatial order
+  struct RoundsOrderScratch *order = nullptr;
   std::map<std::pair<const void *, size_t>, int> occ;  // co-resident workgroups per kernel
   int max_blocks(const KernelEntry *k, size_t shmem);
   // Autotuned plans: (n_points, dim, tie) -> the plan the tuner chose.

@@ -88,6 +88,39 @@ def test_rounds_ties_special_values_and_prefixes(gpu, rounds_env, shape):
 def test_rounds_planner_sizes(gpu):
     # The planner's own shapes on both sides of each of its lines.
     rng = np.random.default_rng(62)
-    for n, m in ((4096, 64), (65536, 1500), (65537, 1500), (524288, 600), (524289, 600),
-                 ((1 << 22) + 1, 100)):
-        check(rng.random((n, 3)).astype(np.float32), m, int(rng.integers(n)), "planner")
+    for n, d, m in ((512, 3, 192), (512, 8, 64), (1024, 3, 256), (1025, 3, 600), (4097, 3, 600),
+                    (8193, 3, 700), (16385, 2, 600), (65536, 3, 1500), (65537, 3, 1500),
+                    (262145, 3, 300), (524289, 3, 600), (300000, 7, 70), ((1 << 22) + 1, 3, 192)):
+        check(rng.random((n, d)).astype(np.float32), m, int(rng.integers(n)), "planner")
+
+
+@pytest.mark.parametrize("d", [1, 2, 4, 5, 6, 7, 8])
+def test_rounds_dimensions(gpu, rounds_env, d):
+    # Every dimension with a kernel, one and several blocks per wave, with and without order.
+    rng = np.random.default_rng(63 + d)
+    for shape in ("4:3:100:1" if d == 1 else "1:40:100:1", "4:2:160:1", "4:64:60:0"):
+        rounds_env(shape)
+        check(rng.random((9001, d)).astype(np.float32), 900, int(rng.integers(9001)), "uniform")
+        check(rng.integers(0, 4, (3000, d)).astype(np.float32), 1500, 5, "lattice")
+        sp = (rng.random((3000, d)) * 4e19).astype(np.float32)
+        sp[[7, 900]] = np.nan
+        sp[11, d - 1] = np.inf
+        check(sp, 300, 1, "special")
+
+
+@pytest.mark.parametrize("n", [8191, 8192, 8193, 20000, 70001])
+def test_rounds_order_sizes(gpu, rounds_env, n):
+    # The order's one-workgroup form, its last size, several chunks, a ragged last chunk;
+    # clouds in one bucket but for an outlier, on a line, and with values it cannot place.
+    rounds_env("1:16:160:1")
+    rng = np.random.default_rng(n)
+    tight = (0.5 + 1e-4 * rng.random((n, 3))).astype(np.float32)
+    tight[n // 2] = 1e6
+    line = np.zeros((n, 3), np.float32)
+    line[:, 1] = rng.random(n)
+    odd = rng.random((n, 3)).astype(np.float32)
+    odd[[3, n - 1], 0] = np.nan
+    odd[5, 2] = np.inf
+    odd[6] = -np.inf
+    for name, pc in (("tight", tight), ("line", line), ("odd", odd)):
+        check(pc, 400, 9, name)
