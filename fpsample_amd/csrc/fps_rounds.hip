@@ -74,60 +74,76 @@ struct alignas(16) Rec {
   float c[(D + 3) / 4 * 4];
 };
 
+// LDS of a workgroup beside its blocks' boxes and best keys.
+template <int D>
+struct RoundsLds {
+  static constexpr int CAP = (int)kRoundsCap;    // candidates the front decides on
+  static constexpr int LIST = (int)kRoundsList;  // candidates that may come in
+  static constexpr int W = kRoundsThreads / 64;
+  alignas(16) uint64_t ck[LIST];  // candidates as they came
+  Rec<D> cc[LIST];
+  Rec<D> pk[CAP];                 // picks of the round
+  uint32_t pt[CAP];               // their tie words
+  uint32_t rank[LIST];
+  uint64_t sk[CAP];               // sorted candidates
+  Rec<D> sc[CAP];
+  uint16_t low[CAP / 32][CAP][2];  // rows: which earlier candidates lower this one
+  uint64_t lk[CAP];                // this workgroup's candidates
+  Rec<D> lc[CAP];
+  uint32_t cnt[2];  // candidates of this workgroup, by round parity
+  uint32_t sum[2];  // candidates of the grid, by round parity
+  uint32_t at[2];   // candidates taken in, by round parity
+  uint64_t wmax[W];
+  uint64_t acc[CAP / 64];
+  uint64_t te;    // the bound that the round's picks exceed
+  uint32_t stop;  // first pick that does not lower itself
+  uint64_t last;  // key of the round's last pick
+  uint32_t np;
+  uint32_t stuck;
+  uint32_t ok;
+};
+
+// Workgroup `group` of G working on one cloud: picks a.s_begin .. a.s_end - 1.
 template <int D, int P, int TIE>
-__global__ void __launch_bounds__(kRoundsThreads) fps_rounds(RoundsParams a) {
-  constexpr int W = kRoundsThreads / 64;
-  constexpr int CAP = (int)kRoundsCap;        // candidates the front decides on
-  constexpr int LIST = (int)kRoundsList;      // candidates that may come in
+__device__ __forceinline__ void rounds_cloud(const RoundsParams &a, const uint32_t group,
+                                             const uint32_t G, RoundsLds<D> &S, uint64_t *s_dyn) {
+  constexpr int W = RoundsLds<D>::W;
+  constexpr int CAP = RoundsLds<D>::CAP;
+  constexpr int LIST = RoundsLds<D>::LIST;
   constexpr int CH = CAP / 64;
   constexpr uint32_t NWC = 2 + D;
-  extern __shared__ uint64_t s_dyn[];  // best key of every block, then the boxes
-
-  __shared__ alignas(16) uint64_t s_ck[LIST];  // candidates as they came
-  __shared__ Rec<D> s_cc[LIST];
-  __shared__ Rec<D> s_pk[CAP];        // picks of the round
-  __shared__ uint32_t s_pt[CAP];      // their tie words
-  __shared__ uint32_t s_rank[LIST];
-  __shared__ uint64_t s_sk[CAP];      // sorted candidates
-  __shared__ Rec<D> s_sc[CAP];
-  __shared__ uint16_t s_low[CAP / 32][CAP][2];  // rows: which earlier candidates lower this one
-  __shared__ uint64_t s_lk[CAP];  // this workgroup's candidates
-  __shared__ Rec<D> s_lc[CAP];
-  __shared__ uint32_t s_cnt[2];  // candidates of this workgroup, by round parity
-  __shared__ uint32_t s_sum[2];  // candidates of the grid, by round parity
-  __shared__ uint32_t s_at[2];   // candidates taken in, by round parity
-  __shared__ uint64_t s_wmax[W];
-  __shared__ uint64_t s_acc[CH];
-  __shared__ uint64_t s_te;    // the bound that the round's picks exceed
-  __shared__ uint32_t s_stop;  // first pick that does not lower itself
-  __shared__ uint32_t s_np;
-  __shared__ uint32_t s_stuck;
-  __shared__ uint32_t s_ok;
-
   const FpsParams &f = a.fps;
   int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const uint32_t G = gridDim.x;
-  uint32_t g = blockIdx.x;
-  const uint32_t nbl = (a.nblocks - g + G - 1) / G;  // this workgroup's blocks: g, g + G, ...
+  const uint32_t nbl = (a.nblocks - group + G - 1) / G;  // blocks group, group + G, ...
   const bool resident = nbl <= (uint32_t)W;          // a block per wave stays in registers
   uint64_t *s_bkey = s_dyn;
   float *s_box = (float *)(s_dyn + nbl);  // [2 * D][nbl]
 
   if (tid == 0) {
-    s_cnt[0] = s_cnt[1] = 0;
-    s_sum[0] = s_sum[1] = 0;
-    s_at[0] = s_at[1] = 0;
-    s_stuck = 0;
-    s_ok = 1;
+    S.last = ~0ull;
+    S.cnt[0] = S.cnt[1] = 0;
+    S.sum[0] = S.sum[1] = 0;
+    S.at[0] = S.at[1] = 0;
+    S.stuck = 0;
+    S.ok = 1;
   }
 
-  uint32_t s = 0;        // picks recorded
-  uint32_t np = 0;       // picks of the last round, in s_pk
-  bool first = true;
+  if (a.s_begin) lds_barrier();  // (a fresh run has one after its forced picks)
+
+  uint32_t s = a.s_begin;  // picks recorded
+  uint32_t np = 0;         // picks of the last round, in S.pk
+  bool first = true;       // the blocks have not been read yet
+  bool last = false;       // the picks are made: apply them and save
   uint64_t T = ~0ull;    // every point's key is at most T
   uint64_t Tg = ~0ull;   // the round's bound
   uint64_t step = (uint64_t)1 << 51;  // a sixteenth of a binade
+  if (a.s_begin) {
+    // A run taken up again: no key exceeds that of its last pick.
+    T = uniform_u64(((uint64_t)a.carry[0] << 32) | a.carry[1]);
+    step = uniform_u64(((uint64_t)a.carry[2] << 32) | a.carry[3]);
+    Tg = T > step ? T - step : 0;
+  }
   uint32_t e = 0;        // rounds
   uint32_t idle = 0;     // rounds since the last pick
   float x[P][D], dm[P];  // the block in hand
@@ -136,51 +152,67 @@ __global__ void __launch_bounds__(kRoundsThreads) fps_rounds(RoundsParams a) {
   for (;;) {
     // Rewritten each round: addresses formed from them would otherwise be kept in registers
     // over the whole loop, beside the block.
-    asm volatile("" : "+v"(tid), "+s"(g));
+    asm volatile("" : "+v"(tid));
+    uint32_t g = (uint32_t)__builtin_amdgcn_readfirstlane((int)group);
+    asm volatile("" : "+s"(g));
     const int lane = tid & 63;
     // ---- forced picks, in pieces of CAP -------------------------------------
     if (s < f.n_starts) {
       np = min(f.n_starts - s, (uint32_t)CAP);
       if ((uint32_t)tid < np) {
-        uint64_t idx = f.starts[s + tid];
+        uint64_t idx = f.starts ? f.starts[s + tid] : a.start;
         if (idx >= f.n) {
           atomicOr(f.status, kStatusBadStart);
           idx = 0;
         }
 #pragma unroll
-        for (int j = 0; j < D; ++j) s_pk[tid].c[j] = f.pts[(size_t)idx * f.sp + (size_t)j * f.ld];
-        s_pt[tid] = tie_of<TIE>((uint32_t)idx);
+        for (int j = 0; j < D; ++j) S.pk[tid].c[j] = f.pts[(size_t)idx * f.sp + (size_t)j * f.ld];
+        S.pt[tid] = tie_of<TIE>((uint32_t)idx);
       }
       lds_barrier();
     }
     // ---- record -------------------------------------------------------------
     if (g == 0) {
       if ((uint32_t)tid < np) {
-        f.out[s + tid] = tie_of<TIE>(s_pt[tid]);
+        f.out[s + tid] = tie_of<TIE>(S.pt[tid]);
         if (f.out_pts != nullptr) {
 #pragma unroll
-          for (int j = 0; j < D; ++j) f.out_pts[(size_t)(s + tid) * D + j] = s_pk[tid].c[j];
+          for (int j = 0; j < D; ++j) f.out_pts[(size_t)(s + tid) * D + j] = S.pk[tid].c[j];
         }
       }
       if (tid == 0) f.status[1] = e;
     }
     s += np;
     if (s >= f.m) return;
-    if (s_stuck) {
+    if (s >= a.s_end) {
+      last = true;
+      if (g == 0 && tid == 0) {
+        a.carry[0] = (uint32_t)(S.last >> 32);
+        a.carry[1] = (uint32_t)S.last;
+        a.carry[2] = (uint32_t)(step >> 32);
+        a.carry[3] = (uint32_t)step;
+      }
+    } else if (np && __builtin_amdgcn_readfirstlane((int)S.stuck)) {
       // The last pick left its own key unchanged, so it stays the best for good.
       if (g == 0) {
-        const uint32_t t = s_pt[np - 1];
-        for (uint32_t q = s + tid; q < f.m; q += kRoundsThreads) {
+        const uint32_t t = S.pt[np - 1];
+        for (uint32_t q = s + tid; q < a.s_end; q += kRoundsThreads) {
           f.out[q] = tie_of<TIE>(t);
           if (f.out_pts != nullptr) {
 #pragma unroll
-            for (int j = 0; j < D; ++j) f.out_pts[(size_t)q * D + j] = s_pk[np - 1].c[j];
+            for (int j = 0; j < D; ++j) f.out_pts[(size_t)q * D + j] = S.pk[np - 1].c[j];
           }
         }
       }
-      return;
+      if (a.s_end >= f.m) return;
+      last = true;  // (the picks so far are applied below; repeating the last changes nothing)
+      if (g == 0 && tid == 0) {
+        a.carry[0] = a.carry[1] = ~0u;
+        a.carry[2] = (uint32_t)(step >> 32);
+        a.carry[3] = (uint32_t)step;
+      }
     }
-    const bool gather = s >= f.n_starts;  // no further forced picks
+    const bool gather = s >= f.n_starts && !last;  // no further forced picks
     if (!gather) Tg = ~0ull;
 
     // ---- 1. update ----------------------------------------------------------
@@ -194,7 +226,7 @@ __global__ void __launch_bounds__(kRoundsThreads) fps_rounds(RoundsParams a) {
 #pragma unroll
       for (int c = 0; c < CH; ++c) hit[c] = 0;
       uint64_t bkey = 0;
-      bool any = first;
+      bool any = first || last;
       if (first) {
 #pragma unroll
         for (int c = 0; c < CH; ++c) {
@@ -213,7 +245,7 @@ __global__ void __launch_bounds__(kRoundsThreads) fps_rounds(RoundsParams a) {
 #pragma unroll
         for (int c = 0; c < CH; ++c) {
           if ((uint32_t)c < nch) {
-            const Rec<D> r = s_pk[c * 64 + lane];
+            const Rec<D> r = S.pk[c * 64 + lane];
             float p[D];
 #pragma unroll
             for (int j = 0; j < D; ++j) p[j] = r.c[j];
@@ -240,7 +272,7 @@ __global__ void __launch_bounds__(kRoundsThreads) fps_rounds(RoundsParams a) {
               for (int j = 0; j < D; ++j) x[k][j] = f.pts[(size_t)pc * f.sp + (size_t)j * f.ld];
               id[k] = pc;
             }
-            dm[k] = first ? f.init : f.dmin[pc];
+            dm[k] = first && a.s_begin == 0 ? f.init : f.dmin[pc];
           }
           if (base + 64 * P > f.n) {
 #pragma unroll
@@ -271,7 +303,7 @@ __global__ void __launch_bounds__(kRoundsThreads) fps_rounds(RoundsParams a) {
           for (int c = 0; c < CH; ++c) {
             uint64_t mm = hit[c];
             if (mm) {
-              const Rec<D> r = s_pk[c * 64 + lane];
+              const Rec<D> r = S.pk[c * 64 + lane];
               do {
                 const int l = __ffsll((unsigned long long)mm) - 1;
                 mm &= mm - 1;
@@ -283,7 +315,7 @@ __global__ void __launch_bounds__(kRoundsThreads) fps_rounds(RoundsParams a) {
               } while (mm);
             }
           }
-          if (!resident) {
+          if (!resident || last) {
 #pragma unroll
             for (int k = 0; k < P; ++k) {
               const uint32_t p = base + (uint32_t)(k * 64 + lane);
@@ -316,17 +348,17 @@ __global__ void __launch_bounds__(kRoundsThreads) fps_rounds(RoundsParams a) {
             total += (uint32_t)__popcll(m[k]);
           }
           uint32_t at = 0;
-          if (lane == 0) at = atomicAdd(&s_cnt[(e + 1) & 1], total);
+          if (lane == 0) at = atomicAdd(&S.cnt[(e + 1) & 1], total);
           at = (uint32_t)__builtin_amdgcn_readfirstlane((int)at);
 #pragma unroll
           for (int k = 0; k < P; ++k) {
             const uint32_t q = at + lanes_below(m[k]);
             if (((m[k] >> lane) & 1) && q < (uint32_t)CAP) {
-              s_lk[q] = make_key(__float_as_int(dm[k]), tie_of<TIE>(id[k]));
+              S.lk[q] = make_key(__float_as_int(dm[k]), tie_of<TIE>(id[k]));
               Rec<D> r;
 #pragma unroll
               for (int j = 0; j < D; ++j) r.c[j] = x[k][j];
-              s_lc[q] = r;
+              S.lc[q] = r;
             }
             at += (uint32_t)__popcll(m[k]);
           }
@@ -335,24 +367,25 @@ __global__ void __launch_bounds__(kRoundsThreads) fps_rounds(RoundsParams a) {
       wmax = bkey > wmax ? bkey : wmax;
     }
     first = false;
+    if (last) return;
     if (!gather) {
       lds_barrier();
       continue;
     }
-    if (lane == 0) s_wmax[wave] = wmax;
+    if (lane == 0) S.wmax[wave] = wmax;
     if (tid < LIST) {
-      s_ck[tid] = 0;
-      s_rank[tid] = 0;
+      S.ck[tid] = 0;
+      S.rank[tid] = 0;
     }
     if (tid == 0) {
-      s_te = Tg;
-      s_stop = ~0u;
+      S.te = Tg;
+      S.stop = ~0u;
     }
     lds_barrier();
     ++e;
     const uint32_t par = e & 1u;
-    const uint32_t own = s_cnt[par];
-    uint64_t U = wave_max_u64(lane < W ? s_wmax[lane] : 0ull);  // this workgroup's best key
+    const uint32_t own = S.cnt[par];
+    uint64_t U = wave_max_u64(lane < W ? S.wmax[lane] : 0ull);  // this workgroup's best key
 
     // ---- 2. exchange --------------------------------------------------------
     // L lanes read one workgroup's header and its first L candidates at once, so most
@@ -360,7 +393,8 @@ __global__ void __launch_bounds__(kRoundsThreads) fps_rounds(RoundsParams a) {
     uint32_t C = own;
     if (G > 1) {
       const uint32_t capw = a.cap_wg;
-      const size_t head = (size_t)kRoundsReplicas * kRoundsHeadWords * kRoundsMaxGrid;
+      const uint32_t hp = G;  // pitch of one header word's array
+      const size_t head = (size_t)kRoundsReplicas * kRoundsHeadWords * hp;
       const size_t cp = (size_t)G * capw;  // pitch of one word's array
       uint64_t *buf = f.xchg + (size_t)par * (head + NWC * cp);
       uint64_t *cbuf = buf + head;
@@ -369,13 +403,13 @@ __global__ void __launch_bounds__(kRoundsThreads) fps_rounds(RoundsParams a) {
           const uint32_t rep = (uint32_t)lane / kRoundsHeadWords;
           const uint32_t k = (uint32_t)lane - rep * kRoundsHeadWords;
           const uint32_t v = k == 0 ? own : (k == 1 ? (uint32_t)(U >> 32) : (uint32_t)U);
-          xchg_store(buf + ((size_t)rep * kRoundsHeadWords + k) * kRoundsMaxGrid + g,
+          xchg_store(buf + ((size_t)rep * kRoundsHeadWords + k) * hp + g,
                      ((uint64_t)v << 32) | e);
         }
       } else if (own <= capw) {
         for (uint32_t q = (uint32_t)tid - 64; q < own; q += kRoundsThreads - 64) {
-          const uint64_t k = s_lk[q];
-          const Rec<D> r = s_lc[q];
+          const uint64_t k = S.lk[q];
+          const Rec<D> r = S.lc[q];
           uint64_t *w = cbuf + (size_t)g * capw + q;
           xchg_store(w, (k & 0xffffffff00000000ull) | e);
           xchg_store(w + cp, (k << 32) | e);
@@ -391,7 +425,7 @@ __global__ void __launch_bounds__(kRoundsThreads) fps_rounds(RoundsParams a) {
       uint64_t w1 = 0, w2 = 0;
       if ((uint32_t)wave * 64 < G * L) {
         const uint64_t *h =
-            buf + (size_t)(g % kRoundsReplicas) * kRoundsHeadWords * kRoundsMaxGrid + q;
+            buf + (size_t)(g % kRoundsReplicas) * kRoundsHeadWords * hp + q;
         const uint64_t *w = cbuf + (size_t)q * capw;
         uint32_t cq = 0;
         uint64_t v[NWC];
@@ -401,8 +435,8 @@ __global__ void __launch_bounds__(kRoundsThreads) fps_rounds(RoundsParams a) {
           const uint64_t deadline = now_ticks() + f.spin_ticks;
           for (;;) {
             const uint64_t w0 = xchg_load(h);
-            w1 = xchg_load(h + kRoundsMaxGrid);
-            w2 = xchg_load(h + 2 * kRoundsMaxGrid);
+            w1 = xchg_load(h + hp);
+            w2 = xchg_load(h + 2 * hp);
 #pragma unroll
             for (uint32_t k = 0; k < NWC; ++k) v[k] = xchg_load(w + l + k * cp);
             bool all = true;
@@ -412,7 +446,7 @@ __global__ void __launch_bounds__(kRoundsThreads) fps_rounds(RoundsParams a) {
             here = l < cq && cq <= capw;
             if ((uint32_t)w0 == e && (uint32_t)w1 == e && (uint32_t)w2 == e && (all || !here)) break;
             if (now_ticks() > deadline) {
-              s_ok = 0;
+              S.ok = 0;
               cq = 0;
               here = false;
               break;
@@ -421,20 +455,20 @@ __global__ void __launch_bounds__(kRoundsThreads) fps_rounds(RoundsParams a) {
         }
         const uint32_t sum =
             (uint32_t)__builtin_amdgcn_readlane((int)wave_scan_add(l == 0 ? cq : 0u), 63);
-        if (lane == 0 && sum) atomicAdd(&s_sum[par], sum);
+        if (lane == 0 && sum) atomicAdd(&S.sum[par], sum);
         uint32_t i = l;
         for (;;) {
           const uint64_t m = __ballot(here);
           if (!m) break;
           uint32_t at = 0;
-          if (lane == 0) at = atomicAdd(&s_at[par], (uint32_t)__popcll(m));
+          if (lane == 0) at = atomicAdd(&S.at[par], (uint32_t)__popcll(m));
           at = (uint32_t)__builtin_amdgcn_readfirstlane((int)at) + lanes_below(m);
           if (here && at < (uint32_t)LIST) {
-            s_ck[at] = (v[0] & 0xffffffff00000000ull) | (v[1] >> 32);
+            S.ck[at] = (v[0] & 0xffffffff00000000ull) | (v[1] >> 32);
             Rec<D> r;
 #pragma unroll
             for (int j = 0; j < D; ++j) r.c[j] = __int_as_float((int)(v[2 + j] >> 32));
-            s_cc[at] = r;
+            S.cc[at] = r;
           }
           i += L;
           here = here && i < cq;
@@ -448,7 +482,7 @@ __global__ void __launch_bounds__(kRoundsThreads) fps_rounds(RoundsParams a) {
               for (uint32_t k = 0; k < NWC; ++k) all = all && (uint32_t)v[k] == e;
               if (all) break;
               if (now_ticks() > deadline) {
-                s_ok = 0;
+                S.ok = 0;
                 here = false;
                 break;
               }
@@ -457,33 +491,33 @@ __global__ void __launch_bounds__(kRoundsThreads) fps_rounds(RoundsParams a) {
         }
       }
       lds_barrier();
-      if (!s_ok) {
+      if (!__builtin_amdgcn_readfirstlane((int)S.ok)) {
         if (tid == 0) atomicOr(f.status, kStatusTimeout);
         return;
       }
-      C = s_sum[par];
-      const uint32_t got = s_at[par];
+      C = S.sum[par];
+      const uint32_t got = S.at[par];
       if (got != C || C > (uint32_t)LIST) C = max(C, (uint32_t)LIST + 1);  // some did not fit
       if (C == 0) {
         // Nobody has a candidate: the best key of all is the exact bound.
         const uint64_t u = wave_max_u64((w1 & 0xffffffff00000000ull) | (w2 >> 32));
-        if (lane == 0) s_wmax[wave] = (uint32_t)wave * 64 < G * L ? u : 0ull;
+        if (lane == 0) S.wmax[wave] = (uint32_t)wave * 64 < G * L ? u : 0ull;
         lds_barrier();
-        U = wave_max_u64(lane < W ? s_wmax[lane] : 0ull);
+        U = wave_max_u64(lane < W ? S.wmax[lane] : 0ull);
       }
     } else {
       if ((uint32_t)tid < own && tid < CAP) {
-        s_ck[tid] = s_lk[tid];
-        s_cc[tid] = s_lc[tid];
+        S.ck[tid] = S.lk[tid];
+        S.cc[tid] = S.lc[tid];
       }
       if (own > (uint32_t)CAP) C = max(own, (uint32_t)LIST + 1);
       lds_barrier();
     }
     if (tid == 0) {  // the other parity's counters: everybody has read them
-      s_np = 0;
-      s_cnt[par ^ 1] = 0;
-      s_sum[par ^ 1] = 0;
-      s_at[par ^ 1] = 0;
+      S.np = 0;
+      S.cnt[par ^ 1] = 0;
+      S.sum[par ^ 1] = 0;
+      S.at[par ^ 1] = 0;
     }
     U = uniform_u64(U);
     C = (uint32_t)__builtin_amdgcn_readfirstlane((int)C);
@@ -516,25 +550,25 @@ __global__ void __launch_bounds__(kRoundsThreads) fps_rounds(RoundsParams a) {
       for (uint32_t job = wave; job < nc * nj; job += W) {
         const uint32_t jc = job / nc, ic = job - jc * nc;
         const uint32_t i = ic * 64 + lane;
-        const uint64_t ki = s_ck[i];
-        const uint64_t *kj = s_ck + jc * 16;
+        const uint64_t ki = S.ck[i];
+        const uint64_t *kj = S.ck + jc * 16;
         uint32_t r = 0;
 #pragma unroll 1
         for (int h = 0; h < 16; h += 8) {
 #pragma unroll
           for (int l = 0; l < 8; ++l) r += kj[h + l] > ki ? 1u : 0u;
         }
-        if (i < C && r) atomicAdd(&s_rank[i], r);
+        if (i < C && r) atomicAdd(&S.rank[i], r);
       }
     }
     lds_barrier();
     if ((uint32_t)tid < C) {
-      const uint32_t r = s_rank[tid];
+      const uint32_t r = S.rank[tid];
       if (r < (uint32_t)CAP) {
-        s_sk[r] = s_ck[tid];
-        s_sc[r] = s_cc[tid];
+        S.sk[r] = S.ck[tid];
+        S.sc[r] = S.cc[tid];
       } else if (r == (uint32_t)CAP) {
-        s_te = s_ck[tid];  // the first one that the front does not see is the bound
+        S.te = S.ck[tid];  // the first one that the front does not see is the bound
       }
     }
     lds_barrier();
@@ -551,8 +585,8 @@ __global__ void __launch_bounds__(kRoundsThreads) fps_rounds(RoundsParams a) {
       const uint32_t j0 = job * 16;
       if (j0 < F) {
         const uint32_t i = c * 64 + lane;
-        const float v = __int_as_float((int)(uint32_t)(s_sk[i] >> 32) - 1);
-        const Rec<D> ri = s_sc[i];
+        const float v = __int_as_float((int)(uint32_t)(S.sk[i] >> 32) - 1);
+        const Rec<D> ri = S.sc[i];
         float xi[D];
 #pragma unroll
         for (int j = 0; j < D; ++j) xi[j] = ri.c[j];
@@ -561,21 +595,21 @@ __global__ void __launch_bounds__(kRoundsThreads) fps_rounds(RoundsParams a) {
         for (int h = 12; h >= 0; h -= 4) {
 #pragma unroll
           for (int l = 3; l >= 0; --l) {
-            const Rec<D> rj = s_sc[j0 + h + l];
+            const Rec<D> rj = S.sc[j0 + h + l];
             float p[D];
 #pragma unroll
             for (int j = 0; j < D; ++j) p[j] = rj.c[j];
             bits = bits + bits + (sqdist<D>(xi, p) < v ? 1u : 0u);
           }
         }
-        s_low[job >> 1][i][job & 1] = (uint16_t)bits;
+        S.low[job >> 1][i][job & 1] = (uint16_t)bits;
       }
       job += W;
     }
     lds_barrier();
     // The picks, were no candidate only partly lowered: each candidate that no earlier pick
     // lowers, settled in a few steps per 64 candidates rather than one by one.
-    const uint32_t *rows = (const uint32_t *)&s_low[0][0][0];
+    const uint32_t *rows = (const uint32_t *)&S.low[0][0][0];
     if (wave == 0) {
       uint64_t low[CH][CH];
 #pragma unroll
@@ -601,7 +635,7 @@ __global__ void __launch_bounds__(kRoundsThreads) fps_rounds(RoundsParams a) {
             open &= ~__ballot((same & free) != 0);
           }
         }
-        if (lane == 0) s_acc[c] = acc[c];
+        if (lane == 0) S.acc[c] = acc[c];
       }
     }
     lds_barrier();
@@ -612,13 +646,13 @@ __global__ void __launch_bounds__(kRoundsThreads) fps_rounds(RoundsParams a) {
     Rec<D> ri;
     if ((uint32_t)wave < nc) {
       const uint32_t i = (uint32_t)tid;
-      key = s_sk[i];
-      ri = s_sc[i];
+      key = S.sk[i];
+      ri = S.sc[i];
       const float v = __int_as_float((int)(uint32_t)(key >> 32) - 1);
       float xi[D];
 #pragma unroll
       for (int j = 0; j < D; ++j) xi[j] = ri.c[j];
-      taken = uniform_u64(s_acc[wave]);
+      taken = uniform_u64(S.acc[wave]);
       const bool mine = (taken >> lane) & 1;
       int by = -1;
 #pragma unroll
@@ -626,44 +660,46 @@ __global__ void __launch_bounds__(kRoundsThreads) fps_rounds(RoundsParams a) {
         if (w <= wave) {
           uint64_t k = ((uint64_t)rows[(2 * w + 1) * CAP + i] << 32) | rows[2 * w * CAP + i];
           if (w == wave) k &= ((uint64_t)1 << lane) - 1;
-          k &= s_acc[w];
+          k &= S.acc[w];
           if (k) by = w * 64 + __ffsll((unsigned long long)k) - 1;
         }
       }
       if (i < F && !mine && by >= 0) {
-        const Rec<D> rb = s_sc[by];
+        const Rec<D> rb = S.sc[by];
         float p[D];
 #pragma unroll
         for (int j = 0; j < D; ++j) p[j] = rb.c[j];
         const uint64_t nk = make_key(__float_as_int(sqdist<D>(xi, p)), (uint32_t)key);
-        if (nk > Tg) atomicMax((unsigned long long *)&s_te, (unsigned long long)nk);
+        if (nk > Tg) atomicMax((unsigned long long *)&S.te, (unsigned long long)nk);
       }
-      if (i < F && mine && !(sqdist<D>(xi, xi) < v)) atomicMin(&s_stop, i);
+      if (i < F && mine && !(sqdist<D>(xi, xi) < v)) atomicMin(&S.stop, i);
     }
     lds_barrier();
-    T = uniform_u64(s_te);
+    T = uniform_u64(S.te);
     if ((uint32_t)wave < nc) {
-      const uint32_t stop = s_stop;
+      const uint32_t stop = S.stop;
       // Keys fall along the chunks: a chunk with picks has those before it whole.
       uint32_t at = 0;
-      for (int w = 0; w < wave; ++w) at += (uint32_t)__popcll(s_acc[w]);
+      for (int w = 0; w < wave; ++w) at += (uint32_t)__popcll(S.acc[w]);
       taken &= __ballot(key > T && (uint32_t)tid <= stop);
       at = (uint32_t)__builtin_amdgcn_readfirstlane((int)at);
-      const uint32_t room = f.m - s;
+      const uint32_t room = a.s_end - s;
       if (taken) {
         const uint32_t q = at + lanes_below(taken);
+        const uint32_t upto = min(at + (uint32_t)__popcll(taken), room);
         if (((taken >> lane) & 1) && q < room) {
-          s_pt[q] = (uint32_t)key;
-          s_pk[q] = ri;
+          S.pt[q] = (uint32_t)key;
+          S.pk[q] = ri;
+          if (q == room - 1) S.last = key;
         }
-        if (lane == 0) atomicMax(&s_np, min(at + (uint32_t)__popcll(taken), room));
+        if (lane == 0) atomicMax(&S.np, upto);
         if (stop - (uint32_t)wave * 64 < 64u && ((taken >> (stop & 63u)) & 1) && lane == 0)
-          s_stuck = 1;
+          S.stuck = 1;
       }
     }
     lds_barrier();
     idle = 0;
-    np = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_np);
+    np = (uint32_t)__builtin_amdgcn_readfirstlane((int)S.np);
     {
       // The square root damps the step against the count's own noise.
       double r = sqrt((double)a.target / (double)C);
@@ -672,6 +708,69 @@ __global__ void __launch_bounds__(kRoundsThreads) fps_rounds(RoundsParams a) {
       step = ns < 1.0 ? 1 : (ns > 4.0e18 ? (uint64_t)1 << 61 : (uint64_t)ns);
       Tg = T > step ? T - step : 0;
     }
+  }
+}
+
+template <int D, int P, int TIE>
+__global__ void __launch_bounds__(kRoundsThreads) fps_rounds(RoundsParams a) {
+  extern __shared__ uint64_t s_dyn[];
+  __shared__ RoundsLds<D> S;
+  rounds_cloud<D, P, TIE>(a, blockIdx.x, gridDim.x, S, s_dyn);
+}
+
+// A table entry in scalar registers: read in place, its fields would come through vector
+// loads again after every store.
+__device__ __forceinline__ RoundsParams uniform_params(const RoundsParams *p) {
+  constexpr int N = sizeof(RoundsParams) / 4;
+  union {
+    RoundsParams a;
+    uint32_t w[N];
+  } u;
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+    u.w[i] = (uint32_t)__builtin_amdgcn_readfirstlane((int)((const uint32_t *)p)[i]);
+  return u.a;
+}
+
+// Many clouds: workgroups claim member slots in order (or own one each), a job's members
+// being consecutive slots.  A team's workgroups all claim before any waits for another: each
+// claims its next slot only when done with the one before, so the first unfinished team is
+// always complete or about to be.
+template <int D, int P>
+__global__ void __launch_bounds__(kRoundsThreads) fps_rounds_jobs(RoundsJobs j) {
+  extern __shared__ uint64_t s_dyn[];
+  __shared__ RoundsLds<D> S;
+  __shared__ uint32_t s_slot;
+  for (;;) {
+    if (threadIdx.x == 0) s_slot = j.one_slot ? blockIdx.x : atomicAdd(j.claim, 1u);
+    __syncthreads();
+    const uint32_t slot = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_slot);
+    if (slot >= j.members) return;
+    const RoundsParams a = uniform_params(
+        j.table + (uint32_t)__builtin_amdgcn_readfirstlane((int)j.member_job[slot]));
+    if (a.team > 1) {
+      // Wait for the team to form, so that exchange waits are short ones.
+      if (threadIdx.x == 0) {
+        atomicAdd(a.ready, 1u);
+        const uint64_t deadline = now_ticks() + j.team_ticks;
+        uint32_t here = 1;
+        while (__hip_atomic_load(a.ready, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < a.team) {
+          if (now_ticks() > deadline) {
+            atomicOr(a.fps.status, kStatusTimeout);
+            here = 0;
+            break;
+          }
+          __builtin_amdgcn_s_sleep(1);
+        }
+        s_slot = here;
+      }
+      __syncthreads();
+      if (!__builtin_amdgcn_readfirstlane((int)s_slot)) return;
+    }
+    rounds_cloud<D, P, kTieHighest>(
+        a, (uint32_t)__builtin_amdgcn_readfirstlane((int)(slot - a.member_base)), a.team, S, s_dyn);
+    if (j.one_slot) return;
+    __syncthreads();
   }
 }
 
@@ -684,6 +783,14 @@ static const KernelEntry kRounds[] = {
     ROUNDS(3, 8), ROUNDS(4, 1), ROUNDS(4, 4), ROUNDS(5, 1), ROUNDS(5, 4), ROUNDS(6, 1),
     ROUNDS(6, 4), ROUNDS(7, 1), ROUNDS(7, 4), ROUNDS(8, 1), ROUNDS(8, 4),
 };
+
+#define JOBS(D) {D, kRoundsThreads, 4, kTieHighest, (const void *)fps_rounds_jobs<D, 4>}
+
+static const KernelEntry kJobs[] = {JOBS(1), JOBS(2), JOBS(3), JOBS(4)};
+
+const KernelEntry *rounds_jobs_kernel(int dim) {
+  return dim >= 1 && dim <= 4 ? &kJobs[dim - 1] : nullptr;
+}
 
 const KernelEntry *rounds_table(size_t *count) {
   *count = sizeof(kRounds) / sizeof(kRounds[0]);

@@ -17,6 +17,24 @@ struct RoundsParams {
   uint32_t nblocks;      // blocks of 64 * P consecutive positions
   uint32_t cap_wg;       // candidates one workgroup may publish per round
   uint32_t target;       // candidates aimed at per round
+  // Picks s_begin .. s_end - 1 of fps.m.  s_begin > 0 continues a run whose min-distances
+  // fps.dmin holds by position, with every pick so far applied; s_end < fps.m saves them so.
+  uint32_t s_begin, s_end;
+  uint32_t *carry;       // four words kept from one part of such a run to the next
+  uint64_t start;        // pick 0 where fps.starts is null
+  // One cloud of several (fps_rounds_jobs): its workgroups, the first one's slot, and a
+  // counter of those that have claimed it, zeroed before the launch.
+  uint32_t team, member_base;
+  uint32_t *ready;
+};
+
+struct RoundsJobs {
+  const RoundsParams *table;
+  const uint32_t *member_job;  // slot -> entry of table
+  uint32_t members;
+  uint32_t *claim;             // zeroed before the launch
+  uint64_t team_ticks;         // bound on a team's forming
+  uint32_t one_slot;           // one workgroup per slot, all co-resident
 };
 
 constexpr int kRoundsThreads = 1024;
@@ -25,15 +43,18 @@ constexpr uint32_t kRoundsList = 512;      // candidates that may come in: the b
 constexpr uint32_t kRoundsMaxGrid = 256;
 constexpr uint32_t kRoundsHeadWords = 3;   // count, high and low half of the best key
 constexpr uint32_t kRoundsReplicas = 4;    // copies of the headers
+// Candidates a round aims at for m picks (fpsx_api.hip has the figures).
+inline uint32_t rounds_target(size_t m) {
+  return m >= 16384 ? 224 : m >= 1280 ? 160 : m <= 512 ? 64 : (uint32_t)(m / 8);
+}
 // Candidates one workgroup may publish: the area stays small enough to clear.
 inline uint32_t rounds_cap_wg(uint32_t grid) {
   return grid <= 8 ? kRoundsCap : grid <= 64 ? 64 : 32;
 }
 // Exchange words of a grid: two buffers of headers and candidates.
-inline size_t rounds_xchg_words(uint32_t grid, uint32_t dim) {
+inline size_t rounds_xchg_words(uint32_t grid, uint32_t dim, uint32_t cap_wg) {
   if (grid <= 1) return 1;
-  return (size_t)2 * ((size_t)kRoundsReplicas * kRoundsHeadWords * kRoundsMaxGrid +
-                      (size_t)(2 + dim) * grid * rounds_cap_wg(grid));
+  return (size_t)2 * grid * (kRoundsReplicas * kRoundsHeadWords + (2 + dim) * cap_wg);
 }
 // Dynamic LDS of a workgroup holding nbl blocks: box and best key of each.
 inline size_t rounds_shmem(uint32_t dim, uint32_t nbl) {
@@ -41,12 +62,17 @@ inline size_t rounds_shmem(uint32_t dim, uint32_t nbl) {
 }
 
 const KernelEntry *rounds_table(size_t *count);
+// The kernel for many clouds of a dimension (highest-index ties); null beyond four, where a
+// batch takes one launch per cloud.
+const KernelEntry *rounds_jobs_kernel(int dim);
 
 // Enqueues the spatial order of a cloud (fps_rounds_order.hip): rec holds n records, rest
 // (dim - 3) * n floats beyond three dimensions.  Returns a FPSX_* code.
 struct RoundsOrderScratch;
 RoundsOrderScratch *new_rounds_order_scratch();
 void delete_rounds_order_scratch(RoundsOrderScratch *s);
+// Sizes the scratch for clouds of up to n points, so that later calls allocate nothing.
+int rounds_order_reserve(RoundsOrderScratch &scratch, uint32_t n);
 int rounds_order(const float *pts, uint64_t sp, uint64_t ld, uint32_t n, uint32_t dim, float4 *rec,
                  float *rest, RoundsOrderScratch &scratch, hipStream_t st);
 

@@ -339,6 +339,28 @@ __global__ void __launch_bounds__(kThreads)
                   std::string(#expr) + ": " + hipGetErrorString(_e));  \
   } while (0)
 
+namespace {
+
+// Buckets of about 2048 points, at most kMaxBuckets; count and scatter by at most 256
+// workgroups of 4096 points and more.
+int bucket_bits(uint32_t n) {
+  int bits = 5;
+  while (bits < 3 * kCoarse && (n >> (bits + 11)) != 0) ++bits;
+  return bits;
+}
+uint32_t count_groups(uint32_t n) { return std::min<uint32_t>(256, (n + 4095) / 4096); }
+
+}  // namespace
+
+int rounds_order_reserve(RoundsOrderScratch &S, uint32_t n) {
+  if (n <= kChunk) return FPSX_OK;
+  const size_t buckets = (size_t)1 << bucket_bits(n);
+  HIP_OR_FAIL(S.part.reserve(kBoxGroups * 6 * sizeof(float)));
+  HIP_OR_FAIL(S.hist.reserve(buckets * (count_groups(n) + 1) * sizeof(uint32_t)));
+  HIP_OR_FAIL(S.tmp.reserve((size_t)n * sizeof(float4)));
+  return FPSX_OK;
+}
+
 int rounds_order(const float *pts, uint64_t sp, uint64_t ld, uint32_t n, uint32_t dim, float4 *rec,
                  float *rest, RoundsOrderScratch &S, hipStream_t st) {
   const Cloud c = {pts, sp, ld, n, dim};
@@ -349,17 +371,13 @@ int rounds_order(const float *pts, uint64_t sp, uint64_t ld, uint32_t n, uint32_
     HIP_OR_FAIL(hipGetLastError());
     return FPSX_OK;
   }
-  // Buckets of about 2048 points, at most kMaxBuckets; count and scatter by at most 256
-  // workgroups of 4096 points and more.
-  int bits = 5;
-  while (bits < 3 * kCoarse && (n >> (bits + 11)) != 0) ++bits;
+  const int bits = bucket_bits(n);
   const uint32_t buckets = 1u << bits;
-  const uint32_t g = std::min<uint32_t>(256, (n + 4095) / 4096);
+  const uint32_t g = count_groups(n);
   const uint32_t per = (n + g - 1) / g;
   const uint32_t gb = std::min<uint32_t>(kBoxGroups, (n + 2047) / 2048);
-  HIP_OR_FAIL(S.part.reserve(kBoxGroups * 6 * sizeof(float)));
-  HIP_OR_FAIL(S.hist.reserve(((size_t)buckets * g + buckets) * sizeof(uint32_t)));
-  HIP_OR_FAIL(S.tmp.reserve((size_t)n * sizeof(float4)));
+  const int rc = rounds_order_reserve(S, n);
+  if (rc) return rc;
   float *part = (float *)S.part.p;
   uint32_t *hist = (uint32_t *)S.hist.p, *total = hist + (size_t)buckets * g;
   const int shift = 3 * kCoarse - bits;

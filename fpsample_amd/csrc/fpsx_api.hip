@@ -448,9 +448,7 @@ static int plan_rounds(Ctx &c, size_t n, size_t dim, int tie, size_t m, Plan &p)
   p.grid = (uint32_t)g;
   p.chunk = (uint32_t)(nbl * 64 * P);
   p.shmem = shmem;
-  p.target = target > 0 ? std::min<uint32_t>((uint32_t)target, kRoundsCap)
-             : m >= 16384 ? 224
-                          : (uint32_t)std::min<size_t>(160, std::max<size_t>(64, m / 8));
+  p.target = target > 0 ? std::min<uint32_t>((uint32_t)target, kRoundsCap) : rounds_target(m);
   p.order = order >= 0 ? order != 0
                        : m >= 512 && (double)n * (double)m >= (n <= 8192 ? 1.5e5 : 6e5) * (double)g;
   return FPSX_OK;
@@ -775,7 +773,7 @@ int launch_fps(Ctx &c, const Plan &p, const float *d_pts, size_t sp, size_t ld, 
   FpsParams a;
   rc = common_params(c, d_pts, sp, ld, n, dim, m, d_starts, n_starts, d_out, d_out_pts, init,
                      p.chunk, st, a,
-                     p.kind == PlanKind::Rounds ? rounds_xchg_words(p.grid, (uint32_t)dim) : 0);
+                     p.kind == PlanKind::Rounds ? rounds_xchg_words(p.grid, (uint32_t)dim, rounds_cap_wg(p.grid)) : 0);
   if (rc) return rc;
   RoundsParams ra;
   if (p.kind == PlanKind::Rounds) {
@@ -788,6 +786,13 @@ int launch_fps(Ctx &c, const Plan &p, const float *d_pts, size_t sp, size_t ld, 
     ra.nblocks = (uint32_t)((n + block - 1) / block);
     ra.cap_wg = rounds_cap_wg(p.grid);
     ra.target = p.target;
+    ra.s_begin = 0;
+    ra.s_end = (uint32_t)m;
+    ra.start = 0;
+    ra.carry = nullptr;
+    ra.team = p.grid;
+    ra.member_base = 0;
+    ra.ready = nullptr;
     if (p.order) {
       HIP_TRY(c.rec.reserve(n * sizeof(float4)));
       if (dim > 3) HIP_TRY(c.rest.reserve(n * (dim - 3) * sizeof(float)));

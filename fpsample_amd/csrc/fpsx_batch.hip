@@ -156,6 +156,160 @@ int BatchRun::enqueue(hipStream_t st) {
   return FPSX_OK;
 }
 
+// Estimated us of one cloud on `team` workgroups: a round costs its front, an exchange beyond
+// one workgroup, and 3.6 us for each block of 256 points that a wave updates.  Fitted to us a
+// round measured at 1, 2, 4, 8, 16 and 32 workgroups: 65536 points 67, 41, 26, 19, 12 and 11;
+// 131072 points 114, 67, 39, 25, 17 and 12; 16384 points 21, 20, 13, 11, 10 and 10.
+static double rounds_us(const JobSpec &s, uint32_t target, uint32_t team) {
+  const double picks = (double)(s.s_end - s.s_begin);
+  const double rounds = 10.0 + picks / (0.55 * target);
+  const double share = (double)s.n / (64.0 * 4.0 * 16.0 * team);  // blocks per wave
+  return rounds * (7.0 + (team > 1 ? 3.0 : 0.0) + 3.6 * (share > 0.25 ? share : 0.25));
+}
+
+// The smallest team (a power of two times `least`, at most `most`) that ends within x us.
+static uint32_t rounds_team(const JobSpec &s, uint32_t target, uint32_t least, uint32_t most,
+                            double x) {
+  uint32_t best = least;
+  double us = rounds_us(s, target, least);
+  for (uint32_t t = least * 2; us > x && t <= most; t *= 2) {
+    const double u = rounds_us(s, target, t);
+    if (u < us) {
+      us = u;
+      best = t;
+    }
+  }
+  return best;
+}
+
+int RoundsRun::prepare(Ctx &c, int dim, const std::vector<JobSpec> &specs, const RoundsBases &b,
+                       const std::vector<uint32_t> *base_team) {
+  const bool one_slot = base_team != nullptr;
+  k = rounds_jobs_kernel(dim);
+  if (!k) return fail(FPSX_EINVAL, "no threshold-round kernel for this dimension");
+  const uint32_t P = (uint32_t)k->ppt;
+  const size_t n = specs.size();
+  const uint32_t gmax = (uint32_t)c.max_blocks(k, 0);
+  std::vector<uint32_t> team(n, 1), target(n), blocks(n);
+  std::vector<size_t> order(n);
+  std::iota(order.begin(), order.end(), 0);
+  for (size_t i = 0; i < n; ++i) {
+    const JobSpec &s = specs[i];
+    target[i] = rounds_target(s.m);
+    blocks[i] = (s.n + 64 * P - 1) / (64 * P);
+    // At most 1024 blocks a workgroup (LDS).
+    team[i] = std::max((blocks[i] + 1023) / 1024, one_slot ? (*base_team)[i] : 1u);
+    team[i] = std::min(team[i], blocks[i]);
+  }
+  // Team sizes for the least time x in which all can end: every cloud gets the smallest team
+  // that ends within x; teams hold their workgroups at once, and the clouds of one workgroup
+  // share the rest (one-slot launches: every cloud holds its own).
+  const std::vector<uint32_t> least = team;
+  auto fits = [&](double x, std::vector<uint32_t> &t) {
+    uint64_t held = 0;
+    double shared = 0.0;
+    for (size_t i = 0; i < n; ++i) {
+      t[i] = rounds_team(specs[i], target[i], least[i], std::min(blocks[i], kMaxTeam), x);
+      if (t[i] > 1 || one_slot)
+        held += t[i];
+      else
+        shared += rounds_us(specs[i], target[i], 1) / x;
+    }
+    return held + (uint64_t)std::ceil(shared) <= gmax;
+  };
+  double lo = 0.0, hi = 1.0;
+  for (size_t i = 0; i < n; ++i) hi = std::max(hi, rounds_us(specs[i], target[i], least[i]));
+  std::vector<uint32_t> t(n);
+  for (int it = 0; it < 24; ++it) {
+    const double x = 0.5 * (lo + hi);
+    if (fits(x, t)) {
+      hi = x;
+      team = t;
+    } else {
+      lo = x;
+    }
+  }
+  uint64_t total = 0;
+  for (size_t i = 0; i < n; ++i) total += team[i];
+  // Teams first (they form at once while the grid is free), longest first.
+  std::stable_sort(order.begin(), order.end(), [&](size_t x, size_t y) {
+    const bool tx = team[x] > 1, ty = team[y] > 1;
+    if (tx != ty) return tx;
+    return rounds_us(specs[x], target[x], team[x]) > rounds_us(specs[y], target[y], team[y]);
+  });
+  members = (uint32_t)total;
+  if (one_slot && members > gmax)
+    return fail(FPSX_ETOOBIG, "one-slot launch: more members than co-resident workgroups");
+  grid = std::min(members, gmax);
+  // One buffer to clear: status and claim, the teams' counters, their exchange areas.
+  size_t words = 2 + (n + 1) / 2;
+  std::vector<size_t> area(n, 0);
+  uint32_t nbl = 1;
+  for (size_t i = 0; i < n; ++i) {
+    nbl = std::max(nbl, (blocks[i] + team[i] - 1) / team[i]);
+    if (team[i] > grid) return fail(FPSX_ETOOBIG, "a team is larger than the co-resident grid");
+    if (team[i] == 1) continue;
+    area[i] = words;
+    words += rounds_xchg_words(team[i], (uint32_t)dim, rounds_cap_wg(team[i]));
+  }
+  clear_words = words;
+  shmem = rounds_shmem((uint32_t)dim, nbl);
+  if (c.max_blocks(k, shmem) < (int)gmax) return fail(FPSX_ETOOBIG, "threshold rounds: LDS");
+  HIP_TRY(d_clear.reserve(words * sizeof(uint64_t)));
+  host.assign(n * sizeof(RoundsParams) + members * sizeof(uint32_t), 0);
+  HIP_TRY(d_tables.reserve(host.size()));
+  RoundsParams *tab = (RoundsParams *)host.data();
+  uint32_t *slot = (uint32_t *)(tab + n);
+  uint64_t *cl = (uint64_t *)d_clear.p;
+  uint32_t at = 0;
+  for (size_t o = 0; o < n; ++o) {
+    const size_t i = order[o];
+    const JobSpec &s = specs[i];
+    RoundsParams &r = tab[o];
+    r.fps.pts = b.pts + s.pt_off;
+    r.fps.ld = s.ld;
+    r.fps.sp = 1;
+    r.fps.n = s.n;
+    r.fps.m = s.m;
+    r.fps.n_starts = 1;
+    r.fps.dim = (uint32_t)dim;
+    r.fps.out = b.out + s.out_off;
+    r.fps.xchg = cl + area[i];
+    r.fps.status = (uint32_t *)d_clear.p;
+    r.fps.dmin = b.state + s.state_off;
+    r.fps.init = INFINITY;
+    r.fps.spin_ticks = c.spin_ticks;
+    r.rec = (const float4 *)(b.sorted + s.sorted_off);
+    r.rest = b.rest ? b.rest + s.perm_off : nullptr;
+    r.nblocks = blocks[i];
+    r.cap_wg = rounds_cap_wg(team[i]);
+    r.target = target[i];
+    r.s_begin = s.s_begin;
+    r.s_end = s.s_end;
+    r.carry = (uint32_t *)(r.fps.dmin + s.n);
+    r.start = s.start;
+    r.team = team[i];
+    r.member_base = at;
+    r.ready = (uint32_t *)(cl + 2) + o;
+    for (uint32_t q = 0; q < team[i]; ++q) slot[at++] = (uint32_t)o;
+  }
+  HIP_TRY(hipMemcpy(d_tables.p, host.data(), host.size(), hipMemcpyHostToDevice));
+  jobs.table = (const RoundsParams *)d_tables.p;
+  jobs.member_job = (const uint32_t *)(jobs.table + n);
+  jobs.members = members;
+  jobs.claim = (uint32_t *)(cl + 1);
+  jobs.team_ticks = c.spin_ticks * 5;
+  jobs.one_slot = one_slot ? 1u : 0u;
+  return FPSX_OK;
+}
+
+int RoundsRun::enqueue(hipStream_t st) {
+  HIP_TRY(launch_fill_u64((uint64_t *)d_clear.p, clear_words, 0, st));
+  void *args[] = {(void *)&jobs};
+  HIP_TRY(hipLaunchKernel(k->fn, dim3(grid), dim3(k->block), args, shmem, st));
+  return FPSX_OK;
+}
+
 }  // namespace fpsx
 
 using namespace fpsx;
@@ -175,6 +329,12 @@ struct fpsx_batch {
   SpatialScratch *spatial = nullptr;
   uint32_t order_block = 0;
   std::vector<uint64_t> offsets;
+  // Threshold rounds: records of cloud c at rec + 4 * offsets[c], coordinates beyond three
+  // at rest, min-distances of clouds too large for registers in state.
+  RoundsRun rounds;
+  bool use_rounds = false;
+  DevBuf rec, rest, state;
+  RoundsOrderScratch *rorder = nullptr;
   bool fallback = false;  // no batch kernel for this dimension or cloud size: one launch per cloud
   std::vector<JobSpec> specs;
   const float *d_pts = nullptr;
@@ -239,6 +399,45 @@ static int batch_order(fpsx_batch *b, uint32_t block) {
   return FPSX_OK;
 }
 
+// The threshold rounds for this batch: order every cloud, build the tables.  ETOOBIG where
+// some cloud is beyond a team of the pass kernels too.  Caller holds the context lock.
+static int batch_prepare_rounds(fpsx_batch *b) {
+  Ctx &c = *b->ctx;
+  const uint64_t total = b->offsets.back();
+  const uint64_t more = b->dim > 3 ? (uint64_t)b->dim - 3 : 0;
+  uint32_t nmax = 0;
+  for (auto &s : b->specs) nmax = std::max(nmax, s.n);
+  if (nmax > kMaxTeam * 16384u) return fail(FPSX_ETOOBIG, "a cloud exceeds a team's capacity");
+  HIP_TRY(b->rec.reserve(total * sizeof(float4)));
+  if (more) HIP_TRY(b->rest.reserve(total * more * sizeof(float)));
+  // (n + 4 floats a cloud, 16-byte aligned)
+  std::vector<uint64_t> state(b->n_clouds);
+  uint64_t at = 0;
+  for (size_t i = 0; i < b->n_clouds; ++i) {
+    state[i] = at;
+    at += ((uint64_t)b->specs[i].n + 7) / 4 * 4;
+  }
+  HIP_TRY(b->state.reserve(at * sizeof(float)));
+  if (!b->rorder) b->rorder = new_rounds_order_scratch();
+  int rc = rounds_order_reserve(*b->rorder, nmax);
+  if (rc) return rc;
+  std::vector<JobSpec> specs = b->specs;
+  for (size_t i = 0; i < b->n_clouds; ++i) {
+    JobSpec &s = specs[i];
+    s.sorted_off = 4 * b->offsets[i];
+    s.perm_off = more * b->offsets[i];
+    s.state_off = state[i];
+    rc = rounds_order(b->d_pts + s.pt_off, 1, b->ld, s.n, (uint32_t)b->dim,
+                      (float4 *)b->rec.p + b->offsets[i],
+                      more ? (float *)b->rest.p + s.perm_off : nullptr, *b->rorder, c.stream);
+    if (rc) return rc;
+  }
+  HIP_TRY(hipStreamSynchronize(c.stream));
+  const RoundsBases bases = {b->d_pts, b->d_out, (float *)b->state.p, (const float *)b->rec.p,
+                             (const float *)b->rest.p};
+  return b->rounds.prepare(c, b->dim, specs, bases);
+}
+
 static int batch_prepare_kernel(fpsx_batch *b, const KernelEntry *k, bool pruned) {
   std::vector<BatchJob> jobs;
   std::vector<uint32_t> mj;
@@ -292,6 +491,31 @@ FPSX_EXPORT int fpsx_batch_create(const float *d_points, size_t ld, size_t dim,
   };
   std::vector<Cand> cands;
   const char *plain = std::getenv("FPSX_BATCH_PLAIN");
+  // Threshold rounds unless a pass kernel is asked for by name; the tuner times them too.
+  bool rounds = rounds_jobs_kernel((int)dim) != nullptr;
+  for (const char *name : {"FPSX_BATCH_SHAPE", "FPSX_BATCH_PLAIN", "FPSX_BATCH_NO_PAIR", "FPSX_NO_ROUNDS"}) {
+    const char *v = std::getenv(name);
+    if (v && *v && std::strcmp(v, "0") != 0) rounds = false;
+  }
+  float rounds_ms = 0.0f;
+  if (rounds) {
+    rc = batch_prepare_rounds(b.get());
+    if (rc != FPSX_OK && rc != FPSX_ETOOBIG) return rc;
+    rounds = rc == FPSX_OK;
+  }
+  if (rounds && (flags & FPSX_BATCH_AUTOTUNE)) {
+    hipEvent_t e0, e1;
+    HIP_TRY(hipEventCreate(&e0));
+    HIP_TRY(hipEventCreate(&e1));
+    HIP_TRY(hipEventRecord(e0, c.stream));
+    rc = b->rounds.enqueue(c.stream);
+    if (rc) return rc;
+    HIP_TRY(hipEventRecord(e1, c.stream));
+    HIP_TRY(hipEventSynchronize(e1));
+    HIP_TRY(hipEventElapsedTime(&rounds_ms, e0, e1));
+    (void)hipEventDestroy(e0);  // timing events only
+    (void)hipEventDestroy(e1);
+  }
   if (dim == 3 && !(plain && plain[0] == '1')) {
     for (int ppt : {8, 16, 4}) {
       const KernelEntry *k = batch_pp_kernel(1024, ppt, false);
@@ -302,7 +526,7 @@ FPSX_EXPORT int fpsx_batch_create(const float *d_points, size_t ld, size_t dim,
   const KernelEntry *t = batch_table(&cnt);
   for (size_t i = 0; i < cnt; ++i)
     if (t[i].dim == (int)dim) cands.push_back({&t[i], false});
-  if (cands.empty()) {
+  if (cands.empty() && !rounds) {
     b->fallback = true;
     *out = b.release();
     return FPSX_OK;
@@ -323,7 +547,7 @@ FPSX_EXPORT int fpsx_batch_create(const float *d_points, size_t ld, size_t dim,
     hipEvent_t e0, e1;
     HIP_TRY(hipEventCreate(&e0));
     HIP_TRY(hipEventCreate(&e1));
-    float best = 1e30f;
+    float best = rounds ? rounds_ms : 1e30f;
     for (const Cand &cd : cands) {
       const KernelEntry *k = cd.k;
       if (batch_prepare_kernel(b.get(), k, cd.pruned) != FPSX_OK) continue;
@@ -343,7 +567,8 @@ FPSX_EXPORT int fpsx_batch_create(const float *d_points, size_t ld, size_t dim,
     (void)hipEventDestroy(e0);  // timing events only
     (void)hipEventDestroy(e1);
   }
-  if (!chosen) {
+  b->use_rounds = rounds && !chosen;
+  if (!chosen && !b->use_rounds) {
     // Heuristic: the first pruned kernel whose teams hold every cloud; else
     // the smallest plain per-workgroup capacity that still fits every cloud
     // in a team the grid can hold (short reduction chains for small clouds),
@@ -373,7 +598,7 @@ FPSX_EXPORT int fpsx_batch_create(const float *d_points, size_t ld, size_t dim,
       chosen_pruned = cands.back().pruned;
     }
   }
-  rc = batch_prepare_kernel(b.get(), chosen, chosen_pruned);
+  rc = b->use_rounds ? FPSX_OK : batch_prepare_kernel(b.get(), chosen, chosen_pruned);
   if (rc == FPSX_ETOOBIG) {
     // Some cloud needs more workgroups than a team may have: every cloud
     // gets a planned launch of its own (the single-cloud kernels have no
@@ -386,7 +611,7 @@ FPSX_EXPORT int fpsx_batch_create(const float *d_points, size_t ld, size_t dim,
   if (flags & FPSX_BATCH_GRAPH) {
     HIP_TRY(hipStreamCreateWithFlags(&b->capture_stream, hipStreamNonBlocking));
     HIP_TRY(hipStreamBeginCapture(b->capture_stream, hipStreamCaptureModeThreadLocal));
-    rc = b->run.enqueue(b->capture_stream);
+    rc = b->use_rounds ? b->rounds.enqueue(b->capture_stream) : b->run.enqueue(b->capture_stream);
     hipGraph_t g = nullptr;
     hipError_t e = hipStreamEndCapture(b->capture_stream, &g);
     if (rc) return rc;
@@ -420,7 +645,7 @@ FPSX_EXPORT int fpsx_batch_run(fpsx_batch *b, void *stream) {
     for (size_t i = 0; i < b->specs.size(); ++i) {
       const JobSpec &s = b->specs[i];
       Plan p;
-      rc = plan(c, s.n, b->dim, kTieHighest, s.m, p);
+      rc = plan_call(c, s.n, b->dim, kTieHighest, s.m, p);
       if (rc) return rc;
       rc = launch_fps(c, p, b->d_pts + s.pt_off, 1, b->ld, s.n, b->dim, s.m,
                       (const uint64_t *)c.starts.p + i, 1, b->d_out + s.out_off, nullptr,
@@ -434,7 +659,7 @@ FPSX_EXPORT int fpsx_batch_run(fpsx_batch *b, void *stream) {
     HIP_TRY(hipGraphLaunch(b->exec, st));
     return FPSX_OK;
   }
-  return b->run.enqueue(st);
+  return b->use_rounds ? b->rounds.enqueue(st) : b->run.enqueue(st);
 }
 
 FPSX_EXPORT int fpsx_batch_status(fpsx_batch *b, void *stream) {
@@ -443,18 +668,20 @@ FPSX_EXPORT int fpsx_batch_status(fpsx_batch *b, void *stream) {
   std::lock_guard<std::mutex> lk(c.mu);
   hipStream_t st = stream ? (hipStream_t)stream : c.stream;
   HIP_TRY(hipStreamSynchronize(st));
-  if (!b->run.d_status.p) return FPSX_OK;  // never run
-  HIP_TRY(hipMemcpy(c.host_status, b->run.d_status.p, sizeof(uint32_t), hipMemcpyDeviceToHost));
+  const void *word = b->use_rounds ? b->rounds.d_clear.p : b->run.d_status.p;
+  if (!word) return FPSX_OK;  // never run
+  HIP_TRY(hipMemcpy(c.host_status, word, sizeof(uint32_t), hipMemcpyDeviceToHost));
   return status_code(*c.host_status);
 }
 
 FPSX_EXPORT int fpsx_batch_info(fpsx_batch *b, int *block, int *ppt, int *grid, int *members,
                                 int *graph) {
   if (!b) return fail(FPSX_EINVAL, "null batch");
-  if (block) *block = b->fallback ? 0 : b->run.k->block;
-  if (ppt) *ppt = b->fallback ? 0 : b->run.k->ppt;
-  if (grid) *grid = b->fallback ? 0 : (int)b->run.grid;
-  if (members) *members = b->fallback ? 0 : (int)b->run.members;
+  const KernelEntry *k = b->fallback ? nullptr : b->use_rounds ? b->rounds.k : b->run.k;
+  if (block) *block = k ? k->block : 0;
+  if (ppt) *ppt = k ? k->ppt : 0;
+  if (grid) *grid = !k ? 0 : (int)(b->use_rounds ? b->rounds.grid : b->run.grid);
+  if (members) *members = !k ? 0 : (int)(b->use_rounds ? b->rounds.members : b->run.members);
   if (graph) *graph = b->exec != nullptr;
   return FPSX_OK;
 }
@@ -467,6 +694,10 @@ FPSX_EXPORT void fpsx_batch_destroy(fpsx_batch *b) {
   if (b->capture_stream) (void)hipStreamDestroy(b->capture_stream);
   b->sorted.free();
   b->perm.free();
+  b->rec.free();
+  b->rest.free();
+  b->state.free();
+  delete_rounds_order_scratch(b->rorder);
   delete_spatial_scratch(b->spatial);
   delete b;
 }

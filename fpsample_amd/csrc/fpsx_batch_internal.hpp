@@ -6,6 +6,7 @@
 #include <vector>
 
 #include "fps_batch.hpp"
+#include "fps_rounds.hpp"
 #include "fpsx_internal.hpp"
 
 namespace fpsx {
@@ -54,6 +55,37 @@ struct BatchRun {
     d_counters.free();
     d_xchg.free();
     d_status.free();
+  }
+};
+
+// Where the threshold rounds find a batch's data; a job's offsets (JobSpec) count from these
+// bases, sorted_off in floats to the cloud's records and state_off in floats to its
+// min-distances by position and four words carried between parts of a run.
+struct RoundsBases {
+  const float *pts;     // SoA points
+  uint64_t *out;
+  float *state;
+  const float *sorted;  // records {x, y, z, original index}
+  const float *rest;    // beyond three dimensions: the further coordinates, at JobSpec::perm_off
+};
+
+// The same for the threshold rounds (fps_rounds_jobs).
+struct RoundsRun {
+  const KernelEntry *k = nullptr;
+  uint32_t members = 0, grid = 0;
+  size_t shmem = 0, clear_words = 0;
+  DevBuf d_tables, d_clear;  // job table and slots; status, claim and team counters, exchange
+  RoundsJobs jobs;
+  std::vector<char> host;    // what d_tables holds
+  uint32_t *status() const { return (uint32_t *)d_clear.p; }
+  // Upload tables for these clouds (host-synchronous).  one_slot: every member has a
+  // workgroup of its own, all co-resident, and base_team[i] is the least team of cloud i.
+  int prepare(Ctx &c, int dim, const std::vector<JobSpec> &specs, const RoundsBases &b,
+              const std::vector<uint32_t> *base_team = nullptr);
+  int enqueue(hipStream_t st);  // graph-capturable
+  ~RoundsRun() {
+    d_tables.free();
+    d_clear.free();
   }
 };
 

@@ -1,5 +1,5 @@
 // fpsx_server.cpp -- FPS serving loop with HBM-budget admission and
-// continuous batching (host runtime, HIP API only; the kernel is fps_batch).
+// continuous batching (host runtime, HIP API only; the kernel is fps_rounds_jobs).
 //
 // Requests (one cloud each, any size) are submitted from any thread.  A
 // scheduler thread owns the device:
@@ -144,9 +144,12 @@ using namespace fpsx;
 struct fpsx_server {
   Ctx *ctx = nullptr;
   const KernelEntry *k = nullptr;
-  // The pruned paired kernel (fps_batch_pp, one slot per member): every
-  // request is put in spatial order on the copy stream after its upload.
-  // FPSX_SERVE_PLAIN=1 at creation keeps the plain batch kernel.
+  // The threshold rounds (fps_rounds_jobs, one slot per member) unless a shape is asked for;
+  // else the pruned paired kernel (fps_batch_pp, the same): every request is put in spatial
+  // order on the copy stream after its upload.  FPSX_SERVE_PLAIN=1 at creation keeps the plain
+  // batch kernel, FPSX_NO_ROUNDS=1 the pruned one.
+  bool rounds = true;
+  RoundsOrderScratch *rorder = nullptr;
   bool pruned = true;
   SpatialScratch *spatial = nullptr;
   uint32_t chunk = 256;
@@ -159,6 +162,7 @@ struct fpsx_server {
   // one, prepared and queued behind it.
   struct Launch {
     BatchRun run;
+    RoundsRun rounds;
     hipEvent_t t0 = nullptr, t1 = nullptr;  // around the kernel, for busy_s
     std::vector<std::shared_ptr<Request>> reqs;
     std::vector<uint32_t> s_end;
@@ -184,12 +188,12 @@ struct fpsx_server {
   std::string fatal_msg;
 
   uint32_t team_of(uint32_t n) const {
-    const uint32_t cap = (uint32_t)(k->block * k->ppt);
+    const uint32_t cap = rounds ? 16384u : (uint32_t)(k->block * k->ppt);
     const uint32_t t = (n + cap - 1) / cap;
     return std::max(1u, t);
   }
-  // Points, min-distances (+ the last pick's coordinates), picks; for the
-  // pruned kernel also the spatially ordered points and their original indices.
+  // Points, min-distances (and four words carried between launches), picks; but for the
+  // plain kernel also the spatially ordered points and their original indices.
   size_t footprint(const Request &r) const {
     size_t b = align_up((size_t)r.n * r.dim * sizeof(float)) +
                align_up(((size_t)r.n + 4) * sizeof(float)) + align_up((size_t)r.m * sizeof(uint64_t));
@@ -305,7 +309,12 @@ int fpsx_server::step() {
     }
     hipError_t e = hipMemcpyAsync(base + r->pts_off, r->soa.data(), r->soa.size() * sizeof(float),
                                   hipMemcpyHostToDevice, copy);
-    if (e == hipSuccess && pruned) {
+    if (e == hipSuccess && rounds) {
+      // (sorted_off and perm_off together hold the 16-byte records)
+      const int rc = rounds_order((const float *)(base + r->pts_off), 1, r->n, r->n, r->dim,
+                                  (float4 *)(base + r->sorted_off), nullptr, *rorder, copy);
+      if (rc) return rc;
+    } else if (e == hipSuccess && pruned) {
       const int rc = spatial_order((const float *)(base + r->pts_off), 1, r->n, r->n,
                                    (uint32_t)(64 * k->ppt), (float *)(base + r->sorted_off),
                                    (uint32_t *)(base + r->perm_off), *spatial, copy);
@@ -320,6 +329,7 @@ int fpsx_server::step() {
   // are paused for this launch), each from where the queued launches leave it.
   std::vector<std::shared_ptr<Request>> in_launch, leaving;
   std::vector<JobSpec> specs;
+  std::vector<uint32_t> teams;
   bool waiting_upload = false;
   {
     std::lock_guard<std::mutex> lk(mu);
@@ -384,6 +394,7 @@ int fpsx_server::step() {
       if (s.s_end >= r->m) r->finishing = true;
       ++r->inflight;
       specs.push_back(s);
+      teams.push_back(r->team);
       in_launch.push_back(r);
     }
   }
@@ -429,21 +440,25 @@ int fpsx_server::step() {
   std::vector<BatchJob> jobs;
   std::vector<uint32_t> mj;
   uint32_t areas = 0;
-  int rc = build_jobs(specs.data(), specs.size(), k, 0, jobs, mj, &areas, pruned);
+  int rc = rounds ? FPSX_OK
+                  : build_jobs(specs.data(), specs.size(), k, 0, jobs, mj, &areas, pruned);
   if (rc) return rc;
   // pt/out/state/sorted/perm offsets are element offsets from the arena base for every view
   {
     std::lock_guard<std::mutex> lk(ctx->mu);
-    rc = pruned ? L.run.prepare(*ctx, k, jobs, mj, areas, (const float *)arena_base,
+    const RoundsBases bases = {(const float *)arena_base, (uint64_t *)arena_base,
+                               (float *)arena_base, (const float *)arena_base, nullptr};
+    rc = rounds   ? L.rounds.prepare(*ctx, 3, specs, bases, &teams)
+         : pruned ? L.run.prepare(*ctx, k, jobs, mj, areas, (const float *)arena_base,
                                 (uint64_t *)arena_base, (float *)arena_base,
                                 (const float *)arena_base, (const uint32_t *)arena_base, true)
-                : L.run.prepare(*ctx, k, jobs, mj, areas, (const float *)arena_base,
-                                (uint64_t *)arena_base, (float *)arena_base);
+                  : L.run.prepare(*ctx, k, jobs, mj, areas, (const float *)arena_base,
+                                  (uint64_t *)arena_base, (float *)arena_base);
   }
   if (rc) return rc;
   hipError_t e = hipEventRecord(L.t0, compute);
   if (e != hipSuccess) return fail(FPSX_EHIP, std::string("serve launch: ") + hipGetErrorString(e));
-  rc = L.run.enqueue(compute);
+  rc = rounds ? L.rounds.enqueue(compute) : L.run.enqueue(compute);
   if (rc) return rc;
   e = hipEventRecord(L.t1, compute);
   if (e != hipSuccess) return fail(FPSX_EHIP, std::string("serve launch: ") + hipGetErrorString(e));
@@ -464,7 +479,8 @@ int fpsx_server::finish(Launch &L) {
   L.busy = false;
   cur ^= 1;  // the other slot (if queued) is now the oldest
   uint32_t st = 0;
-  e = hipMemcpy(&st, L.run.d_status.p, sizeof(uint32_t), hipMemcpyDeviceToHost);
+  e = hipMemcpy(&st, rounds ? L.rounds.status() : (uint32_t *)L.run.d_status.p, sizeof(uint32_t),
+                hipMemcpyDeviceToHost);
   if (e != hipSuccess) return fail(FPSX_EHIP, std::string("status: ") + hipGetErrorString(e));
   if (st) return status_code(st);
   ++launches;
@@ -548,7 +564,10 @@ FPSX_EXPORT int fpsx_server_create(size_t hbm_budget_bytes, unsigned chunk_passe
   const int B = block ? block : 1024, P = ppt ? ppt : 16;
   const char *plain = std::getenv("FPSX_SERVE_PLAIN");
   s->pruned = !(plain && plain[0] == '1');
-  if (s->pruned) {
+  const char *no_rounds = std::getenv("FPSX_NO_ROUNDS");
+  s->rounds = s->pruned && !block && !ppt && !(no_rounds && no_rounds[0] == '1');
+  if (s->rounds) s->k = rounds_jobs_kernel(3);
+  if (s->pruned && !s->rounds) {
     s->k = batch_pp_kernel(B, P, true);
     if (!s->k) s->pruned = false;  // no pruned kernel of that shape: the plain one
   }
@@ -569,7 +588,15 @@ FPSX_EXPORT int fpsx_server_create(size_t hbm_budget_bytes, unsigned chunk_passe
   hipError_t e = hipMalloc(&s->arena_base, s->budget);
   if (e != hipSuccess) return fail(FPSX_ENOMEM, "arena: " + std::string(hipGetErrorString(e)));
   s->arena.reset(new Arena(s->budget));
-  if (s->pruned) {
+  if (s->rounds) {
+    s->rorder = new_rounds_order_scratch();
+    rc = rounds_order_reserve(*s->rorder, std::min<uint32_t>(s->grid_cap, kMaxTeam) * 16384u);
+    if (rc) {
+      delete_rounds_order_scratch(s->rorder);
+      (void)hipFree(s->arena_base);
+      return rc;
+    }
+  } else if (s->pruned) {
     // Scratch of the spatial order sized once for the largest request a team
     // can hold, so admissions allocate nothing.
     s->spatial = new_spatial_scratch();
@@ -587,6 +614,7 @@ FPSX_EXPORT int fpsx_server_create(size_t hbm_budget_bytes, unsigned chunk_passe
     const std::string msg = "streams: " + std::string(hipGetErrorString(e));
     if (s->compute) (void)hipStreamDestroy(s->compute);
     delete_spatial_scratch(s->spatial);
+    delete_rounds_order_scratch(s->rorder);
     (void)hipFree(s->arena_base);
     return fail(FPSX_EHIP, msg);
   }
@@ -599,6 +627,7 @@ FPSX_EXPORT int fpsx_server_create(size_t hbm_budget_bytes, unsigned chunk_passe
     (void)hipStreamDestroy(s->compute);
     (void)hipStreamDestroy(s->copy);
     delete_spatial_scratch(s->spatial);
+    delete_rounds_order_scratch(s->rorder);
     (void)hipFree(s->arena_base);
     return fail(FPSX_EHIP, msg);
   }
@@ -771,6 +800,7 @@ FPSX_EXPORT void fpsx_server_destroy(fpsx_server *s) {
   }
   if (s->arena_base) (void)hipFree(s->arena_base);
   delete_spatial_scratch(s->spatial);
+  delete_rounds_order_scratch(s->rorder);
   (void)hipStreamDestroy(s->compute);
   (void)hipStreamDestroy(s->copy);
   delete s;
