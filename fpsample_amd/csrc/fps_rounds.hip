@@ -31,52 +31,13 @@
 
 #include "fps_device.hpp"
 #include "fps_kernels.hpp"
+#include "fps_rounds_device.hpp"
 
 namespace fpsx {
 
-namespace {
-
-__device__ __forceinline__ uint64_t make_key(int value_bits, uint32_t tie) {
-  return ((uint64_t)((uint32_t)value_bits + 1u) << 32) | tie;
-}
-template <int TIE>
-__device__ __forceinline__ uint32_t tie_of(uint32_t idx) {
-  return TIE == kTieHighest ? idx : ~idx;
-}
-
-// Wave-wide maximum of a 64-bit key (uniform).
-__device__ __forceinline__ uint64_t wave_max_u64(uint64_t k) {
-  const uint32_t hi = wave_max_u32((uint32_t)(k >> 32));
-  const uint32_t lo = wave_max_u32((uint32_t)(k >> 32) == hi ? (uint32_t)k : 0u);
-  return ((uint64_t)hi << 32) | lo;
-}
-
-__device__ __forceinline__ uint32_t lanes_below(uint64_t mask) {
-  return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32),
-                                   __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
-}
-
-__device__ __forceinline__ uint64_t readlane_u64(uint64_t v, int lane) {
-  return ((uint64_t)(uint32_t)readlane_i((int)(v >> 32), lane) << 32) |
-         (uint32_t)readlane_i((int)(uint32_t)v, lane);
-}
-
-__device__ __forceinline__ uint64_t uniform_u64(uint64_t v) {
-  return ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32) |
-         (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v);
-}
-
-}  // namespace
-
-// One record of a candidate's coordinates in LDS, read 16 bytes at a time.
-template <int D>
-struct alignas(16) Rec {
-  float c[(D + 3) / 4 * 4];
-};
-
 // LDS of a workgroup beside its blocks' boxes and best keys.
 template <int D>
-struct RoundsLds {
+struct RoundsLds : RoundsCounts {
   static constexpr int CAP = (int)kRoundsCap;    // candidates the front decides on
   static constexpr int LIST = (int)kRoundsList;  // candidates that may come in
   static constexpr int W = kRoundsThreads / 64;
@@ -90,32 +51,21 @@ struct RoundsLds {
   uint16_t low[CAP / 32][CAP][2];  // rows: which earlier candidates lower this one
   uint64_t lk[CAP];                // this workgroup's candidates
   Rec<D> lc[CAP];
-  uint32_t cnt[2];  // candidates of this workgroup, by round parity
-  uint32_t sum[2];  // candidates of the grid, by round parity
-  uint32_t at[2];   // candidates taken in, by round parity
-  uint64_t wmax[W];
   uint64_t acc[CAP / 64];
-  uint64_t te;    // the bound that the round's picks exceed
-  uint32_t stop;  // first pick that does not lower itself
-  uint64_t last;  // key of the round's last pick
-  uint32_t np;
-  uint32_t stuck;
-  uint32_t ok;
 };
 
 // Workgroup `group` of G working on one cloud: picks a.s_begin .. a.s_end - 1.
 template <int D, int P, int TIE>
-__device__ __forceinline__ void rounds_cloud(const RoundsParams &a, const uint32_t group,
+__device__ __forceinline__ void rounds_cloud(ParamsPtr params, const uint32_t group,
                                              const uint32_t G, RoundsLds<D> &S, uint64_t *s_dyn) {
   constexpr int W = RoundsLds<D>::W;
   constexpr int CAP = RoundsLds<D>::CAP;
   constexpr int LIST = RoundsLds<D>::LIST;
   constexpr int CH = CAP / 64;
-  constexpr uint32_t NWC = 2 + D;
-  const FpsParams &f = a.fps;
   int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const uint32_t nbl = (a.nblocks - group + G - 1) / G;  // blocks group, group + G, ...
+  const uint32_t s_begin = params->s_begin;
+  const uint32_t nbl = (params->nblocks - group + G - 1) / G;  // blocks group, group + G, ...
   const bool resident = nbl <= (uint32_t)W;          // a block per wave stays in registers
   uint64_t *s_bkey = s_dyn;
   float *s_box = (float *)(s_dyn + nbl);  // [2 * D][nbl]
@@ -129,19 +79,19 @@ __device__ __forceinline__ void rounds_cloud(const RoundsParams &a, const uint32
     S.ok = 1;
   }
 
-  if (a.s_begin) lds_barrier();  // (a fresh run has one after its forced picks)
+  if (s_begin) lds_barrier();  // (a fresh run has one after its forced picks)
 
-  uint32_t s = a.s_begin;  // picks recorded
+  uint32_t s = s_begin;    // picks recorded
   uint32_t np = 0;         // picks of the last round, in S.pk
-  bool first = true;       // the blocks have not been read yet
-  bool last = false;       // the picks are made: apply them and save
+  uint32_t fresh = 1;      // the blocks have not been read yet
   uint64_t T = ~0ull;    // every point's key is at most T
   uint64_t Tg = ~0ull;   // the round's bound
   uint64_t step = (uint64_t)1 << 51;  // a sixteenth of a binade
-  if (a.s_begin) {
+  if (s_begin) {
     // A run taken up again: no key exceeds that of its last pick.
-    T = uniform_u64(((uint64_t)a.carry[0] << 32) | a.carry[1]);
-    step = uniform_u64(((uint64_t)a.carry[2] << 32) | a.carry[3]);
+    const uint32_t *carry = params->carry;
+    T = uniform_u64(((uint64_t)carry[0] << 32) | carry[1]);
+    step = uniform_u64(((uint64_t)carry[2] << 32) | carry[3]);
     Tg = T > step ? T - step : 0;
   }
   uint32_t e = 0;        // rounds
@@ -152,10 +102,23 @@ __device__ __forceinline__ void rounds_cloud(const RoundsParams &a, const uint32
   for (;;) {
     // Rewritten each round: addresses formed from them would otherwise be kept in registers
     // over the whole loop, beside the block.
-    asm volatile("" : "+v"(tid));
+    asm volatile("" : "+v"(tid), "+s"(params));
+    const __attribute__((address_space(4))) RoundsParams &a = *params;
+    const __attribute__((address_space(4))) FpsParams &f = a.fps;
     uint32_t g = (uint32_t)__builtin_amdgcn_readfirstlane((int)group);
     asm volatile("" : "+s"(g));
     const int lane = tid & 63;
+    // What the rounds carry is the same in every lane, which the compiler cannot see through
+    // the loop's several exits; in vector registers its branches would run under masks (the
+    // update loop a fifth slower).
+    s = uniform_u32(s);
+    np = uniform_u32(np);
+    e = uniform_u32(e);
+    idle = uniform_u32(idle);
+    T = uniform_u64(T);
+    Tg = uniform_u64(Tg);
+    step = uniform_u64(step);
+    const bool first = uniform_u32(fresh) != 0;
     // ---- forced picks, in pieces of CAP -------------------------------------
     if (s < f.n_starts) {
       np = min(f.n_starts - s, (uint32_t)CAP);
@@ -184,33 +147,27 @@ __device__ __forceinline__ void rounds_cloud(const RoundsParams &a, const uint32
     }
     s += np;
     if (s >= f.m) return;
-    if (s >= a.s_end) {
-      last = true;
-      if (g == 0 && tid == 0) {
-        a.carry[0] = (uint32_t)(S.last >> 32);
-        a.carry[1] = (uint32_t)S.last;
-        a.carry[2] = (uint32_t)(step >> 32);
-        a.carry[3] = (uint32_t)step;
-      }
-    } else if (np && __builtin_amdgcn_readfirstlane((int)S.stuck)) {
-      // The last pick left its own key unchanged, so it stays the best for good.
-      if (g == 0) {
-        const uint32_t t = S.pt[np - 1];
-        for (uint32_t q = s + tid; q < a.s_end; q += kRoundsThreads) {
-          f.out[q] = tie_of<TIE>(t);
-          if (f.out_pts != nullptr) {
+    const bool cut = s >= a.s_end;
+    // (a last pick that left its own key unchanged stays the best for good)
+    const bool stuck = uniform_u32(!cut && np && S.stuck) != 0;
+    if (stuck && g == 0) {
+      const uint32_t t = S.pt[np - 1];
+      for (uint32_t q = s + tid; q < a.s_end; q += kRoundsThreads) {
+        f.out[q] = tie_of<TIE>(t);
+        if (f.out_pts != nullptr) {
 #pragma unroll
-            for (int j = 0; j < D; ++j) f.out_pts[(size_t)q * D + j] = S.pk[np - 1].c[j];
-          }
+          for (int j = 0; j < D; ++j) f.out_pts[(size_t)q * D + j] = S.pk[np - 1].c[j];
         }
       }
-      if (a.s_end >= f.m) return;
-      last = true;  // (the picks so far are applied below; repeating the last changes nothing)
-      if (g == 0 && tid == 0) {
-        a.carry[0] = a.carry[1] = ~0u;
-        a.carry[2] = (uint32_t)(step >> 32);
-        a.carry[3] = (uint32_t)step;
-      }
+    }
+    if (stuck && a.s_end >= f.m) return;
+    // The picks of this part are made: apply them and save.
+    const bool last = cut || stuck;
+    if (last && g == 0 && tid == 0) {
+      a.carry[0] = cut ? (uint32_t)(S.last >> 32) : ~0u;
+      a.carry[1] = cut ? (uint32_t)S.last : ~0u;
+      a.carry[2] = (uint32_t)(step >> 32);
+      a.carry[3] = (uint32_t)step;
     }
     const bool gather = s >= f.n_starts && !last;  // no further forced picks
     if (!gather) Tg = ~0ull;
@@ -272,7 +229,7 @@ __device__ __forceinline__ void rounds_cloud(const RoundsParams &a, const uint32
               for (int j = 0; j < D; ++j) x[k][j] = f.pts[(size_t)pc * f.sp + (size_t)j * f.ld];
               id[k] = pc;
             }
-            dm[k] = first && a.s_begin == 0 ? f.init : f.dmin[pc];
+            dm[k] = first && s_begin == 0 ? f.init : f.dmin[pc];
           }
           if (base + 64 * P > f.n) {
 #pragma unroll
@@ -338,6 +295,7 @@ __device__ __forceinline__ void rounds_cloud(const RoundsParams &a, const uint32
           bkey = make_key(wv, wt);
           if (lane == 0) s_bkey[lb] = bkey;
         }
+        bkey = uniform_u64(bkey);
         if (bkey > Tg) {
           uint64_t m[P];
           uint32_t total = 0;
@@ -364,9 +322,9 @@ __device__ __forceinline__ void rounds_cloud(const RoundsParams &a, const uint32
           }
         }
       }
-      wmax = bkey > wmax ? bkey : wmax;
+      wmax = uniform_u64(bkey > wmax ? bkey : wmax);
     }
-    first = false;
+    fresh = 0;
     if (last) return;
     if (!gather) {
       lds_barrier();
@@ -388,122 +346,12 @@ __device__ __forceinline__ void rounds_cloud(const RoundsParams &a, const uint32
     uint64_t U = wave_max_u64(lane < W ? S.wmax[lane] : 0ull);  // this workgroup's best key
 
     // ---- 2. exchange --------------------------------------------------------
-    // L lanes read one workgroup's header and its first L candidates at once, so most
-    // candidates are here as soon as their header is; those beyond L follow.
     uint32_t C = own;
     if (G > 1) {
-      const uint32_t capw = a.cap_wg;
-      const uint32_t hp = G;  // pitch of one header word's array
-      const size_t head = (size_t)kRoundsReplicas * kRoundsHeadWords * hp;
-      const size_t cp = (size_t)G * capw;  // pitch of one word's array
-      uint64_t *buf = f.xchg + (size_t)par * (head + NWC * cp);
-      uint64_t *cbuf = buf + head;
-      if (wave == 0) {
-        if (lane < (int)(kRoundsReplicas * kRoundsHeadWords)) {
-          const uint32_t rep = (uint32_t)lane / kRoundsHeadWords;
-          const uint32_t k = (uint32_t)lane - rep * kRoundsHeadWords;
-          const uint32_t v = k == 0 ? own : (k == 1 ? (uint32_t)(U >> 32) : (uint32_t)U);
-          xchg_store(buf + ((size_t)rep * kRoundsHeadWords + k) * hp + g,
-                     ((uint64_t)v << 32) | e);
-        }
-      } else if (own <= capw) {
-        for (uint32_t q = (uint32_t)tid - 64; q < own; q += kRoundsThreads - 64) {
-          const uint64_t k = S.lk[q];
-          const Rec<D> r = S.lc[q];
-          uint64_t *w = cbuf + (size_t)g * capw + q;
-          xchg_store(w, (k & 0xffffffff00000000ull) | e);
-          xchg_store(w + cp, (k << 32) | e);
-#pragma unroll
-          for (int j = 0; j < D; ++j)
-            xchg_store(w + (size_t)(2 + j) * cp,
-                       ((uint64_t)(uint32_t)__float_as_int(r.c[j]) << 32) | e);
-        }
-      }
-      const uint32_t L = G <= 128 ? 8 : 4;
-      const uint32_t q = (uint32_t)tid / L;
-      const uint32_t l = (uint32_t)tid & (L - 1);
-      uint64_t w1 = 0, w2 = 0;
-      if ((uint32_t)wave * 64 < G * L) {
-        const uint64_t *h =
-            buf + (size_t)(g % kRoundsReplicas) * kRoundsHeadWords * hp + q;
-        const uint64_t *w = cbuf + (size_t)q * capw;
-        uint32_t cq = 0;
-        uint64_t v[NWC];
-        const bool mine = q < G;
-        bool here = false;  // candidate l of workgroup q is there
-        if (mine) {
-          const uint64_t deadline = now_ticks() + f.spin_ticks;
-          for (;;) {
-            const uint64_t w0 = xchg_load(h);
-            w1 = xchg_load(h + hp);
-            w2 = xchg_load(h + 2 * hp);
-#pragma unroll
-            for (uint32_t k = 0; k < NWC; ++k) v[k] = xchg_load(w + l + k * cp);
-            bool all = true;
-#pragma unroll
-            for (uint32_t k = 0; k < NWC; ++k) all = all && (uint32_t)v[k] == e;
-            cq = (uint32_t)(w0 >> 32);
-            here = l < cq && cq <= capw;
-            if ((uint32_t)w0 == e && (uint32_t)w1 == e && (uint32_t)w2 == e && (all || !here)) break;
-            if (now_ticks() > deadline) {
-              S.ok = 0;
-              cq = 0;
-              here = false;
-              break;
-            }
-          }
-        }
-        const uint32_t sum =
-            (uint32_t)__builtin_amdgcn_readlane((int)wave_scan_add(l == 0 ? cq : 0u), 63);
-        if (lane == 0 && sum) atomicAdd(&S.sum[par], sum);
-        uint32_t i = l;
-        for (;;) {
-          const uint64_t m = __ballot(here);
-          if (!m) break;
-          uint32_t at = 0;
-          if (lane == 0) at = atomicAdd(&S.at[par], (uint32_t)__popcll(m));
-          at = (uint32_t)__builtin_amdgcn_readfirstlane((int)at) + lanes_below(m);
-          if (here && at < (uint32_t)LIST) {
-            S.ck[at] = (v[0] & 0xffffffff00000000ull) | (v[1] >> 32);
-            Rec<D> r;
-#pragma unroll
-            for (int j = 0; j < D; ++j) r.c[j] = __int_as_float((int)(v[2 + j] >> 32));
-            S.cc[at] = r;
-          }
-          i += L;
-          here = here && i < cq;
-          if (here) {
-            const uint64_t deadline = now_ticks() + f.spin_ticks;
-            for (;;) {
-              bool all = true;
-#pragma unroll
-              for (uint32_t k = 0; k < NWC; ++k) v[k] = xchg_load(w + i + k * cp);
-#pragma unroll
-              for (uint32_t k = 0; k < NWC; ++k) all = all && (uint32_t)v[k] == e;
-              if (all) break;
-              if (now_ticks() > deadline) {
-                S.ok = 0;
-                here = false;
-                break;
-              }
-            }
-          }
-        }
-      }
-      lds_barrier();
-      if (!__builtin_amdgcn_readfirstlane((int)S.ok)) {
+      if (!rounds_exchange<D, LIST>(f.xchg, f.spin_ticks, a.cap_wg, G, g, e, tid, wave, S, S.lk,
+                                    S.lc, S.ck, S.cc, C, U)) {
         if (tid == 0) atomicOr(f.status, kStatusTimeout);
         return;
-      }
-      C = S.sum[par];
-      const uint32_t got = S.at[par];
-      if (got != C || C > (uint32_t)LIST) C = max(C, (uint32_t)LIST + 1);  // some did not fit
-      if (C == 0) {
-        // Nobody has a candidate: the best key of all is the exact bound.
-        const uint64_t u = wave_max_u64((w1 & 0xffffffff00000000ull) | (w2 >> 32));
-        if (lane == 0) S.wmax[wave] = (uint32_t)wave * 64 < G * L ? u : 0ull;
-        lds_barrier();
-        U = wave_max_u64(lane < W ? S.wmax[lane] : 0ull);
       }
     } else {
       if ((uint32_t)tid < own && tid < CAP) {
@@ -543,24 +391,7 @@ __device__ __forceinline__ void rounds_cloud(const RoundsParams &a, const uint32
     }
 
     // ---- 3. front -----------------------------------------------------------
-    // Order of the candidates: how many keys exceed one's own, 16 at a time.
-    {
-      const uint32_t nc = (C + 63u) >> 6;
-      const uint32_t nj = (C + 15u) >> 4;
-      for (uint32_t job = wave; job < nc * nj; job += W) {
-        const uint32_t jc = job / nc, ic = job - jc * nc;
-        const uint32_t i = ic * 64 + lane;
-        const uint64_t ki = S.ck[i];
-        const uint64_t *kj = S.ck + jc * 16;
-        uint32_t r = 0;
-#pragma unroll 1
-        for (int h = 0; h < 16; h += 8) {
-#pragma unroll
-          for (int l = 0; l < 8; ++l) r += kj[h + l] > ki ? 1u : 0u;
-        }
-        if (i < C && r) atomicAdd(&S.rank[i], r);
-      }
-    }
+    rank_candidates(S.ck, S.rank, C, tid, wave);
     lds_barrier();
     if ((uint32_t)tid < C) {
       const uint32_t r = S.rank[tid];
@@ -607,37 +438,8 @@ __device__ __forceinline__ void rounds_cloud(const RoundsParams &a, const uint32
       job += W;
     }
     lds_barrier();
-    // The picks, were no candidate only partly lowered: each candidate that no earlier pick
-    // lowers, settled in a few steps per 64 candidates rather than one by one.
     const uint32_t *rows = (const uint32_t *)&S.low[0][0][0];
-    if (wave == 0) {
-      uint64_t low[CH][CH];
-#pragma unroll
-      for (int c = 0; c < CH; ++c)
-#pragma unroll
-        for (int w = 0; w <= c; ++w)
-          low[c][w] = ((uint64_t)rows[(2 * w + 1) * CAP + c * 64 + lane] << 32) |
-                      rows[2 * w * CAP + c * 64 + lane];
-      uint64_t acc[CH];
-#pragma unroll
-      for (int c = 0; c < CH; ++c) {
-        acc[c] = 0;
-        if ((uint32_t)c < nc) {
-          uint64_t before = 0;
-#pragma unroll
-          for (int w = 0; w < c; ++w) before |= low[c][w] & acc[w];
-          const uint64_t same = low[c][c] & (((uint64_t)1 << lane) - 1);
-          uint64_t open = __ballot((uint32_t)(c * 64 + lane) < F && before == 0);
-          while (open) {
-            const uint64_t free = __ballot((same & open) == 0) & open;
-            acc[c] |= free;
-            open &= ~free;
-            open &= ~__ballot((same & free) != 0);
-          }
-        }
-        if (lane == 0) S.acc[c] = acc[c];
-      }
-    }
+    if (wave == 0) settle_candidates<CAP>(rows, F, lane, S.acc);
     lds_barrier();
     // A candidate whose first lowering pick leaves its key above the bound raises the bound
     // to that key; a pick that does not lower itself ends the round.
@@ -700,36 +502,18 @@ __device__ __forceinline__ void rounds_cloud(const RoundsParams &a, const uint32
     lds_barrier();
     idle = 0;
     np = (uint32_t)__builtin_amdgcn_readfirstlane((int)S.np);
-    {
-      // The square root damps the step against the count's own noise.
-      double r = sqrt((double)a.target / (double)C);
-      r = r > 4.0 ? 4.0 : r;
-      const double ns = (double)step * r;
-      step = ns < 1.0 ? 1 : (ns > 4.0e18 ? (uint64_t)1 << 61 : (uint64_t)ns);
-      Tg = T > step ? T - step : 0;
-    }
+    step = next_step(step, a.target, C);
+    Tg = T > step ? T - step : 0;
   }
 }
 
 template <int D, int P, int TIE>
-__global__ void __launch_bounds__(kRoundsThreads) fps_rounds(RoundsParams a) {
+__global__ void __launch_bounds__(kRoundsThreads) fps_rounds(RoundsParams) {
   extern __shared__ uint64_t s_dyn[];
   __shared__ RoundsLds<D> S;
-  rounds_cloud<D, P, TIE>(a, blockIdx.x, gridDim.x, S, s_dyn);
-}
-
-// A table entry in scalar registers: read in place, its fields would come through vector
-// loads again after every store.
-__device__ __forceinline__ RoundsParams uniform_params(const RoundsParams *p) {
-  constexpr int N = sizeof(RoundsParams) / 4;
-  union {
-    RoundsParams a;
-    uint32_t w[N];
-  } u;
-#pragma unroll
-  for (int i = 0; i < N; ++i)
-    u.w[i] = (uint32_t)__builtin_amdgcn_readfirstlane((int)((const uint32_t *)p)[i]);
-  return u.a;
+  // (its only argument)
+  rounds_cloud<D, P, TIE>((ParamsPtr)__builtin_amdgcn_kernarg_segment_ptr(), blockIdx.x, gridDim.x,
+                          S, s_dyn);
 }
 
 // Many clouds: workgroups claim member slots in order (or own one each), a job's members
@@ -746,17 +530,16 @@ __global__ void __launch_bounds__(kRoundsThreads) fps_rounds_jobs(RoundsJobs j) 
     __syncthreads();
     const uint32_t slot = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_slot);
     if (slot >= j.members) return;
-    const RoundsParams a = uniform_params(
-        j.table + (uint32_t)__builtin_amdgcn_readfirstlane((int)j.member_job[slot]));
-    if (a.team > 1) {
+    const ParamsPtr p = (ParamsPtr)j.table + uniform_u32(j.member_job[slot]);
+    if (p->team > 1) {
       // Wait for the team to form, so that exchange waits are short ones.
       if (threadIdx.x == 0) {
-        atomicAdd(a.ready, 1u);
+        atomicAdd(p->ready, 1u);
         const uint64_t deadline = now_ticks() + j.team_ticks;
         uint32_t here = 1;
-        while (__hip_atomic_load(a.ready, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < a.team) {
+        while (__hip_atomic_load(p->ready, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < p->team) {
           if (now_ticks() > deadline) {
-            atomicOr(a.fps.status, kStatusTimeout);
+            atomicOr(p->fps.status, kStatusTimeout);
             here = 0;
             break;
           }
@@ -767,8 +550,7 @@ __global__ void __launch_bounds__(kRoundsThreads) fps_rounds_jobs(RoundsJobs j) 
       __syncthreads();
       if (!__builtin_amdgcn_readfirstlane((int)s_slot)) return;
     }
-    rounds_cloud<D, P, kTieHighest>(
-        a, (uint32_t)__builtin_amdgcn_readfirstlane((int)(slot - a.member_base)), a.team, S, s_dyn);
+    rounds_cloud<D, P, kTieHighest>(p, uniform_u32(slot - p->member_base), p->team, S, s_dyn);
     if (j.one_slot) return;
     __syncthreads();
   }

@@ -28,6 +28,15 @@ struct RoundsParams {
   uint32_t *ready;
 };
 
+// Any dimension (fps_rounds_any.hip): candidates a round decides on; rest holds the points by
+// coordinate (j at rest[j * n + i]), rec is unused.
+constexpr uint32_t kAnyCap = 128;
+constexpr uint32_t kAnyMaxDim = 256;
+inline size_t rounds_any_shmem(uint32_t dim, uint32_t nbl) {
+  return ((size_t)kAnyCap * (dim | 1u) + (size_t)nbl * 64) * sizeof(float);
+}
+const KernelEntry *rounds_any_kernel(int tie);
+
 struct RoundsJobs {
   const RoundsParams *table;
   const uint32_t *member_job;  // slot -> entry of table
@@ -51,10 +60,17 @@ inline uint32_t rounds_target(size_t m) {
 inline uint32_t rounds_cap_wg(uint32_t grid) {
   return grid <= 8 ? kRoundsCap : grid <= 64 ? 64 : 32;
 }
+// Words between the arrays of a header's words: 2 KiB apart they lie on different memory
+// channels, which all workgroups' polls then share (64 workgroups, 50 K points: 9.1 us a round
+// against 9.6 with the arrays end to end).  Small teams, of which a launch has many, stay close.
+constexpr __host__ __device__ uint32_t rounds_head_pitch(uint32_t grid) {
+  return grid < 16 ? 16 : 256;
+}
 // Exchange words of a grid: two buffers of headers and candidates.
 inline size_t rounds_xchg_words(uint32_t grid, uint32_t dim, uint32_t cap_wg) {
   if (grid <= 1) return 1;
-  return (size_t)2 * grid * (kRoundsReplicas * kRoundsHeadWords + (2 + dim) * cap_wg);
+  return (size_t)2 * ((size_t)kRoundsReplicas * kRoundsHeadWords * rounds_head_pitch(grid) +
+                      (size_t)(2 + dim) * grid * cap_wg);
 }
 // Dynamic LDS of a workgroup holding nbl blocks: box and best key of each.
 inline size_t rounds_shmem(uint32_t dim, uint32_t nbl) {

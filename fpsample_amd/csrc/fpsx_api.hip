@@ -424,6 +424,28 @@ static int plan_rounds(Ctx &c, size_t n, size_t dim, int tie, size_t m, Plan &p)
   int P = 0, G = 0, target = 0, order = -1;
   if (const char *env = std::getenv("FPSX_ROUNDS"))
     if (*env) std::sscanf(env, "%d:%d:%d:%d", &P, &G, &target, &order);
+  if (dim > 8) {
+    // Any dimension: blocks of 64 points, one or two a workgroup.
+    const KernelEntry *k = rounds_any_kernel(tie);
+    if (dim > kAnyMaxDim) return fail(FPSX_ETOOBIG, "threshold rounds: too many dimensions");
+    const size_t nblocks = (n + 63) / 64;
+    size_t g = G > 0 ? (size_t)G : std::min<size_t>(nblocks, 256);
+    g = std::min<size_t>(std::min<size_t>(g, nblocks), kRoundsMaxGrid);
+    const size_t nbl = (nblocks + g - 1) / g;
+    const size_t shmem = rounds_any_shmem((uint32_t)dim, (uint32_t)nbl);
+    if (shmem > 144 * 1024) return fail(FPSX_ETOOBIG, "threshold rounds: too many points");
+    if (g > (size_t)c.max_blocks(k, shmem))
+      return fail(FPSX_ETOOBIG, "threshold rounds: grid exceeds co-residency");
+    p.kind = PlanKind::Rounds;
+    p.k = k;
+    p.block = kRoundsThreads;
+    p.grid = (uint32_t)g;
+    p.chunk = (uint32_t)(nbl * 64);
+    p.shmem = shmem;
+    p.target = target > 0 ? std::min<uint32_t>((uint32_t)target, kAnyCap) : 64;
+    p.order = false;
+    return FPSX_OK;
+  }
   if (P <= 0) P = n <= 65536 && dim != 1 ? 1 : n <= 524288 || dim == 1 || dim > 3 ? 4 : 8;
   size_t cnt;
   const KernelEntry *t = rounds_table(&cnt);
@@ -773,18 +795,23 @@ int launch_fps(Ctx &c, const Plan &p, const float *d_pts, size_t sp, size_t ld, 
   FpsParams a;
   rc = common_params(c, d_pts, sp, ld, n, dim, m, d_starts, n_starts, d_out, d_out_pts, init,
                      p.chunk, st, a,
-                     p.kind == PlanKind::Rounds ? rounds_xchg_words(p.grid, (uint32_t)dim, rounds_cap_wg(p.grid)) : 0);
+                     p.kind == PlanKind::Rounds
+                         ? rounds_xchg_words(p.grid, p.k->dim ? (uint32_t)dim : 0,
+                                             rounds_cap_wg(p.grid))
+                         : 0);
   if (rc) return rc;
   RoundsParams ra;
   if (p.kind == PlanKind::Rounds) {
-    HIP_TRY(c.dmin.reserve(n * sizeof(float)));
-    a.dmin = (float *)c.dmin.p;
+    if (p.k->dim) {
+      HIP_TRY(c.dmin.reserve(n * sizeof(float)));
+      a.dmin = (float *)c.dmin.p;
+    }
     const uint32_t block = (uint32_t)(64 * p.k->ppt);
     ra.fps = a;
     ra.rec = nullptr;
     ra.rest = nullptr;
     ra.nblocks = (uint32_t)((n + block - 1) / block);
-    ra.cap_wg = rounds_cap_wg(p.grid);
+    ra.cap_wg = p.k->dim ? rounds_cap_wg(p.grid) : std::min(rounds_cap_wg(p.grid), kAnyCap);
     ra.target = p.target;
     ra.s_begin = 0;
     ra.s_end = (uint32_t)m;
@@ -793,6 +820,16 @@ int launch_fps(Ctx &c, const Plan &p, const float *d_pts, size_t sp, size_t ld, 
     ra.team = p.grid;
     ra.member_base = 0;
     ra.ready = nullptr;
+    if (!p.k->dim) {
+      // The points by coordinate, n apart: in place when they lie so.
+      ra.rest = d_pts;
+      if (sp != 1 || ld != n) {
+        HIP_TRY(c.rest.reserve(n * dim * sizeof(float)));
+        HIP_TRY(launch_strided_to_soa(d_pts, sp, ld, (float *)c.rest.p, (uint32_t)n,
+                                      (uint32_t)dim, n, st));
+        ra.rest = (const float *)c.rest.p;
+      }
+    }
     if (p.order) {
       HIP_TRY(c.rec.reserve(n * sizeof(float4)));
       if (dim > 3) HIP_TRY(c.rest.reserve(n * (dim - 3) * sizeof(float)));

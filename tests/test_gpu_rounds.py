@@ -108,6 +108,26 @@ def test_rounds_dimensions(gpu, rounds_env, d):
         check(sp, 300, 1, "special")
 
 
+@pytest.mark.parametrize("d", [9, 32, 63, 256])
+def test_rounds_any_dimension(gpu, rounds_env, d):
+    # Beyond eight dimensions: one and several workgroups, several blocks of one workgroup,
+    # dimensions around the unrolled four, the largest; prefixes beyond a round's 128 picks.
+    rng = np.random.default_rng(80 + d)
+    for shape in ("1:1", "1:3:100", "1:40:30"):
+        rounds_env(shape)
+        for n, m in ((1, 1), (65, 65), (2001, 300)):
+            check(rng.standard_normal((n, d)).astype(np.float32), m, int(rng.integers(n)), "any")
+        check(rng.integers(0, 2, (700, d)).astype(np.float32), 700, 5, "ties")
+        sp = (rng.random((900, d)) * 4e19).astype(np.float32)
+        sp[11, d - 1] = np.inf
+        check(sp, 100, 1, "overflow")
+        sp[[7, 800], 0] = np.nan
+        check(sp, 100, 1, "nan")
+        pc = rng.random((1500, d)).astype(np.float32)
+        for count in (128, 129, 300):
+            check(pc, 330, [int(v) for v in rng.integers(0, 1500, count)], f"prefix {count}")
+
+
 @pytest.mark.parametrize("n", [8191, 8192, 8193, 20000, 70001])
 def test_rounds_order_sizes(gpu, rounds_env, n):
     # The order's one-workgroup form, its last size, several chunks, a ragged last chunk;
