@@ -213,23 +213,37 @@ __device__ __forceinline__ void rounds_cloud(ParamsPtr params, const uint32_t gr
       }
       if (any || bkey > Tg) {
         if (first || !resident) {
+          // Every load of the block before any use: one memory round trip (chosen per point, the
+          // kind of load made one trip of each: 2^24 points, 2048 picks, 4.84 against 4.58 ms;
+          // 256 clouds of 2 K to 65 K points 3.72 against 3.24 ms).
+          uint32_t pc[P];
 #pragma unroll
-          for (int k = 0; k < P; ++k) {
-            const uint32_t p = base + (uint32_t)(k * 64 + lane);
-            const uint32_t pc = min(p, f.n - 1);
-            if (a.rec) {
-              const float4 r = a.rec[pc];
+          for (int k = 0; k < P; ++k) pc[k] = min(base + (uint32_t)(k * 64 + lane), f.n - 1);
+          if (first && s_begin == 0) {
+#pragma unroll
+            for (int k = 0; k < P; ++k) dm[k] = f.init;
+          } else {
+#pragma unroll
+            for (int k = 0; k < P; ++k) dm[k] = f.dmin[pc[k]];
+          }
+          if (a.rec) {
+#pragma unroll
+            for (int k = 0; k < P; ++k) {
+              const float4 r = a.rec[pc[k]];
               const float r3[3] = {r.x, r.y, r.z};
 #pragma unroll
               for (int j = 0; j < D; ++j)
-                x[k][j] = j < 3 ? r3[j < 3 ? j : 0] : a.rest[(size_t)(j - 3) * f.n + pc];
+                x[k][j] = j < 3 ? r3[j < 3 ? j : 0] : a.rest[(size_t)(j - 3) * f.n + pc[k]];
               id[k] = (uint32_t)__float_as_int(r.w);
-            } else {
-#pragma unroll
-              for (int j = 0; j < D; ++j) x[k][j] = f.pts[(size_t)pc * f.sp + (size_t)j * f.ld];
-              id[k] = pc;
             }
-            dm[k] = first && s_begin == 0 ? f.init : f.dmin[pc];
+          } else {
+#pragma unroll
+            for (int k = 0; k < P; ++k) {
+#pragma unroll
+              for (int j = 0; j < D; ++j)
+                x[k][j] = f.pts[(size_t)pc[k] * f.sp + (size_t)j * f.ld];
+              id[k] = pc[k];
+            }
           }
           if (base + 64 * P > f.n) {
 #pragma unroll
