@@ -20,13 +20,13 @@
 // of equal distances.
 //
 // What bounds it: a round's serial chain, not bytes (2^20 clustered points, 16384 picks, 128
-// workgroups: 224 rounds of 9.5 us).  Of a round (100 K points, 64 workgroups, 363 rounds of
-// 9.5 us): update 2.2 us with the wait for the slowest wave, exchange 2.9, sorting 1.4, rows
-// 1.9 (the vector ALUs are busy throughout: 10 instructions for 64 pairs), settling 0.4, the
-// bound and the picks 1.1.  Settling the candidates one by one instead took 450 ns a pick.
-// A block per wave in registers, the candidates loaded beside the headers and the best 256
-// taken from up to 512 brought gauss1m from 2.67 to 2.13 ms, 100 K / 50 K picks from 4.52 to
-// 3.44 ms.
+// workgroups: 206 rounds of 10.3 us).  Of a round (50 K points, 64 workgroups, 73 rounds of 9
+// us): update 2.2 us with the wait for the slowest wave, exchange 3.0, sorting 0.9, rows 1.4,
+// settling 0.4, the bound and the picks 0.6.  Settling the candidates one by one instead took
+// 450 ns a pick.  A block per wave in registers, the candidates loaded beside the headers and
+// the best 256 taken from up to 512 brought 2^20 clustered points from 2.67 to 2.13 ms, 100 K /
+// 50 K picks from 4.52 to 3.44 ms; jobs of half-waves in the sorting and the rows and one pass
+// for bound and picks, 50 K / 4096 picks from 668 to 654 us, 2^22 / 4096 picks 2.09 to 2.03 ms.
 #include "fps_rounds.hpp"
 
 #include "fps_device.hpp"
@@ -44,7 +44,8 @@ struct RoundsLds : RoundsCounts {
   alignas(16) uint64_t ck[LIST];  // candidates as they came
   Rec<D> cc[LIST];
   Rec<D> pk[CAP];                 // picks of the round
-  uint32_t pt[CAP];               // their tie words
+  uint32_t pt[CAP];               // their keys' low halves: tie words
+  uint32_t pv[CAP];               // and high halves
   uint32_t rank[LIST];
   uint64_t sk[CAP];               // sorted candidates
   Rec<D> sc[CAP];
@@ -72,9 +73,8 @@ __device__ __forceinline__ void rounds_cloud(ParamsPtr params, const uint32_t gr
 
   if (tid == 0) {
     S.last = ~0ull;
-    S.cnt[0] = S.cnt[1] = 0;
-    S.sum[0] = S.sum[1] = 0;
-    S.at[0] = S.at[1] = 0;
+    S.clear(0);
+    S.clear(1);
     S.stuck = 0;
     S.ok = 1;
   }
@@ -349,10 +349,6 @@ __device__ __forceinline__ void rounds_cloud(ParamsPtr params, const uint32_t gr
       S.ck[tid] = 0;
       S.rank[tid] = 0;
     }
-    if (tid == 0) {
-      S.te = Tg;
-      S.stop = ~0u;
-    }
     lds_barrier();
     ++e;
     const uint32_t par = e & 1u;
@@ -375,12 +371,7 @@ __device__ __forceinline__ void rounds_cloud(ParamsPtr params, const uint32_t gr
       if (own > (uint32_t)CAP) C = max(own, (uint32_t)LIST + 1);
       lds_barrier();
     }
-    if (tid == 0) {  // the other parity's counters: everybody has read them
-      S.np = 0;
-      S.cnt[par ^ 1] = 0;
-      S.sum[par ^ 1] = 0;
-      S.at[par ^ 1] = 0;
-    }
+    if (tid == 0) S.clear(par ^ 1);  // everybody has read the last round's
     U = uniform_u64(U);
     C = (uint32_t)__builtin_amdgcn_readfirstlane((int)C);
     if (C > (uint32_t)LIST || C == 0) {
@@ -413,62 +404,68 @@ __device__ __forceinline__ void rounds_cloud(ParamsPtr params, const uint32_t gr
         S.sk[r] = S.ck[tid];
         S.sc[r] = S.cc[tid];
       } else if (r == (uint32_t)CAP) {
-        S.te = S.ck[tid];  // the first one that the front does not see is the bound
+        S.te[par] = S.ck[tid];  // the first one that the front does not see is the bound
       }
     }
     lds_barrier();
     const uint32_t F = min(C, (uint32_t)CAP);
     const uint32_t nc = (F + 63u) >> 6;
     // Which earlier candidates lower a candidate: bit j of candidate i's row, j < i, for the
-    // sorted candidates.  A job is 64 candidates against 16 earlier ones.
-    for (uint32_t job = wave, c = 0; c < nc;) {
-      if (job >= 4 * (c + 1)) {
-        job -= 4 * (c + 1);
+    // sorted candidates.  A job is 32 candidates against 32 earlier ones, 16 for each half of
+    // the wave: the triangle and its ragged end then waste few lanes (146 candidates: 15 jobs,
+    // one a wave, against 22 of 64 x 16: 1.3 us a round against 1.65).
+    for (uint32_t job = wave, c = 0; c * 32 < F;) {
+      if (job > c) {
+        job -= c + 1;
         ++c;
         continue;
       }
-      const uint32_t j0 = job * 16;
-      if (j0 < F) {
-        const uint32_t i = c * 64 + lane;
-        const float v = __int_as_float((int)(uint32_t)(S.sk[i] >> 32) - 1);
-        const Rec<D> ri = S.sc[i];
-        float xi[D];
+      const uint32_t i = c * 32 + (lane & 31);
+      const uint32_t jb = job * 2 + (lane >> 5);  // block of 16 earlier ones
+      const float v = __int_as_float((int)(uint32_t)(S.sk[i] >> 32) - 1);
+      const Rec<D> ri = S.sc[i];
+      float xi[D];
 #pragma unroll
-        for (int j = 0; j < D; ++j) xi[j] = ri.c[j];
-        uint32_t bits = 0;
+      for (int j = 0; j < D; ++j) xi[j] = ri.c[j];
+      uint32_t bits = 0;
 #pragma unroll 1
-        for (int h = 12; h >= 0; h -= 4) {
+      for (int h = 12; h >= 0; h -= 4) {
 #pragma unroll
-          for (int l = 3; l >= 0; --l) {
-            const Rec<D> rj = S.sc[j0 + h + l];
-            float p[D];
+        for (int l = 3; l >= 0; --l) {
+          const Rec<D> rj = S.sc[jb * 16 + h + l];
+          float p[D];
 #pragma unroll
-            for (int j = 0; j < D; ++j) p[j] = rj.c[j];
-            bits = bits + bits + (sqdist<D>(xi, p) < v ? 1u : 0u);
-          }
+          for (int j = 0; j < D; ++j) p[j] = rj.c[j];
+          bits = bits + bits + (sqdist<D>(xi, p) < v ? 1u : 0u);
         }
-        S.low[job >> 1][i][job & 1] = (uint16_t)bits;
       }
+      S.low[job][i][lane >> 5] = (uint16_t)bits;
       job += W;
     }
     lds_barrier();
     const uint32_t *rows = (const uint32_t *)&S.low[0][0][0];
     if (wave == 0) settle_candidates<CAP>(rows, F, lane, S.acc);
     lds_barrier();
-    // A candidate whose first lowering pick leaves its key above the bound raises the bound
-    // to that key; a pick that does not lower itself ends the round.
-    uint64_t key = 0;
-    uint64_t taken = 0;
-    Rec<D> ri;
+    // The picks, in order.  A candidate whose first lowering pick leaves its key above the
+    // bound raises the bound to that key, and a pick that does not lower itself ends the round:
+    // both are rare and cut the picks below.
     if ((uint32_t)wave < nc) {
       const uint32_t i = (uint32_t)tid;
-      key = S.sk[i];
-      ri = S.sc[i];
+      const uint64_t key = S.sk[i];
+      const Rec<D> ri = S.sc[i];
       const float v = __int_as_float((int)(uint32_t)(key >> 32) - 1);
       float xi[D];
 #pragma unroll
       for (int j = 0; j < D; ++j) xi[j] = ri.c[j];
-      taken = uniform_u64(S.acc[wave]);
+      uint64_t acc[CH];
+      uint32_t at = 0, all = 0;
+#pragma unroll
+      for (int w = 0; w < CH; ++w) {
+        acc[w] = uniform_u64(S.acc[w]);
+        if (w < wave) at += (uint32_t)__popcll(acc[w]);
+        all += (uint32_t)__popcll(acc[w]);
+      }
+      const uint64_t taken = uniform_u64(S.acc[wave]);
       const bool mine = (taken >> lane) & 1;
       int by = -1;
 #pragma unroll
@@ -476,46 +473,51 @@ __device__ __forceinline__ void rounds_cloud(ParamsPtr params, const uint32_t gr
         if (w <= wave) {
           uint64_t k = ((uint64_t)rows[(2 * w + 1) * CAP + i] << 32) | rows[2 * w * CAP + i];
           if (w == wave) k &= ((uint64_t)1 << lane) - 1;
-          k &= S.acc[w];
+          k &= acc[w];
           if (k) by = w * 64 + __ffsll((unsigned long long)k) - 1;
         }
       }
-      if (i < F && !mine && by >= 0) {
+      const uint32_t q = at + lanes_below(taken);
+      if (mine) {
+        S.pt[q] = (uint32_t)key;
+        S.pv[q] = (uint32_t)(key >> 32);
+        S.pk[q] = ri;
+        if (!(sqdist<D>(xi, xi) < v)) atomicMin(&S.stop[par], q);
+      } else if (i < F && by >= 0) {
         const Rec<D> rb = S.sc[by];
         float p[D];
 #pragma unroll
         for (int j = 0; j < D; ++j) p[j] = rb.c[j];
-        const uint64_t nk = make_key(__float_as_int(sqdist<D>(xi, p)), (uint32_t)key);
-        if (nk > Tg) atomicMax((unsigned long long *)&S.te, (unsigned long long)nk);
+        const float d = sqdist<D>(xi, p);
+        const uint64_t nk = make_key(__float_as_int(d), (uint32_t)key);
+        if (nk > Tg) atomicMax((unsigned long long *)&S.te[par], (unsigned long long)nk);
       }
-      if (i < F && mine && !(sqdist<D>(xi, xi) < v)) atomicMin(&S.stop, i);
+      if (tid == 0) S.np[par] = all;
     }
     lds_barrier();
-    T = uniform_u64(S.te);
-    if ((uint32_t)wave < nc) {
-      const uint32_t stop = S.stop;
-      // Keys fall along the chunks: a chunk with picks has those before it whole.
-      uint32_t at = 0;
-      for (int w = 0; w < wave; ++w) at += (uint32_t)__popcll(S.acc[w]);
-      taken &= __ballot(key > T && (uint32_t)tid <= stop);
-      at = (uint32_t)__builtin_amdgcn_readfirstlane((int)at);
-      const uint32_t room = a.s_end - s;
-      if (taken) {
-        const uint32_t q = at + lanes_below(taken);
-        const uint32_t upto = min(at + (uint32_t)__popcll(taken), room);
-        if (((taken >> lane) & 1) && q < room) {
-          S.pt[q] = (uint32_t)key;
-          S.pk[q] = ri;
-          if (q == room - 1) S.last = key;
-        }
-        if (lane == 0) atomicMax(&S.np, upto);
-        if (stop - (uint32_t)wave * 64 < 64u && ((taken >> (stop & 63u)) & 1) && lane == 0)
-          S.stuck = 1;
+    np = uniform_u32(S.np[par]);
+    T = uniform_u64(S.te[par]);
+    T = T > Tg ? T : Tg;
+    const uint32_t stop = uniform_u32(S.stop[par]);
+    if (T > Tg || stop < np) {
+      // Picks up to the stop whose keys exceed the bound (keys fall along the picks).
+      uint32_t keep = 0;
+      for (uint32_t c = 0; c < np; c += 64) {
+        const uint32_t q = c + lane;
+        const uint64_t k = q < np ? ((uint64_t)S.pv[q] << 32) | S.pt[q] : 0ull;
+        keep += (uint32_t)__popcll(__ballot(k > T && q <= stop));
+      }
+      np = keep;
+      if (stop < np) {
+        lds_barrier();  // (nobody reads S.stuck between)
+        if (tid == 0) S.stuck = 1;
+        lds_barrier();
       }
     }
-    lds_barrier();
+    np = min(np, a.s_end - s);
+    if (s + np == a.s_end && a.s_end < f.m && tid == 0)
+      S.last = ((uint64_t)S.pv[np - 1] << 32) | S.pt[np - 1];
     idle = 0;
-    np = (uint32_t)__builtin_amdgcn_readfirstlane((int)S.np);
     step = next_step(step, a.target, C);
     Tg = T > step ? T - step : 0;
   }

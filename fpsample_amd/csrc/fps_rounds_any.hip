@@ -81,9 +81,8 @@ __global__ void __launch_bounds__(kRoundsThreads) fps_rounds_any(RoundsParams) {
   int *s_dm = (int *)(s_any + (size_t)CAP * pitch);
 
   if (tid == 0) {
-    S.cnt[0] = S.cnt[1] = 0;
-    S.sum[0] = S.sum[1] = 0;
-    S.at[0] = S.at[1] = 0;
+    S.clear(0);
+    S.clear(1);
     S.stuck = 0;
     S.ok = 1;
   }
@@ -204,10 +203,6 @@ __global__ void __launch_bounds__(kRoundsThreads) fps_rounds_any(RoundsParams) {
       s_ck[tid] = 0;
       s_rank[tid] = 0;
     }
-    if (tid == 0) {
-      S.te = Tg;
-      S.stop = ~0u;
-    }
     lds_barrier();
     ++e;
     const uint32_t par = e & 1u;
@@ -227,12 +222,7 @@ __global__ void __launch_bounds__(kRoundsThreads) fps_rounds_any(RoundsParams) {
       if (own > (uint32_t)CAP) C = max(own, (uint32_t)LIST + 1);
       lds_barrier();
     }
-    if (tid == 0) {  // the other parity's counters: everybody has read them
-      S.np = 0;
-      S.cnt[par ^ 1] = 0;
-      S.sum[par ^ 1] = 0;
-      S.at[par ^ 1] = 0;
-    }
+    if (tid == 0) S.clear(par ^ 1);  // everybody has read the last round's
     U = uniform_u64(U);
     C = (uint32_t)__builtin_amdgcn_readfirstlane((int)C);
     if (C > (uint32_t)LIST || C == 0) {
@@ -262,7 +252,7 @@ __global__ void __launch_bounds__(kRoundsThreads) fps_rounds_any(RoundsParams) {
       if (r < (uint32_t)CAP)
         s_sk[r] = s_ck[tid];
       else if (r == (uint32_t)CAP)
-        S.te = s_ck[tid];  // the first one that the front does not see is the bound
+        S.te[par] = s_ck[tid];  // the first one that the front does not see is the bound
     }
     lds_barrier();
     const uint32_t F = min(C, (uint32_t)CAP);
@@ -324,17 +314,18 @@ __global__ void __launch_bounds__(kRoundsThreads) fps_rounds_any(RoundsParams) {
           d = d + df * df;
         }
         if (mine) {
-          if (!(d < v)) atomicMin(&S.stop, i);
+          if (!(d < v)) atomicMin(&S.stop[par], i);
         } else {
           const uint64_t nk = make_key(__float_as_int(d), (uint32_t)key);
-          if (nk > Tg) atomicMax((unsigned long long *)&S.te, (unsigned long long)nk);
+          if (nk > Tg) atomicMax((unsigned long long *)&S.te[par], (unsigned long long)nk);
         }
       }
     }
     lds_barrier();
-    T = uniform_u64(S.te);
+    T = uniform_u64(S.te[par]);
+    T = T > Tg ? T : Tg;
     if ((uint32_t)wave < nc) {
-      const uint32_t stop = S.stop;
+      const uint32_t stop = S.stop[par];
       uint32_t at = 0;
       for (int w = 0; w < wave; ++w) at += (uint32_t)__popcll(s_acc[w]);
       taken &= __ballot(key > T && (uint32_t)tid <= stop);
@@ -346,14 +337,14 @@ __global__ void __launch_bounds__(kRoundsThreads) fps_rounds_any(RoundsParams) {
           s_pt[q] = (uint32_t)key;
           s_pp[q] = (uint32_t)tid;
         }
-        if (lane == 0) atomicMax(&S.np, min(at + (uint32_t)__popcll(taken), room));
+        if (lane == 0) atomicMax(&S.np[par], min(at + (uint32_t)__popcll(taken), room));
         if (stop - (uint32_t)wave * 64 < 64u && ((taken >> (stop & 63u)) & 1) && lane == 0)
           S.stuck = 1;
       }
     }
     lds_barrier();
     idle = 0;
-    np = (uint32_t)__builtin_amdgcn_readfirstlane((int)S.np);
+    np = uniform_u32(S.np[par]);
     step = next_step(step, a.target, C);
     Tg = T > step ? T - step : 0;
   }

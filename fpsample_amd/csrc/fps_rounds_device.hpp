@@ -56,12 +56,19 @@ struct RoundsCounts {
   uint32_t sum[2];  // candidates of the grid, by round parity
   uint32_t at[2];   // candidates taken in, by round parity
   uint64_t wmax[kRoundsThreads / 64];  // best key of every wave
-  uint64_t te;      // the bound that the round's picks exceed
+  uint64_t te[2];   // keys that the round's picks must exceed beside its bound, by round parity
+  uint32_t stop[2]; // first pick that does not lower itself, by round parity
+  uint32_t np[2];   // picks, by round parity
   uint64_t last;    // key of the last pick where the run is cut there
-  uint32_t stop;    // first pick that does not lower itself
-  uint32_t np;
   uint32_t stuck;
   uint32_t ok;
+
+  __device__ __forceinline__ void clear(int parity) {
+    cnt[parity] = sum[parity] = at[parity] = 0;
+    te[parity] = 0;
+    stop[parity] = ~0u;
+    np[parity] = 0;
+  }
 };
 
 // The exchange of round e: own candidates (keys lk, coordinates lc) out, everybody's into ck and
@@ -215,26 +222,45 @@ __device__ __forceinline__ bool rounds_exchange(uint64_t *xchg, uint64_t spin_ti
   return true;
 }
 
-// Adds to rank[i] how many of the C keys exceed key i, 16 at a time (ck is 0 beyond C, up to
-// the next multiple of 16; rank starts at 0).
+// Adds to rank[i] how many of the C keys exceed key i (ck is 0 beyond C, up to the next
+// multiple of 16; rank starts at 0).  A job is 32 keys against 16, eight for each half of the
+// wave, so that a last piece of few keys costs little.  The comparison is a subtraction's
+// borrow, added with carry: three instructions a pair and no 64-bit compare (the compiler
+// makes that compare again of __builtin_subc).
 __device__ __forceinline__ void rank_candidates(const uint64_t *ck, uint32_t *rank, uint32_t C,
                                                 int tid, int wave) {
   const int lane = tid & 63;
   constexpr int W = kRoundsThreads / 64;
-  const uint32_t nc = (C + 63u) >> 6;
+  const uint32_t nc = (C + 31u) >> 5;
   const uint32_t nj = (C + 15u) >> 4;
-  for (uint32_t job = wave; job < nc * nj; job += W) {
-    const uint32_t jc = job / nc, ic = job - jc * nc;
-    const uint32_t i = ic * 64 + lane;
+  uint32_t ic = wave;
+  uint32_t jc = 0;
+  while (ic >= nc) {
+    ic -= nc;
+    ++jc;
+  }
+  while (jc < nj) {
+    const uint32_t i = ic * 32 + (lane & 31);
     const uint64_t ki = ck[i];
-    const uint64_t *kj = ck + jc * 16;
+    const uint64_t *kj = ck + jc * 16 + (lane >> 5) * 8;
     uint32_t r = 0;
-#pragma unroll 1
-    for (int h = 0; h < 16; h += 8) {
 #pragma unroll
-      for (int l = 0; l < 8; ++l) r += kj[h + l] > ki ? 1u : 0u;
+    for (int l = 0; l < 8; ++l) {
+      const uint64_t k = kj[l];
+      uint32_t t;
+      asm("v_sub_co_u32 %1, vcc, %2, %3\n\t"
+          "v_subb_co_u32 %1, vcc, %4, %5, vcc\n\t"
+          "v_addc_co_u32 %0, vcc, 0, %0, vcc"
+          : "+v"(r), "=&v"(t)
+          : "v"((uint32_t)ki), "v"((uint32_t)k), "v"((uint32_t)(ki >> 32)), "v"((uint32_t)(k >> 32))
+          : "vcc");
     }
     if (i < C && r) atomicAdd(&rank[i], r);
+    ic += W;
+    while (ic >= nc) {
+      ic -= nc;
+      ++jc;
+    }
   }
 }
 
