@@ -125,7 +125,7 @@ __device__ __forceinline__ void rounds_cloud(ParamsPtr params, const uint32_t gr
       if ((uint32_t)tid < np) {
         uint64_t idx = f.starts ? f.starts[s + tid] : a.start;
         if (idx >= f.n) {
-          atomicOr(f.status, kStatusBadStart);
+          rounds_fail(params, kStatusBadStart);
           idx = 0;
         }
 #pragma unroll
@@ -358,9 +358,9 @@ __device__ __forceinline__ void rounds_cloud(ParamsPtr params, const uint32_t gr
     // ---- 2. exchange --------------------------------------------------------
     uint32_t C = own;
     if (G > 1) {
-      if (!rounds_exchange<D, LIST>(f.xchg, f.spin_ticks, a.cap_wg, G, g, e, tid, wave, S, S.lk,
-                                    S.lc, S.ck, S.cc, C, U)) {
-        if (tid == 0) atomicOr(f.status, kStatusTimeout);
+      if (!rounds_exchange<D, LIST>(f.xchg, e == 1 ? a.form_ticks : f.spin_ticks, a.cap_wg, G, g,
+                                    e, tid, wave, S, S.lk, S.lc, S.ck, S.cc, C, U)) {
+        if (tid == 0) rounds_fail(params, kStatusTimeout);
         return;
       }
     } else {
@@ -380,7 +380,7 @@ __device__ __forceinline__ void rounds_cloud(ParamsPtr params, const uint32_t gr
       // comes within some 64 rounds; the count only guards the loop's end.
       np = 0;
       if (++idle > 1024) {
-        if (tid == 0) atomicOr(f.status, kStatusTimeout);
+        if (tid == 0) rounds_fail(params, kStatusTimeout);
         return;
       }
       if (C) {
@@ -547,15 +547,16 @@ __global__ void __launch_bounds__(kRoundsThreads) fps_rounds_jobs(RoundsJobs j) 
     const uint32_t slot = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_slot);
     if (slot >= j.members) return;
     const ParamsPtr p = (ParamsPtr)j.table + uniform_u32(j.member_job[slot]);
-    if (p->team > 1) {
-      // Wait for the team to form, so that exchange waits are short ones.
+    if (p->team > 1 && !j.one_slot) {
+      // Wait for the team to form, so that exchange waits are short ones.  (With a slot each, a
+      // team's workgroups start together, and the first exchange finds out.)
       if (threadIdx.x == 0) {
         atomicAdd(p->ready, 1u);
         const uint64_t deadline = now_ticks() + j.team_ticks;
         uint32_t here = 1;
         while (__hip_atomic_load(p->ready, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < p->team) {
           if (now_ticks() > deadline) {
-            atomicOr(p->fps.status, kStatusTimeout);
+            rounds_fail(p, kStatusTimeout);
             here = 0;
             break;
           }

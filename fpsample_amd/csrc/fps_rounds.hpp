@@ -26,6 +26,8 @@ struct RoundsParams {
   // counter of those that have claimed it, zeroed before the launch.
   uint32_t team, member_base;
   uint32_t *ready;
+  uint64_t form_ticks;    // bound on the wait of the first exchange
+  uint32_t *host_status;  // where not null, a host word that a failure is stored to as well
 };
 
 // Any dimension (fps_rounds_any.hip): candidates a round decides on; rest holds the points by

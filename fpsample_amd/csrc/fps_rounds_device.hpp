@@ -50,6 +50,13 @@ struct alignas(16) Rec {
   float c[D > 0 ? (D + 3) / 4 * 4 : 4];
 };
 
+// Reports a failure (one thread).
+__device__ __forceinline__ void rounds_fail(ParamsPtr a, uint32_t code) {
+  atomicOr(a->fps.status, code);
+  if (a->host_status)
+    __hip_atomic_store(a->host_status, code, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // Counters of a workgroup's rounds in LDS.
 struct RoundsCounts {
   uint32_t cnt[2];  // candidates of this workgroup, by round parity

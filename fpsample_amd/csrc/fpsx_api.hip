@@ -820,6 +820,8 @@ int launch_fps(Ctx &c, const Plan &p, const float *d_pts, size_t sp, size_t ld, 
     ra.team = p.grid;
     ra.member_base = 0;
     ra.ready = nullptr;
+    ra.form_ticks = a.spin_ticks;
+    ra.host_status = nullptr;
     if (!p.k->dim) {
       // The points by coordinate, n apart: in place when they lie so.
       ra.rest = d_pts;

@@ -2,6 +2,8 @@
 // (device tables + a captured HIP graph of its launch sequence) and its C ABI.
 #include <hip/hip_runtime.h>
 
+#include <hip/hip_ext.h>
+
 #include <algorithm>
 #include <cfloat>
 #include <cmath>
@@ -167,19 +169,37 @@ static double rounds_us(const JobSpec &s, uint32_t target, uint32_t team) {
   return rounds * (7.0 + (team > 1 ? 3.0 : 0.0) + 3.6 * (share > 0.25 ? share : 0.25));
 }
 
-// The smallest team (a power of two times `least`, at most `most`) that ends within x us.
-static uint32_t rounds_team(const JobSpec &s, uint32_t target, uint32_t least, uint32_t most,
-                            double x) {
-  uint32_t best = least;
-  double us = rounds_us(s, target, least);
-  for (uint32_t t = least * 2; us > x && t <= most; t *= 2) {
-    const double u = rounds_us(s, target, t);
-    if (u < us) {
-      us = u;
-      best = t;
-    }
+// The team sizes to choose from for one cloud: powers of two times the least, while each is
+// faster than the ones before, with their times.
+struct RoundsTeams {
+  uint32_t n = 0;
+  uint32_t team[9];
+  double us[9];
+  uint32_t smallest(double x) const {  // the first that ends within x us, or the fastest
+    uint32_t i = 0;
+    while (i + 1 < n && us[i] > x) ++i;
+    return i;
   }
-  return best;
+};
+
+static RoundsTeams rounds_teams(const JobSpec &s, uint32_t target, uint32_t least, uint32_t most) {
+  RoundsTeams r;
+  for (uint32_t t = least; r.n < 9 && (r.n == 0 || t <= most); t *= 2) {
+    const double u = rounds_us(s, target, t);
+    if (r.n && u >= r.us[r.n - 1]) continue;
+    r.team[r.n] = t;
+    r.us[r.n++] = u;
+  }
+  return r;
+}
+
+// The tables of a launch out of host memory, and the clearing of what it counts in.
+__global__ void stage_jobs(const uint64_t *tables, uint64_t *dst, size_t words, uint64_t *clear,
+                           size_t clear_words) {
+  const size_t step = (size_t)gridDim.x * blockDim.x;
+  const size_t i0 = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  for (size_t i = i0; i < words; i += step) dst[i] = tables[i];
+  for (size_t i = i0; i < clear_words; i += step) clear[i] = 0;
 }
 
 int RoundsRun::prepare(Ctx &c, int dim, const std::vector<JobSpec> &specs, const RoundsBases &b,
@@ -204,27 +224,32 @@ int RoundsRun::prepare(Ctx &c, int dim, const std::vector<JobSpec> &specs, const
   // Team sizes for the least time x in which all can end: every cloud gets the smallest team
   // that ends within x; teams hold their workgroups at once, and the clouds of one workgroup
   // share the rest (one-slot launches: every cloud holds its own).
-  const std::vector<uint32_t> least = team;
-  auto fits = [&](double x, std::vector<uint32_t> &t) {
+  std::vector<RoundsTeams> choice(n);
+  double lo = 0.0, hi = 1.0;
+  for (size_t i = 0; i < n; ++i) {
+    choice[i] = rounds_teams(specs[i], target[i], team[i], std::min(blocks[i], kMaxTeam));
+    hi = std::max(hi, choice[i].us[0]);
+  }
+  std::vector<double> us(n);
+  for (size_t i = 0; i < n; ++i) us[i] = choice[i].us[0];
+  for (int it = 0; it < 24; ++it) {
+    const double x = 0.5 * (lo + hi);
     uint64_t held = 0;
     double shared = 0.0;
     for (size_t i = 0; i < n; ++i) {
-      t[i] = rounds_team(specs[i], target[i], least[i], std::min(blocks[i], kMaxTeam), x);
-      if (t[i] > 1 || one_slot)
-        held += t[i];
+      const uint32_t t = choice[i].smallest(x);
+      if (choice[i].team[t] > 1 || one_slot)
+        held += choice[i].team[t];
       else
-        shared += rounds_us(specs[i], target[i], 1) / x;
+        shared += choice[i].us[t] / x;
     }
-    return held + (uint64_t)std::ceil(shared) <= gmax;
-  };
-  double lo = 0.0, hi = 1.0;
-  for (size_t i = 0; i < n; ++i) hi = std::max(hi, rounds_us(specs[i], target[i], least[i]));
-  std::vector<uint32_t> t(n);
-  for (int it = 0; it < 24; ++it) {
-    const double x = 0.5 * (lo + hi);
-    if (fits(x, t)) {
+    if (held + (uint64_t)std::ceil(shared) <= gmax) {
       hi = x;
-      team = t;
+      for (size_t i = 0; i < n; ++i) {
+        const uint32_t t = choice[i].smallest(x);
+        team[i] = choice[i].team[t];
+        us[i] = choice[i].us[t];
+      }
     } else {
       lo = x;
     }
@@ -235,7 +260,7 @@ int RoundsRun::prepare(Ctx &c, int dim, const std::vector<JobSpec> &specs, const
   std::stable_sort(order.begin(), order.end(), [&](size_t x, size_t y) {
     const bool tx = team[x] > 1, ty = team[y] > 1;
     if (tx != ty) return tx;
-    return rounds_us(specs[x], target[x], team[x]) > rounds_us(specs[y], target[y], team[y]);
+    return us[x] > us[y];
   });
   members = (uint32_t)total;
   if (one_slot && members > gmax)
@@ -256,9 +281,22 @@ int RoundsRun::prepare(Ctx &c, int dim, const std::vector<JobSpec> &specs, const
   shmem = rounds_shmem((uint32_t)dim, nbl);
   if (c.max_blocks(k, shmem) < (int)gmax) return fail(FPSX_ETOOBIG, "threshold rounds: LDS");
   HIP_TRY(d_clear.reserve(words * sizeof(uint64_t)));
-  host.assign(n * sizeof(RoundsParams) + members * sizeof(uint32_t), 0);
-  HIP_TRY(d_tables.reserve(host.size()));
-  RoundsParams *tab = (RoundsParams *)host.data();
+  table_words = (n * sizeof(RoundsParams) + members * sizeof(uint32_t) + 7) / 8;
+  HIP_TRY(d_tables.reserve(table_words * sizeof(uint64_t)));
+  if (one_slot) {
+    const size_t need = kPinnedHead + table_words * sizeof(uint64_t);
+    if (need > pinned_cap) {
+      if (pinned) (void)hipHostFree(pinned);
+      pinned = nullptr;
+      pinned_cap = 0;
+      HIP_TRY(hipHostMalloc((void **)&pinned, 2 * need, hipHostMallocDefault));
+      pinned_cap = 2 * need;
+    }
+    std::memset(pinned, 0, need);
+  } else {
+    host.assign(table_words * sizeof(uint64_t), 0);
+  }
+  RoundsParams *tab = (RoundsParams *)(one_slot ? pinned + kPinnedHead : host.data());
   uint32_t *slot = (uint32_t *)(tab + n);
   uint64_t *cl = (uint64_t *)d_clear.p;
   uint32_t at = 0;
@@ -268,7 +306,7 @@ int RoundsRun::prepare(Ctx &c, int dim, const std::vector<JobSpec> &specs, const
     RoundsParams &r = tab[o];
     r.fps.pts = b.pts + s.pt_off;
     r.fps.ld = s.ld;
-    r.fps.sp = 1;
+    r.fps.sp = s.sp;
     r.fps.n = s.n;
     r.fps.m = s.m;
     r.fps.n_starts = 1;
@@ -291,9 +329,12 @@ int RoundsRun::prepare(Ctx &c, int dim, const std::vector<JobSpec> &specs, const
     r.team = team[i];
     r.member_base = at;
     r.ready = (uint32_t *)(cl + 2) + o;
+    r.form_ticks = one_slot ? c.spin_ticks * 5 : c.spin_ticks;
+    r.host_status = one_slot ? (uint32_t *)pinned : nullptr;
     for (uint32_t q = 0; q < team[i]; ++q) slot[at++] = (uint32_t)o;
   }
-  HIP_TRY(hipMemcpy(d_tables.p, host.data(), host.size(), hipMemcpyHostToDevice));
+  if (!one_slot)
+    HIP_TRY(hipMemcpy(d_tables.p, host.data(), host.size(), hipMemcpyHostToDevice));
   jobs.table = (const RoundsParams *)d_tables.p;
   jobs.member_job = (const uint32_t *)(jobs.table + n);
   jobs.members = members;
@@ -303,10 +344,22 @@ int RoundsRun::prepare(Ctx &c, int dim, const std::vector<JobSpec> &specs, const
   return FPSX_OK;
 }
 
-int RoundsRun::enqueue(hipStream_t st) {
-  HIP_TRY(launch_fill_u64((uint64_t *)d_clear.p, clear_words, 0, st));
+int RoundsRun::enqueue(hipStream_t st, hipEvent_t begin, hipEvent_t end) {
+  if (jobs.one_slot) {
+    const size_t w = std::max(clear_words, table_words);
+    hipLaunchKernelGGL(stage_jobs, dim3((unsigned)std::min<size_t>(1024, (w + 255) / 256)),
+                       dim3(256), 0, st, (const uint64_t *)(pinned + kPinnedHead),
+                       (uint64_t *)d_tables.p, table_words, (uint64_t *)d_clear.p, clear_words);
+    HIP_TRY(hipGetLastError());
+  } else {
+    HIP_TRY(launch_fill_u64((uint64_t *)d_clear.p, clear_words, 0, st));
+  }
   void *args[] = {(void *)&jobs};
-  HIP_TRY(hipLaunchKernel(k->fn, dim3(grid), dim3(k->block), args, shmem, st));
+  if (end) {
+    HIP_TRY(hipExtLaunchKernel(k->fn, dim3(grid), dim3(k->block), args, shmem, st, begin, end, 0));
+  } else {
+    HIP_TRY(hipLaunchKernel(k->fn, dim3(grid), dim3(k->block), args, shmem, st));
+  }
   return FPSX_OK;
 }
 

@@ -16,6 +16,7 @@ struct JobSpec {
   uint64_t pt_off, ld, out_off, state_off, start;
   uint32_t n, m, s_begin, s_end;
   uint64_t sorted_off = 0, perm_off = 0;  // pruned kernel: the spatial order
+  uint64_t sp = 1;                        // threshold rounds: floats from point to point
 };
 
 // Team sizes (ceil(n / min(B * PPT, share_cap))), claim order (teams first,
@@ -76,16 +77,25 @@ struct RoundsRun {
   size_t shmem = 0, clear_words = 0;
   DevBuf d_tables, d_clear;  // job table and slots; status, claim and team counters, exchange
   RoundsJobs jobs;
-  std::vector<char> host;    // what d_tables holds
+  // The tables as built.  one_slot: pinned, with a status word before them that the kernel sets,
+  // and copied by the launch itself; no call waits for a copy in either direction.
+  std::vector<char> host;
+  char *pinned = nullptr;
+  size_t pinned_cap = 0, table_words = 0;
+  static constexpr size_t kPinnedHead = 64;
+  uint32_t host_status() const { return *(volatile uint32_t *)pinned; }
   uint32_t *status() const { return (uint32_t *)d_clear.p; }
-  // Upload tables for these clouds (host-synchronous).  one_slot: every member has a
-  // workgroup of its own, all co-resident, and base_team[i] is the least team of cloud i.
+  // Tables for these clouds (uploaded host-synchronously unless one_slot).  one_slot: every
+  // member has a workgroup of its own, all co-resident, and base_team[i] is the least team of
+  // cloud i; the run's last launch has ended.
   int prepare(Ctx &c, int dim, const std::vector<JobSpec> &specs, const RoundsBases &b,
               const std::vector<uint32_t> *base_team = nullptr);
-  int enqueue(hipStream_t st);  // graph-capturable
+  // (graph-capturable without events, which time the kernel alone and mark its end)
+  int enqueue(hipStream_t st, hipEvent_t begin = nullptr, hipEvent_t end = nullptr);
   ~RoundsRun() {
     d_tables.free();
     d_clear.free();
+    if (pinned) (void)hipHostFree(pinned);
   }
 };
 

@@ -111,7 +111,7 @@ size_t align_up(size_t v) { return (v + Arena::kAlign - 1) / Arena::kAlign * Are
 
 struct Request {
   uint64_t id = 0;
-  std::vector<float> soa;  // host copy of the cloud, SoA (dim x n)
+  std::vector<float> pts;  // host copy of the cloud: as given for the rounds, else dim x n
   uint32_t n = 0, m = 0, dim = 0;
   uint64_t start = 0;
   // device placement (byte offsets into the arena)
@@ -203,8 +203,8 @@ struct fpsx_server {
   // Ends a request that will not finish (caller holds mu; wakes no one).  Its
   // host copy is no longer read by any upload.
   void end_request(Request &r, int code, Clock::time_point now) {
-    r.soa.clear();
-    r.soa.shrink_to_fit();
+    r.pts.clear();
+    r.pts.shrink_to_fit();
     r.saved.clear();
     r.saved.shrink_to_fit();
     r.done = true;
@@ -307,11 +307,11 @@ int fpsx_server::step() {
       if (e != hipSuccess) return fail(FPSX_EHIP, std::string("restore: ") + hipGetErrorString(e));
       continue;
     }
-    hipError_t e = hipMemcpyAsync(base + r->pts_off, r->soa.data(), r->soa.size() * sizeof(float),
+    hipError_t e = hipMemcpyAsync(base + r->pts_off, r->pts.data(), r->pts.size() * sizeof(float),
                                   hipMemcpyHostToDevice, copy);
     if (e == hipSuccess && rounds) {
       // (sorted_off and perm_off together hold the 16-byte records)
-      const int rc = rounds_order((const float *)(base + r->pts_off), 1, r->n, r->n, r->dim,
+      const int rc = rounds_order((const float *)(base + r->pts_off), r->dim, 1, r->n, r->dim,
                                   (float4 *)(base + r->sorted_off), nullptr, *rorder, copy);
       if (rc) return rc;
     } else if (e == hipSuccess && pruned) {
@@ -367,14 +367,15 @@ int fpsx_server::step() {
           continue;
         }
         r->ready = true;
-        r->soa.clear();
-        r->soa.shrink_to_fit();
+        r->pts.clear();
+        r->pts.shrink_to_fit();
         r->saved.clear();
         r->saved.shrink_to_fit();
       }
       JobSpec s;
       s.pt_off = r->pts_off / sizeof(float);
-      s.ld = r->n;
+      s.ld = rounds ? 1 : r->n;
+      s.sp = rounds ? r->dim : 1;
       s.out_off = r->out_off / sizeof(uint64_t);
       s.state_off = r->state_off / sizeof(float);
       s.start = r->start;
@@ -456,12 +457,19 @@ int fpsx_server::step() {
                                   (uint64_t *)arena_base, (float *)arena_base);
   }
   if (rc) return rc;
-  hipError_t e = hipEventRecord(L.t0, compute);
-  if (e != hipSuccess) return fail(FPSX_EHIP, std::string("serve launch: ") + hipGetErrorString(e));
-  rc = rounds ? L.rounds.enqueue(compute) : L.run.enqueue(compute);
-  if (rc) return rc;
-  e = hipEventRecord(L.t1, compute);
-  if (e != hipSuccess) return fail(FPSX_EHIP, std::string("serve launch: ") + hipGetErrorString(e));
+  if (rounds) {
+    // The events ride on the kernel's own packet: recorded beside it they are packets of their
+    // own between one launch and the next (24 requests, 258 launches: 15.3 ms against 13.4).
+    rc = L.rounds.enqueue(compute, L.t0, L.t1);
+    if (rc) return rc;
+  } else {
+    hipError_t e = hipEventRecord(L.t0, compute);
+    if (e != hipSuccess) return fail(FPSX_EHIP, std::string("serve launch: ") + hipGetErrorString(e));
+    rc = L.run.enqueue(compute);
+    if (rc) return rc;
+    e = hipEventRecord(L.t1, compute);
+    if (e != hipSuccess) return fail(FPSX_EHIP, std::string("serve launch: ") + hipGetErrorString(e));
+  }
   L.reqs = in_launch;
   L.s_end.resize(specs.size());
   for (size_t i = 0; i < specs.size(); ++i) L.s_end[i] = specs[i].s_end;
@@ -479,9 +487,12 @@ int fpsx_server::finish(Launch &L) {
   L.busy = false;
   cur ^= 1;  // the other slot (if queued) is now the oldest
   uint32_t st = 0;
-  e = hipMemcpy(&st, rounds ? L.rounds.status() : (uint32_t *)L.run.d_status.p, sizeof(uint32_t),
-                hipMemcpyDeviceToHost);
-  if (e != hipSuccess) return fail(FPSX_EHIP, std::string("status: ") + hipGetErrorString(e));
+  if (rounds) {
+    st = L.rounds.host_status();
+  } else {
+    e = hipMemcpy(&st, L.run.d_status.p, sizeof(uint32_t), hipMemcpyDeviceToHost);
+    if (e != hipSuccess) return fail(FPSX_EHIP, std::string("status: ") + hipGetErrorString(e));
+  }
   if (st) return status_code(st);
   ++launches;
   // Retire the requests this launch finished.
@@ -658,9 +669,12 @@ FPSX_EXPORT int fpsx_server_submit_ex(fpsx_server *s, const float *points, size_
                                   " bytes of HBM, more than the whole budget");
   if (r->team > s->grid_cap || r->team > kMaxTeam || r->team > (uint32_t)s->k->block)
     return fail(FPSX_ETOOBIG, "cloud too large for the serving kernel's team limit");
-  r->soa.resize(n_points * dim);
-  for (size_t i = 0; i < n_points; ++i)
-    for (size_t d = 0; d < dim; ++d) r->soa[d * n_points + i] = points[i * dim + d];
+  r->pts.resize(n_points * dim);
+  if (s->rounds)
+    std::memcpy(r->pts.data(), points, n_points * dim * sizeof(float));
+  else
+    for (size_t i = 0; i < n_points; ++i)
+      for (size_t d = 0; d < dim; ++d) r->pts[d * n_points + i] = points[i * dim + d];
   r->priority = priority;
   r->t_submit = Clock::now();
   if (deadline_s > 0) {
