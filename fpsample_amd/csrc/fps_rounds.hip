@@ -375,7 +375,7 @@ __device__ __forceinline__ void rounds_cloud(ParamsPtr params, const uint32_t gr
     U = uniform_u64(U);
     C = (uint32_t)__builtin_amdgcn_readfirstlane((int)C);
     if (C > (uint32_t)LIST || C == 0) {
-      // No picks: a smaller step, or the exact bound and a larger one.  From an exact bound
+      // No picks: a smaller step, or the exact bound.  From an exact bound
       // every step has a candidate, and halving ends at the best point alone, so a pick
       // comes within some 64 rounds; the count only guards the loop's end.
       np = 0;
@@ -388,7 +388,6 @@ __device__ __forceinline__ void rounds_cloud(ParamsPtr params, const uint32_t gr
         step = ns < 1 ? 1 : ns;
       } else {
         T = U;
-        if (Tg != ~0ull) step = step < ((uint64_t)1 << 60) ? step << 1 : step;
       }
       Tg = T > step ? T - step : 0;
       lds_barrier();
@@ -445,6 +444,7 @@ __device__ __forceinline__ void rounds_cloud(ParamsPtr params, const uint32_t gr
     lds_barrier();
     const uint32_t *rows = (const uint32_t *)&S.low[0][0][0];
     if (wave == 0) settle_candidates<CAP>(rows, F, lane, S.acc);
+    if (wave == 1 && lane == 0) S.step = next_step(step, a.target, C);  // (in its shadow)
     lds_barrier();
     // The picks, in order.  A candidate whose first lowering pick leaves its key above the
     // bound raises the bound to that key, and a pick that does not lower itself ends the round:
@@ -518,7 +518,7 @@ __device__ __forceinline__ void rounds_cloud(ParamsPtr params, const uint32_t gr
     if (s + np == a.s_end && a.s_end < f.m && tid == 0)
       S.last = ((uint64_t)S.pv[np - 1] << 32) | S.pt[np - 1];
     idle = 0;
-    step = next_step(step, a.target, C);
+    step = uniform_u64(S.step);
     Tg = T > step ? T - step : 0;
   }
 }

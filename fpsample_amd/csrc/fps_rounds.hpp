@@ -58,9 +58,13 @@ constexpr uint32_t kRoundsReplicas = 4;    // copies of the headers
 inline uint32_t rounds_target(size_t m) {
   return m >= 16384 ? 224 : m >= 1280 ? 160 : m <= 512 ? 64 : (uint32_t)(m / 8);
 }
-// Candidates one workgroup may publish: the area stays small enough to clear.
+// Candidates one workgroup may publish: a round in which one has more is lost, which clustered
+// clouds do to small limits, and larger areas cost their clearing and the candidates' way (us a
+// run and rounds at 64 / 32 for up to 64 and more workgroups, at 128 / 64 and at 256 / 128: 2^24
+// lattice points, 2048 picks 3608 (220), 3321 (168), 3305 (147); 2^20 clustered points, 16384
+// picks 2035 (196), 1989 (181), 2027 (171); 2^22 / 4096 1999, 1983, 2040).
 inline uint32_t rounds_cap_wg(uint32_t grid) {
-  return grid <= 8 ? kRoundsCap : grid <= 64 ? 64 : 32;
+  return grid <= 8 ? kRoundsCap : grid <= 64 ? 128 : 64;
 }
 // Words between the arrays of a header's words: 2 KiB apart they lie on different memory
 // channels, which all workgroups' polls then share (64 workgroups, 50 K points: 9.1 us a round

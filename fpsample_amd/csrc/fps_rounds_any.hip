@@ -226,7 +226,7 @@ __global__ void __launch_bounds__(kRoundsThreads) fps_rounds_any(RoundsParams) {
     U = uniform_u64(U);
     C = (uint32_t)__builtin_amdgcn_readfirstlane((int)C);
     if (C > (uint32_t)LIST || C == 0) {
-      // No picks: a smaller step, or the exact bound and a larger one (see fps_rounds.hip).
+      // No picks: a smaller step, or the exact bound (see fps_rounds.hip).
       np = 0;
       if (++idle > 1024) {
         if (tid == 0) atomicOr(f.status, kStatusTimeout);
@@ -237,7 +237,6 @@ __global__ void __launch_bounds__(kRoundsThreads) fps_rounds_any(RoundsParams) {
         step = ns < 1 ? 1 : ns;
       } else {
         T = U;
-        if (Tg != ~0ull) step = step < ((uint64_t)1 << 60) ? step << 1 : step;
       }
       Tg = T > step ? T - step : 0;
       lds_barrier();
@@ -286,6 +285,7 @@ __global__ void __launch_bounds__(kRoundsThreads) fps_rounds_any(RoundsParams) {
     lds_barrier();
     const uint32_t *low = (const uint32_t *)&s_low[0][0][0];
     if (wave == 0) settle_candidates<CAP>(low, F, lane, s_acc);
+    if (wave == 1 && lane == 0) S.step = next_step(step, a.target, C);  // (in its shadow)
     lds_barrier();
     uint64_t key = 0, taken = 0;
     if ((uint32_t)wave < nc) {
@@ -345,7 +345,7 @@ __global__ void __launch_bounds__(kRoundsThreads) fps_rounds_any(RoundsParams) {
     lds_barrier();
     idle = 0;
     np = uniform_u32(S.np[par]);
-    step = next_step(step, a.target, C);
+    step = uniform_u64(S.step);
     Tg = T > step ? T - step : 0;
   }
 }
