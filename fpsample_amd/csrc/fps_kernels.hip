@@ -300,6 +300,14 @@ __global__ void __launch_bounds__(B) fps_stream(FpsParams a) {
 
 // Fill kernel: clears the exchange area / status and fills min-distances.
 // (A kernel rather than hipMemsetAsync so callers may capture it in graphs.)
+// What a launch starts from: its exchange area and its status word zero.  One launch for
+// both: with a second one 1024 points / 256 picks from host memory took 190 us against 170.
+__global__ void clear_launch(uint64_t *area, size_t n, uint64_t *status) {
+  const size_t step = (size_t)gridDim.x * blockDim.x;
+  const size_t i0 = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i0 == 0) *status = 0;
+  for (size_t i = i0; i < n; i += step) area[i] = 0;
+}
 __global__ void fill_u64(uint64_t *p, size_t n, uint64_t v) {
   for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += (size_t)gridDim.x * blockDim.x)
@@ -367,6 +375,11 @@ const KernelEntry *stream_table(size_t *count) {
   return kStream;
 }
 
+hipError_t launch_clear(uint64_t *area, size_t n, uint64_t *status, hipStream_t st) {
+  const unsigned blocks = (unsigned)max((size_t)1, min((size_t)1024, (n + 255) / 256));
+  hipLaunchKernelGGL(clear_launch, dim3(blocks), dim3(256), 0, st, area, n, status);
+  return hipGetLastError();
+}
 hipError_t launch_fill_u64(uint64_t *p, size_t n, uint64_t v, hipStream_t st) {
   if (n == 0) return hipSuccess;
   unsigned blocks = (unsigned)min((size_t)1024, (n + 255) / 256);

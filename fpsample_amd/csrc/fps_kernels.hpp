@@ -48,6 +48,7 @@ const KernelEntry *resident_table(size_t *count);
 const KernelEntry *stream_table(size_t *count);
 
 // Enqueue helpers; each returns the launch status.
+hipError_t launch_clear(uint64_t *area, size_t n, uint64_t *status, hipStream_t st);
 hipError_t launch_fill_u64(uint64_t *p, size_t n, uint64_t v, hipStream_t st);
 hipError_t launch_fill_f32(float *p, size_t n, float v, hipStream_t st);
 // acc[0] |= src[0] on the stream (one status word folded into another).

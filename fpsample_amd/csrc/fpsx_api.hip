@@ -724,8 +724,7 @@ static int common_params(Ctx &c, const float *d_pts, size_t sp, size_t ld, size_
   const size_t xwords = words ? words : xchg_words(reps);
   HIP_TRY(c.xchg.reserve(xwords * sizeof(uint64_t)));
   HIP_TRY(c.status.reserve(sizeof(uint64_t)));
-  HIP_TRY(launch_fill_u64((uint64_t *)c.xchg.p, xwords, 0, st));
-  HIP_TRY(launch_fill_u64((uint64_t *)c.status.p, 1, 0, st));
+  HIP_TRY(launch_clear((uint64_t *)c.xchg.p, xwords, (uint64_t *)c.status.p, st));
   std::memset(&a, 0, sizeof(a));
   a.pts = d_pts;
   a.ld = ld;
