@@ -20,13 +20,15 @@
 // of equal distances.
 //
 // What bounds it: a round's serial chain, not bytes (2^20 clustered points, 16384 picks, 128
-// workgroups: 206 rounds of 10.3 us).  Of a round (50 K points, 64 workgroups, 73 rounds of 9
-// us): update 2.2 us with the wait for the slowest wave, exchange 3.0, sorting 0.9, rows 1.4,
-// settling 0.4, the bound and the picks 0.6.  Settling the candidates one by one instead took
-// 450 ns a pick.  A block per wave in registers, the candidates loaded beside the headers and
-// the best 256 taken from up to 512 brought 2^20 clustered points from 2.67 to 2.13 ms, 100 K /
-// 50 K picks from 4.52 to 3.44 ms; jobs of half-waves in the sorting and the rows and one pass
-// for bound and picks, 50 K / 4096 picks from 668 to 654 us, 2^22 / 4096 picks 2.09 to 2.03 ms.
+// workgroups: 181 rounds of 11 us, the paired pass kernel 8203 exchanges of 3.4 us).  Of a
+// round (50 K points, 64 workgroups, 65 rounds of 9.7 us): update 2.2 us with the wait for the
+// slowest wave, exchange 3.0, sorting 0.9, rows 1.4, settling 0.4, the bound and the picks 0.6.
+// Settling the candidates one by one instead took 450 ns a pick.  A block per wave in
+// registers, the candidates loaded beside the headers and the best 256 taken from up to 512
+// brought 2^20 clustered points from 2.67 to 2.13 ms, 100 K / 50 K picks from 4.52 to 3.44 ms;
+// jobs of half-waves in the sorting and the rows and one pass for bound and picks, 50 K / 4096
+// picks from 668 to 654 us, 2^22 / 4096 picks 2.09 to 2.03 ms.  Deciding the candidates that a
+// cut leaves in a further pass saves one round in ten to five, and costs as much.
 #include "fps_rounds.hpp"
 
 #include "fps_device.hpp"

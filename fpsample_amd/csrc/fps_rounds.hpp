@@ -78,6 +78,12 @@ inline size_t rounds_xchg_words(uint32_t grid, uint32_t dim, uint32_t cap_wg) {
   return (size_t)2 * ((size_t)kRoundsReplicas * kRoundsHeadWords * rounds_head_pitch(grid) +
                       (size_t)(2 + dim) * grid * cap_wg);
 }
+// The largest single-cloud area: reserved at once, so that it never moves under a captured call.
+inline size_t rounds_xchg_most() {
+  const size_t a = rounds_xchg_words(kRoundsMaxGrid, 8, rounds_cap_wg(kRoundsMaxGrid));
+  const size_t b = rounds_xchg_words(64, 8, rounds_cap_wg(64));
+  return a > b ? a : b;
+}
 // Dynamic LDS of a workgroup holding nbl blocks: box and best key of each.
 inline size_t rounds_shmem(uint32_t dim, uint32_t nbl) {
   return (size_t)nbl * (2 * dim * sizeof(float) + sizeof(uint64_t));
@@ -95,6 +101,8 @@ RoundsOrderScratch *new_rounds_order_scratch();
 void delete_rounds_order_scratch(RoundsOrderScratch *s);
 // Sizes the scratch for clouds of up to n points, so that later calls allocate nothing.
 int rounds_order_reserve(RoundsOrderScratch &scratch, uint32_t n);
+// Whether a call for n points would allocate nothing.
+bool rounds_order_ready(const RoundsOrderScratch *scratch, uint32_t n);
 int rounds_order(const float *pts, uint64_t sp, uint64_t ld, uint32_t n, uint32_t dim, float4 *rec,
                  float *rest, RoundsOrderScratch &scratch, hipStream_t st);
 

@@ -9,7 +9,7 @@
 //
 // What bounds it: the vector ALUs, in the update (three operations per point, pick and
 // coordinate) and in the candidates' rows.  20000 points of 32 dimensions, 2000 picks: the
-// one-pick streaming kernel takes 5.2 us a pick.
+// one-pick streaming kernel takes 5.2 us a pick, this one 0.39 (49 rounds of 16 us).
 #include "fps_device.hpp"
 #include "fps_rounds.hpp"
 #include "fps_rounds_device.hpp"

@@ -361,6 +361,14 @@ int rounds_order_reserve(RoundsOrderScratch &S, uint32_t n) {
   return FPSX_OK;
 }
 
+bool rounds_order_ready(const RoundsOrderScratch *S, uint32_t n) {
+  if (n <= kChunk) return true;
+  const size_t buckets = (size_t)1 << bucket_bits(n);
+  return S && S->part.cap >= kBoxGroups * 6 * sizeof(float) &&
+         S->hist.cap >= buckets * (count_groups(n) + 1) * sizeof(uint32_t) &&
+         S->tmp.cap >= (size_t)n * sizeof(float4);
+}
+
 int rounds_order(const float *pts, uint64_t sp, uint64_t ld, uint32_t n, uint32_t dim, float4 *rec,
                  float *rest, RoundsOrderScratch &S, hipStream_t st) {
   const Cloud c = {pts, sp, ld, n, dim};

@@ -722,7 +722,8 @@ static int common_params(Ctx &c, const float *d_pts, size_t sp, size_t ld, size_
   if (c.backoff < 0) c.backoff = 0;
   const uint32_t reps = (uint32_t)c.replicas;
   const size_t xwords = words ? words : xchg_words(reps);
-  HIP_TRY(c.xchg.reserve(xwords * sizeof(uint64_t)));
+  HIP_TRY(c.xchg.reserve(std::max(std::max(xwords, xchg_words(kMaxReplicas)), rounds_xchg_most()) *
+                         sizeof(uint64_t)));
   HIP_TRY(c.status.reserve(sizeof(uint64_t)));
   HIP_TRY(launch_clear((uint64_t *)c.xchg.p, xwords, (uint64_t *)c.status.p, st));
   std::memset(&a, 0, sizeof(a));
@@ -777,6 +778,11 @@ static int dispatch(Ctx &c, const Plan &p, void *arg, hipStream_t st) {
   return FPSX_OK;
 }
 
+// Whether min-distances go to memory: more blocks than waves in a workgroup.
+static bool rounds_spill(const Plan &p) {
+  return p.k->dim && p.chunk > (uint32_t)(kRoundsThreads * p.k->ppt);
+}
+
 int launch_fps(Ctx &c, const Plan &p, const float *d_pts, size_t sp, size_t ld, size_t n,
                size_t dim, size_t m, const uint64_t *d_starts, size_t n_starts, uint64_t *d_out,
                float *d_out_pts, float init, hipStream_t st) {
@@ -801,7 +807,7 @@ int launch_fps(Ctx &c, const Plan &p, const float *d_pts, size_t sp, size_t ld, 
   if (rc) return rc;
   RoundsParams ra;
   if (p.kind == PlanKind::Rounds) {
-    if (p.k->dim) {
+    if (rounds_spill(p)) {
       HIP_TRY(c.dmin.reserve(n * sizeof(float)));
       a.dmin = (float *)c.dmin.p;
     }
@@ -913,6 +919,30 @@ int launch_npdu(Ctx &c, const Plan &p, const float *d_pts, size_t sp, size_t ld,
 static bool capturing(hipStream_t st) {
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   return hipStreamIsCapturing(st, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone;
+}
+
+// The plan of a call on `st`.  Under stream capture nothing can be allocated and a later call may
+// move what was: the resident pass kernels, which need no scratch of the cloud's size, stay in
+// front there, and the rounds run where an earlier call has left them all they need.
+static int plan_on_stream(Ctx &c, size_t sp, size_t ld, size_t n, size_t dim, int tie, size_t m,
+                          hipStream_t st, Plan &p) {
+  int rc = plan_call(c, n, dim, tie, m, p);
+  if (rc || p.kind != PlanKind::Rounds || !capturing(st)) return rc;
+  Plan q;
+  rc = plan(c, n, dim, tie, m, q);
+  if (rc) {
+    t_err.clear();
+    return FPSX_OK;
+  }
+  const bool soa = sp == 1 && ld == n;
+  const bool ready =
+      (!rounds_spill(p) || c.dmin.cap >= n * sizeof(float)) &&
+      (p.k->dim || soa || c.rest.cap >= n * dim * sizeof(float)) &&
+      (!p.order || (c.rec.cap >= n * sizeof(float4) &&
+                    (dim <= 3 || c.rest.cap >= n * (dim - 3) * sizeof(float)) &&
+                    c.order && rounds_order_ready(c.order, (uint32_t)n)));
+  if (q.kind == PlanKind::Resident || !ready) p = q;
+  return FPSX_OK;
 }
 
 int scratch_acquire(Ctx &c, hipStream_t st) {
@@ -1033,9 +1063,9 @@ FPSX_EXPORT int fpsx_fps_sampling_device_strided(const float *d_points, size_t s
   Ctx &c = *cp;
   std::lock_guard<std::mutex> lk(c.mu);
   Plan p;
-  rc = plan_call(c, n_points, dim, tie, n_samples, p);
-  if (rc) return rc;
   hipStream_t st = stream ? (hipStream_t)stream : c.stream;
+  rc = plan_on_stream(c, stride_point, stride_dim, n_points, dim, tie, n_samples, st, p);
+  if (rc) return rc;
   return launch_fps(c, p, d_points, stride_point, stride_dim, n_points, dim, n_samples, d_start,
                     n_start, d_out, d_out_points, init, st);
 }

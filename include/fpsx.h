@@ -102,7 +102,9 @@ int fpsx_plan_info(size_t n_points, size_t dim, int tie, size_t n_samples, int *
  * FPSX_NO_ROUNDS=1, or a tuned plan that is a pass kernel; FPSX_ROUNDS=
  * "P:G[:target[:order]]" sets their shape (points per lane, workgroups,
  * candidates aimed at per round, spatial order 0 or 1) and takes them at any
- * size.  The picks are the same either way.
+ * size.  The picks are the same either way.  Under stream capture a cloud that
+ * the resident pass kernels hold keeps them, and the rounds run where an earlier
+ * call of that size has left the buffers they need.
  */
 int fpsx_call_info(size_t n_points, size_t dim, int tie, size_t n_samples, int *kind, int *block,
                    int *ppt, int *grid, int *chunk);
@@ -326,7 +328,8 @@ int fpsx_fps_batch(const float *points, size_t dim, const uint64_t *offsets, siz
  *     while others run join at the next launch; uploads overlap the kernel);
  *   - retires finished requests and wakes their waiters.
  * Each request's picks equal fpsx_fps_sampling on its cloud alone.
- * block/ppt select the batch-kernel shape (0, 0: 1024 x 16).
+ * block/ppt 0, 0: the threshold rounds (FPSX_NO_ROUNDS=1: the batch kernel at
+ * 1024 x 16); else the batch kernel of that shape.
  * fpsx_server_submit returns FPSX_EBUDGET for a request larger than the whole
  * budget.  fpsx_server_wait blocks until the request is done, copies its
  * picks and its latency (submit to completion, seconds).  Destroy drains.

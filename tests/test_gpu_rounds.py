@@ -144,3 +144,40 @@ def test_rounds_order_sizes(gpu, rounds_env, n):
     odd[6] = -np.inf
     for name, pc in (("tight", tight), ("line", line), ("odd", odd)):
         check(pc, 400, 9, name)
+
+
+@pytest.mark.parametrize("n,d,m", [(1000, 3, 250), (20_001, 3, 700), (70_001, 6, 300),
+                                   (3001, 20, 200)])
+def test_rounds_under_capture(gpu, n, d, m):
+    # A call captured after one that left its buffers, replayed on new points each time.
+    import torch
+
+    from fpsample_amd import device as D
+
+    log(f"capture n={n} d={d} m={m}")
+    rng = np.random.default_rng(66)
+    pts = torch.zeros((n, d), dtype=torch.float32, device="cuda")
+    start = torch.zeros(1, dtype=torch.int64, device="cuda")
+    out = torch.zeros(m, dtype=torch.int64, device="cuda")
+
+    def call(stream):
+        D.fps_sampling_device_strided(pts.data_ptr(), d, 1, n, d, m, start.data_ptr(), 1,
+                                      out.data_ptr(), stream=stream)
+
+    side = torch.cuda.Stream()
+    pts.copy_(torch.from_numpy(rng.random((n, d), dtype=np.float32)))
+    torch.cuda.synchronize()
+    call(side.cuda_stream)
+    side.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        call(torch.cuda.current_stream().cuda_stream)
+    for rep in range(3):
+        pc = rng.random((n, d), dtype=np.float32)
+        pts.copy_(torch.from_numpy(pc))
+        out.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(out.cpu().numpy().astype(np.uint64), O.fps(pc, m, 0),
+                                      err_msg=f"replay {rep}")
