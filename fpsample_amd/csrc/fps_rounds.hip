@@ -94,7 +94,7 @@ __device__ __forceinline__ void rounds_cloud(ParamsPtr params, const uint32_t gr
     const uint32_t *carry = params->carry;
     T = uniform_u64(((uint64_t)carry[0] << 32) | carry[1]);
     step = uniform_u64(((uint64_t)carry[2] << 32) | carry[3]);
-    Tg = T > step ? T - step : 0;
+    Tg = round_bound(T, step);
   }
   uint32_t e = 0;        // rounds
   uint32_t idle = 0;     // rounds since the last pick
@@ -377,21 +377,19 @@ __device__ __forceinline__ void rounds_cloud(ParamsPtr params, const uint32_t gr
     U = uniform_u64(U);
     C = (uint32_t)__builtin_amdgcn_readfirstlane((int)C);
     if (C > (uint32_t)LIST || C == 0) {
-      // No picks: a smaller step, or the exact bound.  From an exact bound
-      // every step has a candidate, and halving ends at the best point alone, so a pick
-      // comes within some 64 rounds; the count only guards the loop's end.
+      // No picks: a smaller step, or the exact bound, so that a pick comes within some 64
+      // rounds; the count only guards the loop's end.
       np = 0;
       if (++idle > 1024) {
         if (tid == 0) rounds_fail(params, kStatusTimeout);
         return;
       }
       if (C) {
-        const uint64_t ns = (uint64_t)((double)step * sqrt((double)a.target / (double)C));
-        step = ns < 1 ? 1 : ns;
+        step = less_step(step, a.target, C);
       } else {
         T = U;
       }
-      Tg = T > step ? T - step : 0;
+      Tg = round_bound(T, step);
       lds_barrier();
       continue;
     }
@@ -521,7 +519,7 @@ __device__ __forceinline__ void rounds_cloud(ParamsPtr params, const uint32_t gr
       S.last = ((uint64_t)S.pv[np - 1] << 32) | S.pt[np - 1];
     idle = 0;
     step = uniform_u64(S.step);
-    Tg = T > step ? T - step : 0;
+    Tg = round_bound(T, step);
   }
 }
 

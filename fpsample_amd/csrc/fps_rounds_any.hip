@@ -233,12 +233,11 @@ __global__ void __launch_bounds__(kRoundsThreads) fps_rounds_any(RoundsParams) {
         return;
       }
       if (C) {
-        const uint64_t ns = (uint64_t)((double)step * sqrt((double)a.target / (double)C));
-        step = ns < 1 ? 1 : ns;
+        step = less_step(step, a.target, C);
       } else {
         T = U;
       }
-      Tg = T > step ? T - step : 0;
+      Tg = round_bound(T, step);
       lds_barrier();
       continue;
     }
@@ -346,7 +345,7 @@ __global__ void __launch_bounds__(kRoundsThreads) fps_rounds_any(RoundsParams) {
     idle = 0;
     np = uniform_u32(S.np[par]);
     step = uniform_u64(S.step);
-    Tg = T > step ? T - step : 0;
+    Tg = round_bound(T, step);
   }
 }
 

@@ -2,13 +2,10 @@
 #pragma once
 #include "fps_device.hpp"
 #include "fps_rounds.hpp"
+#include "fps_rounds_bound.hpp"
 
 namespace fpsx {
 
-// A point's key: (min-distance, index) in 64 bits, larger first; 0 is below every point.
-__device__ __forceinline__ uint64_t make_key(int value_bits, uint32_t tie) {
-  return ((uint64_t)((uint32_t)value_bits + 1u) << 32) | tie;
-}
 template <int TIE>
 __device__ __forceinline__ uint32_t tie_of(uint32_t idx) {
   return TIE == kTieHighest ? idx : ~idx;
@@ -306,17 +303,6 @@ __device__ __forceinline__ void settle_candidates(const uint32_t *rows, uint32_t
     }
     if (lane == 0) out[c] = acc[c];
   }
-}
-
-// The step after a round of C candidates: the square root damps it against the count's noise,
-// and it at most doubles, since a round with too many candidates for the list is lost (2^20
-// clustered points, 16384 picks: 205 rounds and 2118 us where it could grow fourfold and doubled
-// after a round without candidates too, 196 and 2035 so).
-__device__ __forceinline__ uint64_t next_step(uint64_t step, uint32_t target, uint32_t C) {
-  double r = sqrt((double)target / (double)C);
-  r = r > 2.0 ? 2.0 : r;
-  const double ns = (double)step * r;
-  return ns < 1.0 ? 1 : (ns > 4.0e18 ? (uint64_t)1 << 61 : (uint64_t)ns);
 }
 
 }  // namespace fpsx
