@@ -4,6 +4,8 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include <vector>
+
 #include "fps_kernels.hpp"
 
 namespace fpsx {
@@ -105,5 +107,17 @@ int rounds_order_reserve(RoundsOrderScratch &scratch, uint32_t n);
 bool rounds_order_ready(const RoundsOrderScratch *scratch, uint32_t n);
 int rounds_order(const float *pts, uint64_t sp, uint64_t ld, uint32_t n, uint32_t dim, float4 *rec,
                  float *rest, RoundsOrderScratch &scratch, hipStream_t st);
+// Many clouds in one launch and without scratch: every 8192 consecutive points of a cloud, one
+// job of a device table, are ordered among themselves.
+struct RoundsOrderJob {
+  const float *pts;
+  uint64_t sp, ld;
+  float4 *rec;
+  float *rest;
+  uint32_t n, dim, base;
+};
+void rounds_order_pieces(const float *pts, uint64_t sp, uint64_t ld, uint32_t n, uint32_t dim,
+                         float4 *rec, float *rest, std::vector<RoundsOrderJob> &jobs);
+hipError_t launch_order_pieces(const RoundsOrderJob *jobs, uint32_t count, hipStream_t st);
 
 }  // namespace fpsx

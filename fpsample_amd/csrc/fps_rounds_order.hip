@@ -231,16 +231,15 @@ __global__ void __launch_bounds__(kThreads)
   }
 }
 
-// Counting sort of the kChunk records from blockIdx.x * kChunk on (in: already in buckets;
-// null: the cloud itself, whose box is then found here) along the curve.
-__global__ void __launch_bounds__(kThreads)
-    order_chunk(Cloud c, const float *part, uint32_t groups, const float4 *in, float4 *out,
-                float *rest) {
+// Counting sort of the kChunk records from base on (in: already in buckets; null: the cloud
+// itself, in the box of these points) along the curve.
+__device__ __forceinline__ void chunk_order(const Cloud &c, const uint32_t base, const float *part,
+                                            uint32_t groups, const float4 *in, float4 *out,
+                                            float *rest) {
   __shared__ float s[kThreads / 64][6];
   __shared__ uint32_t s_sum[kThreads / 64];
   __shared__ uint32_t s_n[kBins];
   __shared__ uint32_t s_lo, s_hi;
-  const uint32_t base = blockIdx.x * kChunk;
   const uint32_t count = min(kChunk, c.n - base);
   float4 r[kPer];
 #pragma unroll
@@ -329,6 +328,18 @@ __global__ void __launch_bounds__(kThreads)
   }
 }
 
+__global__ void __launch_bounds__(kThreads)
+    order_chunk(Cloud c, const float *part, uint32_t groups, const float4 *in, float4 *out,
+                float *rest) {
+  chunk_order(c, blockIdx.x * kChunk, part, groups, in, out, rest);
+}
+
+__global__ void __launch_bounds__(kThreads) order_pieces(const RoundsOrderJob *jobs) {
+  const RoundsOrderJob j = jobs[blockIdx.x];
+  const Cloud c = {j.pts, j.sp, j.ld, j.n, j.dim};
+  chunk_order(c, j.base, nullptr, 0, nullptr, j.rec, j.rest);
+}
+
 }  // namespace
 
 #define HIP_OR_FAIL(expr)                                              \
@@ -404,6 +415,17 @@ int rounds_order(const float *pts, uint64_t sp, uint64_t ld, uint32_t n, uint32_
                      (const float4 *)S.tmp.p, rec, rest);
   HIP_OR_FAIL(hipGetLastError());
   return FPSX_OK;
+}
+
+void rounds_order_pieces(const float *pts, uint64_t sp, uint64_t ld, uint32_t n, uint32_t dim,
+                         float4 *rec, float *rest, std::vector<RoundsOrderJob> &jobs) {
+  for (uint64_t base = 0; base < n; base += kChunk)
+    jobs.push_back({pts, sp, ld, rec, rest, n, dim, (uint32_t)base});
+}
+
+hipError_t launch_order_pieces(const RoundsOrderJob *jobs, uint32_t count, hipStream_t st) {
+  hipLaunchKernelGGL(order_pieces, dim3(count), dim3(kThreads), 0, st, jobs);
+  return hipGetLastError();
 }
 
 }  // namespace fpsx

@@ -387,6 +387,8 @@ struct fpsx_batch {
   RoundsRun rounds;
   bool use_rounds = false;
   DevBuf rec, rest, state;
+  DevBuf d_order;  // but for 3-D: the pieces that every run puts in spatial order
+  uint32_t order_jobs = 0;
   RoundsOrderScratch *rorder = nullptr;
   bool fallback = false;  // no batch kernel for this dimension or cloud size: one launch per cloud
   std::vector<JobSpec> specs;
@@ -452,8 +454,13 @@ static int batch_order(fpsx_batch *b, uint32_t block) {
   return FPSX_OK;
 }
 
-// The threshold rounds for this batch: order every cloud, build the tables.  ETOOBIG where
+// The threshold rounds for this batch: order its clouds, build the tables.  ETOOBIG where
 // some cloud is beyond a team of the pass kernels too.  Caller holds the context lock.
+//   3-D clouds are put in spatial order here, as for the pruned kernels.  For other dimensions
+//   nothing reads the caller's points before a run does, at its place in the stream: each run
+//   orders them anew, in one launch and so in pieces of 8192 (batch_enqueue).  Two dimensions,
+//   us a run so, without any order, and with a whole order made here: 48 clouds of 1024 to 16384
+//   points 661, 853 and 636; 16 of 20 K to 200 K 2152, 4308 and 1678.
 static int batch_prepare_rounds(fpsx_batch *b) {
   Ctx &c = *b->ctx;
   const uint64_t total = b->offsets.back();
@@ -464,31 +471,46 @@ static int batch_prepare_rounds(fpsx_batch *b) {
   HIP_TRY(b->rec.reserve(total * sizeof(float4)));
   if (more) HIP_TRY(b->rest.reserve(total * more * sizeof(float)));
   // (n + 4 floats a cloud, 16-byte aligned)
-  std::vector<uint64_t> state(b->n_clouds);
+  std::vector<JobSpec> specs = b->specs;
   uint64_t at = 0;
   for (size_t i = 0; i < b->n_clouds; ++i) {
-    state[i] = at;
-    at += ((uint64_t)b->specs[i].n + 7) / 4 * 4;
+    specs[i].sorted_off = 4 * b->offsets[i];
+    specs[i].perm_off = more * b->offsets[i];
+    specs[i].state_off = at;
+    at += ((uint64_t)specs[i].n + 7) / 4 * 4;
   }
   HIP_TRY(b->state.reserve(at * sizeof(float)));
-  if (!b->rorder) b->rorder = new_rounds_order_scratch();
-  int rc = rounds_order_reserve(*b->rorder, nmax);
-  if (rc) return rc;
-  std::vector<JobSpec> specs = b->specs;
-  for (size_t i = 0; i < b->n_clouds; ++i) {
-    JobSpec &s = specs[i];
-    s.sorted_off = 4 * b->offsets[i];
-    s.perm_off = more * b->offsets[i];
-    s.state_off = state[i];
-    rc = rounds_order(b->d_pts + s.pt_off, 1, b->ld, s.n, (uint32_t)b->dim,
-                      (float4 *)b->rec.p + b->offsets[i],
-                      more ? (float *)b->rest.p + s.perm_off : nullptr, *b->rorder, c.stream);
+  int rc = FPSX_OK;
+  if (b->dim == 3) {
+    if (!b->rorder) b->rorder = new_rounds_order_scratch();
+    rc = rounds_order_reserve(*b->rorder, nmax);
+    for (size_t i = 0; i < b->n_clouds && !rc; ++i)
+      rc = rounds_order(b->d_pts + specs[i].pt_off, 1, b->ld, specs[i].n, 3,
+                        (float4 *)b->rec.p + b->offsets[i], nullptr, *b->rorder, c.stream);
     if (rc) return rc;
+    HIP_TRY(hipStreamSynchronize(c.stream));
+  } else {
+    std::vector<RoundsOrderJob> jobs;
+    for (size_t i = 0; i < b->n_clouds; ++i)
+      rounds_order_pieces(b->d_pts + specs[i].pt_off, 1, b->ld, specs[i].n, (uint32_t)b->dim,
+                          (float4 *)b->rec.p + b->offsets[i],
+                          more ? (float *)b->rest.p + specs[i].perm_off : nullptr, jobs);
+    b->order_jobs = (uint32_t)jobs.size();
+    HIP_TRY(b->d_order.reserve(jobs.size() * sizeof(RoundsOrderJob)));
+    HIP_TRY(hipMemcpy(b->d_order.p, jobs.data(), jobs.size() * sizeof(RoundsOrderJob),
+                      hipMemcpyHostToDevice));
   }
-  HIP_TRY(hipStreamSynchronize(c.stream));
   const RoundsBases bases = {b->d_pts, b->d_out, (float *)b->state.p, (const float *)b->rec.p,
                              (const float *)b->rest.p};
   return b->rounds.prepare(c, b->dim, specs, bases);
+}
+
+// One run's launches (graph-capturable).
+static int batch_enqueue(fpsx_batch *b, hipStream_t st) {
+  if (!b->use_rounds) return b->run.enqueue(st);
+  if (b->order_jobs)
+    HIP_TRY(launch_order_pieces((const RoundsOrderJob *)b->d_order.p, b->order_jobs, st));
+  return b->rounds.enqueue(st);
 }
 
 static int batch_prepare_kernel(fpsx_batch *b, const KernelEntry *k, bool pruned) {
@@ -561,7 +583,8 @@ FPSX_EXPORT int fpsx_batch_create(const float *d_points, size_t ld, size_t dim,
     HIP_TRY(hipEventCreate(&e0));
     HIP_TRY(hipEventCreate(&e1));
     HIP_TRY(hipEventRecord(e0, c.stream));
-    rc = b->rounds.enqueue(c.stream);
+    b->use_rounds = true;
+    rc = batch_enqueue(b.get(), c.stream);
     if (rc) return rc;
     HIP_TRY(hipEventRecord(e1, c.stream));
     HIP_TRY(hipEventSynchronize(e1));
@@ -664,7 +687,7 @@ FPSX_EXPORT int fpsx_batch_create(const float *d_points, size_t ld, size_t dim,
   if (flags & FPSX_BATCH_GRAPH) {
     HIP_TRY(hipStreamCreateWithFlags(&b->capture_stream, hipStreamNonBlocking));
     HIP_TRY(hipStreamBeginCapture(b->capture_stream, hipStreamCaptureModeThreadLocal));
-    rc = b->use_rounds ? b->rounds.enqueue(b->capture_stream) : b->run.enqueue(b->capture_stream);
+    rc = batch_enqueue(b.get(), b->capture_stream);
     hipGraph_t g = nullptr;
     hipError_t e = hipStreamEndCapture(b->capture_stream, &g);
     if (rc) return rc;
@@ -712,7 +735,7 @@ FPSX_EXPORT int fpsx_batch_run(fpsx_batch *b, void *stream) {
     HIP_TRY(hipGraphLaunch(b->exec, st));
     return FPSX_OK;
   }
-  return b->use_rounds ? b->rounds.enqueue(st) : b->run.enqueue(st);
+  return batch_enqueue(b, st);
 }
 
 FPSX_EXPORT int fpsx_batch_status(fpsx_batch *b, void *stream) {
@@ -748,6 +771,7 @@ FPSX_EXPORT void fpsx_batch_destroy(fpsx_batch *b) {
   b->sorted.free();
   b->perm.free();
   b->rec.free();
+  b->d_order.free();
   b->rest.free();
   b->state.free();
   delete_rounds_order_scratch(b->rorder);

@@ -299,6 +299,9 @@ int fpsx_npdu_plan_info(size_t n_points, size_t dim, int *kernel_dim, int *block
  *   FPSX_BATCH_GRAPH     capture the launch sequence in a HIP graph, replayed by run
  *   FPSX_BATCH_AUTOTUNE  time every batch-kernel shape once at creation, keep the fastest
  * Clouds of a dimension with no batch kernel run one launch per cloud.
+ * A 3-D batch is put in spatial order at creation: d_points holds the clouds
+ * by then and is not changed afterwards.  In other dimensions every run reads
+ * d_points anew, in stream order, and creation does not read it.
  * Clouds that need several workgroups settle up to two picks per exchange
  * (same picks); FPSX_BATCH_NO_PAIR=1, read at creation, keeps one per exchange.
  */
