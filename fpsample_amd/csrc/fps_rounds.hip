@@ -541,6 +541,7 @@ __global__ void __launch_bounds__(kRoundsThreads) fps_rounds_jobs(RoundsJobs j) 
   extern __shared__ uint64_t s_dyn[];
   __shared__ RoundsLds<D> S;
   __shared__ uint32_t s_slot;
+  __shared__ uint32_t s_here;  // (a word of its own: waves read s_slot while it is written)
   for (;;) {
     if (threadIdx.x == 0) s_slot = j.one_slot ? blockIdx.x : atomicAdd(j.claim, 1u);
     __syncthreads();
@@ -553,19 +554,18 @@ __global__ void __launch_bounds__(kRoundsThreads) fps_rounds_jobs(RoundsJobs j) 
       if (threadIdx.x == 0) {
         atomicAdd(p->ready, 1u);
         const uint64_t deadline = now_ticks() + j.team_ticks;
-        uint32_t here = 1;
+        s_here = 1;
         while (__hip_atomic_load(p->ready, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < p->team) {
           if (now_ticks() > deadline) {
             rounds_fail(p, kStatusTimeout);
-            here = 0;
+            s_here = 0;
             break;
           }
           __builtin_amdgcn_s_sleep(1);
         }
-        s_slot = here;
       }
       __syncthreads();
-      if (!__builtin_amdgcn_readfirstlane((int)s_slot)) return;
+      if (!__builtin_amdgcn_readfirstlane((int)s_here)) return;
     }
     rounds_cloud<D, P, kTieHighest>(p, uniform_u32(slot - p->member_base), p->team, S, s_dyn);
     if (j.one_slot) return;

@@ -1,0 +1,29 @@
+"""GPU tests of the threshold rounds over many clouds in one launch (fps_rounds_jobs)."""
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def test_teams_and_a_queue_of_clouds(gpu):
+    # More members than workgroups: some workgroups form teams, which wait for each other, and
+    # go on to clouds of their own afterwards.
+    from fpsample_amd.batch import DeviceBatch
+
+    rng = np.random.default_rng(20)
+    sizes = [50_000] * 12 + [9000] * 30 + [int(n) for n in rng.integers(1, 900, 500)]
+    clouds = [rng.random((n, 3)).astype(np.float32) for n in sizes]
+    ms = [max(1, n // 8) for n in sizes]
+    b = DeviceBatch(clouds, ms, [0] * len(sizes))
+    info = b.info()
+    print(f"queue: {info}", flush=True)
+    assert info["ppt"] == 4 and info["members"] > info["grid"] and info["members"] > len(sizes)
+    want = [O.fps(pc, m, 0) for pc, m in zip(clouds, ms)]
+    for rep in range(3):
+        b.run()
+        b.status()
+        for i, (g, w) in enumerate(zip(b.picks(), want)):
+            np.testing.assert_array_equal(g, w, err_msg=f"run {rep} cloud {i} n={sizes[i]}")
+    b.close()
