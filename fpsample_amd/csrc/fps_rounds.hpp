@@ -101,6 +101,7 @@ const KernelEntry *rounds_jobs_kernel(int dim);
 struct RoundsOrderScratch;
 RoundsOrderScratch *new_rounds_order_scratch();
 void delete_rounds_order_scratch(RoundsOrderScratch *s);
+void hold_rounds_order_scratch(RoundsOrderScratch *s);
 // Sizes the scratch for clouds of up to n points, so that later calls allocate nothing.
 int rounds_order_reserve(RoundsOrderScratch &scratch, uint32_t n);
 // Whether a call for n points would allocate nothing.

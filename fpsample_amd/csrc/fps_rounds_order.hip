@@ -38,6 +38,11 @@ void delete_rounds_order_scratch(RoundsOrderScratch *S) {
   delete S;
 }
 
+void hold_rounds_order_scratch(RoundsOrderScratch *S) {
+  if (!S) return;
+  for (DevBuf *b : {&S->part, &S->hist, &S->tmp}) b->held = b->p != nullptr;
+}
+
 namespace {
 
 constexpr int kThreads = 1024;

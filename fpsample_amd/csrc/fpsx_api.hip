@@ -54,15 +54,33 @@ static int hip_fail(hipError_t e, const char *what) {
 
 hipError_t DevBuf::reserve(size_t bytes) {
   if (bytes <= cap) return hipSuccess;
-  if (p) {
+  const size_t least = bytes < 4096 ? 4096 : bytes;
+  size_t want = least;
+  if (held) {
+    // Graphs replay on this memory, so it is left to them.  At least twice as much is taken
+    // where it is to be had: all that is left behind then stays below the buffer's size.
+    want = std::max(least, 2 * cap);
+  } else if (p) {
     hipError_t e = hipFree(p);
-    p = nullptr;
-    cap = 0;
-    if (e != hipSuccess) return e;
+    if (e != hipSuccess) {
+      p = nullptr;
+      cap = 0;
+      return e;
+    }
   }
-  size_t want = bytes < 4096 ? 4096 : bytes;
+  p = nullptr;
+  cap = 0;
+  held = false;
   hipError_t e = hipMalloc(&p, want);
-  if (e == hipSuccess) cap = want;
+  if (e == hipErrorOutOfMemory && want > least) {
+    (void)hipGetLastError();  // (dealt with here)
+    want = least;
+    e = hipMalloc(&p, want);
+  }
+  if (e == hipSuccess)
+    cap = want;
+  else
+    p = nullptr;
   return e;
 }
 
@@ -70,6 +88,7 @@ void DevBuf::free() {
   if (p) (void)hipFree(p);  // release path: nothing to report to
   p = nullptr;
   cap = 0;
+  held = false;
 }
 
 DevBuf::~DevBuf() {
@@ -123,6 +142,13 @@ int Ctx::max_blocks(const KernelEntry *k, size_t shmem) {
   int total = nb * cus;
   occ[key] = total;
   return total;
+}
+
+void Ctx::hold_scratch() {
+  for (DevBuf *b : {&pts, &starts, &xchg, &status, &dmin, &sorted, &perm, &rec, &rest})
+    b->held = b->p != nullptr;
+  hold_spatial_scratch(spatial);
+  hold_rounds_order_scratch(order);
 }
 
 // ---------------------------------------------------------------------------
@@ -921,9 +947,9 @@ static bool capturing(hipStream_t st) {
   return hipStreamIsCapturing(st, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone;
 }
 
-// The plan of a call on `st`.  Under stream capture nothing can be allocated and a later call may
-// move what was: the resident pass kernels, which need no scratch of the cloud's size, stay in
-// front there, and the rounds run where an earlier call has left them all they need.
+// The plan of a call on `st`.  Under stream capture nothing can be allocated: the resident pass
+// kernels, which need no scratch of the cloud's size, stay in front there, and the rounds run
+// where an earlier call has left them all they need (which then stays, Ctx::hold_scratch).
 static int plan_on_stream(Ctx &c, size_t sp, size_t ld, size_t n, size_t dim, int tie, size_t m,
                           hipStream_t st, Plan &p) {
   int rc = plan_call(c, n, dim, tie, m, p);
@@ -952,7 +978,10 @@ int scratch_acquire(Ctx &c, hipStream_t st) {
 }
 
 int scratch_release(Ctx &c, hipStream_t st) {
-  if (capturing(st)) return FPSX_OK;
+  if (capturing(st)) {
+    c.hold_scratch();
+    return FPSX_OK;
+  }
   if (!c.scratch_ev) HIP_TRY(hipEventCreateWithFlags(&c.scratch_ev, hipEventDisableTiming));
   HIP_TRY(hipEventRecord(c.scratch_ev, st));
   c.scratch_owner = st;

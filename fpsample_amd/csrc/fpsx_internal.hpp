@@ -22,6 +22,7 @@ namespace fpsx {
 struct DevBuf {
   void *p = nullptr;
   size_t cap = 0;
+  bool held = false;  // a captured launch refers to this memory: it stays when the buffer grows
   hipError_t reserve(size_t bytes);
   void free();
   ~DevBuf();
@@ -58,6 +59,7 @@ struct Ctx {
   struct SpatialScratch *spatial = nullptr;
   DevBuf rec, rest;  // threshold rounds: the points in spatial order
   struct RoundsOrderScratch *order = nullptr;
+  void hold_scratch();  // a captured launch refers to the buffers above
   std::map<std::pair<const void *, size_t>, int> occ;  // co-resident workgroups per kernel
   int max_blocks(const KernelEntry *k, size_t shmem);
   // Autotuned plans: (n_points, dim, tie) -> the plan the tuner chose.
@@ -175,6 +177,7 @@ int scratch_release(Ctx &c, hipStream_t st);
 struct SpatialScratch *new_spatial_scratch();
 // Frees the scratch's device buffers (owners with a shorter life than the process).
 void delete_spatial_scratch(struct SpatialScratch *s);
+void hold_spatial_scratch(struct SpatialScratch *s);
 int fps_host(const float *points, size_t n, size_t dim, int layout, size_t m,
              const uint64_t *starts, size_t n_starts, uint64_t *out, int tie, float init);
 

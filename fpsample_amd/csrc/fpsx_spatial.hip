@@ -37,6 +37,13 @@ void delete_spatial_scratch(SpatialScratch *S) {
   delete S;
 }
 
+void hold_spatial_scratch(SpatialScratch *S) {
+  if (!S) return;
+  for (DevBuf *b : {&S->part, &S->box, &S->keys, &S->vals, &S->keys_alt, &S->vals_alt, &S->keys64,
+                    &S->keys64_alt, &S->tmp})
+    b->held = b->p != nullptr;
+}
+
 namespace {
 
 constexpr int kBoxThreads = 256;

@@ -104,7 +104,8 @@ int fpsx_plan_info(size_t n_points, size_t dim, int tie, size_t n_samples, int *
  * candidates aimed at per round, spatial order 0 or 1) and takes them at any
  * size.  The picks are the same either way.  Under stream capture a cloud that
  * the resident pass kernels hold keeps them, and the rounds run where an earlier
- * call of that size has left the buffers they need.
+ * call of that size has left the buffers they need; these then stay where they
+ * are, for the graph's replays, when later calls need larger ones.
  */
 int fpsx_call_info(size_t n_points, size_t dim, int tie, size_t n_samples, int *kind, int *block,
                    int *ppt, int *grid, int *chunk);
