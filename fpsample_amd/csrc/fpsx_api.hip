@@ -507,6 +507,12 @@ static bool env_set(const char *name) {
   return v && *v && std::strcmp(v, "0") != 0;
 }
 
+// Whether a pass plan is asked for by name or by the tuner.
+static bool passes_asked(Ctx &c, size_t n, size_t dim, int tie) {
+  return env_set("FPSX_PLAN") || env_set("FPSX_NO_PAIR") || env_set("FPSX_NO_PRUNE") ||
+         env_set("FPSX_NO_ROUNDS") || c.tuned.find(std::make_tuple(n, dim, tie)) != c.tuned.end();
+}
+
 // Threshold rounds from 512 points and 192 picks (64 beyond three dimensions), unless a pass
 // plan is asked for by name or by the tuner: the first picks come one or two a round, at 5 to
 // 10 us, where a pass takes 0.6 to 3 us.  Passes against rounds, us a call: 512 points / 128
@@ -515,11 +521,8 @@ static bool env_set(const char *name) {
 // and 686; eight dimensions, 4096 / 64 106 and 120, 65536 / 64 207 and 165, 2^20 / 64 456
 // and 251.
 int plan_call(Ctx &c, size_t n, size_t dim, int tie, size_t m, Plan &p) {
-  const bool passes = env_set("FPSX_PLAN") || env_set("FPSX_NO_PAIR") || env_set("FPSX_NO_PRUNE") ||
-                      env_set("FPSX_NO_ROUNDS") ||
-                      c.tuned.find(std::make_tuple(n, dim, tie)) != c.tuned.end();
   const bool serves = n >= 512 && m >= (dim <= 3 ? 192u : 64u);
-  if (!passes && (env_set("FPSX_ROUNDS") || serves) &&
+  if (!passes_asked(c, n, dim, tie) && (env_set("FPSX_ROUNDS") || serves) &&
       plan_rounds(c, n, dim, tie, m, p) == FPSX_OK)
     return FPSX_OK;
   t_err.clear();
@@ -947,28 +950,47 @@ static bool capturing(hipStream_t st) {
   return hipStreamIsCapturing(st, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone;
 }
 
-// The plan of a call on `st`.  Under stream capture nothing can be allocated: the resident pass
-// kernels, which need no scratch of the cloud's size, stay in front there, and the rounds run
-// where an earlier call has left them all they need (which then stays, Ctx::hold_scratch).
+// Whether a launch of this plan allocates nothing and records kernels alone.  Never one with the
+// library's sort: it may clear its counters by a memory fill, and graphs with such fills have gone
+// wrong on replays after the first (an order with indices beyond the cloud is a memory fault).
+static bool capturable(Ctx &c, const Plan &p, size_t sp, size_t ld, size_t n, size_t dim) {
+  const size_t word = sizeof(float);
+  if (p.kind == PlanKind::Resident) return true;
+  if (p.kind == PlanKind::Stream)
+    return c.dmin.cap >= n * word && (sp == 1 || c.pts.cap >= n * dim * word);
+  if (p.kind != PlanKind::Rounds) return false;
+  if (rounds_spill(p) && c.dmin.cap < n * word) return false;
+  if (!p.k->dim) return (sp == 1 && ld == n) || c.rest.cap >= n * dim * word;
+  return !p.order || (c.rec.cap >= n * sizeof(float4) &&
+                      (dim <= 3 || c.rest.cap >= n * (dim - 3) * word) && c.order &&
+                      rounds_order_ready(c.order, (uint32_t)n));
+}
+
+// The plan of a call on `st`.  Under stream capture nothing can be allocated: a cloud whose pass
+// plan is a resident one, which needs no scratch of the cloud's size, keeps it.  Else it is the
+// first of these that an earlier call has left all it needs (which then stays, Ctx::hold_scratch):
+// what the call would run, the rounds without a spatial order, any resident kernel; and else the
+// streaming one.
 static int plan_on_stream(Ctx &c, size_t sp, size_t ld, size_t n, size_t dim, int tie, size_t m,
                           hipStream_t st, Plan &p) {
   int rc = plan_call(c, n, dim, tie, m, p);
-  if (rc || p.kind != PlanKind::Rounds || !capturing(st)) return rc;
+  if (rc || p.kind == PlanKind::Resident || !capturing(st)) return rc;
   Plan q;
-  rc = plan(c, n, dim, tie, m, q);
-  if (rc) {
-    t_err.clear();
+  const bool passes = plan(c, n, dim, tie, m, q) == FPSX_OK;
+  t_err.clear();
+  if (passes && q.kind == PlanKind::Resident) {
+    p = q;
     return FPSX_OK;
   }
-  const bool soa = sp == 1 && ld == n;
-  const bool ready =
-      (!rounds_spill(p) || c.dmin.cap >= n * sizeof(float)) &&
-      (p.k->dim || soa || c.rest.cap >= n * dim * sizeof(float)) &&
-      (!p.order || (c.rec.cap >= n * sizeof(float4) &&
-                    (dim <= 3 || c.rest.cap >= n * (dim - 3) * sizeof(float)) &&
-                    c.order && rounds_order_ready(c.order, (uint32_t)n)));
-  if (q.kind == PlanKind::Resident || !ready) p = q;
-  return FPSX_OK;
+  if (capturable(c, p, sp, ld, n, dim)) return FPSX_OK;
+  if (!passes_asked(c, n, dim, tie) && plan_rounds(c, n, dim, tie, m, p) == FPSX_OK) {
+    p.order = false;
+    if (capturable(c, p, sp, ld, n, dim)) return FPSX_OK;
+  }
+  t_err.clear();
+  if (plan_resident_only(n, dim, tie, [&](const KernelEntry *k) { return c.max_blocks(k, 0); }, p))
+    return FPSX_OK;
+  return plan_stream(c, n, dim, tie, 1024, 0, false, p);
 }
 
 int scratch_acquire(Ctx &c, hipStream_t st) {

@@ -103,9 +103,10 @@ int fpsx_plan_info(size_t n_points, size_t dim, int tie, size_t n_samples, int *
  * "P:G[:target[:order]]" sets their shape (points per lane, workgroups,
  * candidates aimed at per round, spatial order 0 or 1) and takes them at any
  * size.  The picks are the same either way.  Under stream capture a cloud that
- * the resident pass kernels hold keeps them, and the rounds run where an earlier
- * call of that size has left the buffers they need; these then stay where they
- * are, for the graph's replays, when later calls need larger ones.
+ * the resident pass kernels hold keeps them; else the rounds run, in spatial
+ * order or not, by the buffers that an earlier call of that size has left, and a
+ * plan that sorts is never captured.  Buffers that a graph refers to stay where
+ * they are when later calls need larger ones.
  */
 int fpsx_call_info(size_t n_points, size_t dim, int tie, size_t n_samples, int *kind, int *block,
                    int *ppt, int *grid, int *chunk);
