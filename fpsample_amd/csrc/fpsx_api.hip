@@ -274,7 +274,7 @@ static int plan_resident_shape(Ctx &c, size_t n, const KernelEntry *k, Plan &p,
 
 static int plan_from_tuned(Ctx &c, size_t n, size_t dim, int tie, Plan &p) {
   auto it = c.tuned.find(std::make_tuple(n, dim, tie));
-  if (it == c.tuned.end()) return -1;
+  if (it == c.tuned.end() || it->second.kind == PlanKind::Rounds) return -1;
   p = it->second;
   return FPSX_OK;
 }
@@ -438,6 +438,7 @@ int plan(Ctx &c, size_t n, size_t dim, int tie, size_t m, Plan &p) {
 //   473, 265, 236 and 243 at 1, 8, 16 and 32; 8192 / 2048 528, 464, 460 and 466 at 8, 16, 32
 //   and 64; gauss1m 2.53, 2.13 and 2.20 ms at 64, 128 and 256; the 16.7 M-point lattice 4.94
 //   and 4.09 ms at 128 and 256 (early rounds sweep the whole cloud).
+//   P0 and G0, where not 0, are a tuned shape; target and order always follow the call's picks.
 //   target: a round costs about 6 us and 20 ns a candidate, so long runs take more per round:
 //   100 K / 50 K picks 4.05, 3.58, 3.39, 3.23 and 3.20 ms at 128, 160, 192, 224 and 256;
 //   gauss1m 2.13 and 2.08 at 160 and 224; 50 K / 4096 picks 0.69, 0.66, 0.69 and 0.72 at 128,
@@ -446,8 +447,9 @@ int plan(Ctx &c, size_t n, size_t dim, int tie, size_t m, Plan &p) {
 //   once most picks reach few blocks.  Call with and without it, us: 2048 / 512 picks 219 and
 //   214; 4096 / 1024 327 and 352; 8192 / 2048 460 and 533; 65536 / 256 367 and 334; 50 K /
 //   4096 716 and 1008; 2^20 / 256 777 and 712; gauss1m / 16384 2160 and 7746.
-static int plan_rounds(Ctx &c, size_t n, size_t dim, int tie, size_t m, Plan &p) {
-  int P = 0, G = 0, target = 0, order = -1;
+static int plan_rounds(Ctx &c, size_t n, size_t dim, int tie, size_t m, Plan &p, int P0 = 0,
+                       int G0 = 0) {
+  int P = P0, G = G0, target = 0, order = -1;
   if (const char *env = std::getenv("FPSX_ROUNDS"))
     if (*env) std::sscanf(env, "%d:%d:%d:%d", &P, &G, &target, &order);
   if (dim > 8) {
@@ -507,10 +509,19 @@ static bool env_set(const char *name) {
   return v && *v && std::strcmp(v, "0") != 0;
 }
 
-// Whether a pass plan is asked for by name or by the tuner.
-static bool passes_asked(Ctx &c, size_t n, size_t dim, int tie) {
+// Whether a pass plan is asked for by name; by name or by the tuner.
+static bool passes_named() {
   return env_set("FPSX_PLAN") || env_set("FPSX_NO_PAIR") || env_set("FPSX_NO_PRUNE") ||
-         env_set("FPSX_NO_ROUNDS") || c.tuned.find(std::make_tuple(n, dim, tie)) != c.tuned.end();
+         env_set("FPSX_NO_ROUNDS");
+}
+static bool passes_asked(Ctx &c, size_t n, size_t dim, int tie) {
+  Plan p;
+  return passes_named() || plan_from_tuned(c, n, dim, tie, p) == FPSX_OK;
+}
+// The rounds' shape that the tuner chose for clouds of this size, or null.
+static const Plan *tuned_rounds(Ctx &c, size_t n, size_t dim, int tie) {
+  auto it = c.tuned.find(std::make_tuple(n, dim, tie));
+  return it != c.tuned.end() && it->second.kind == PlanKind::Rounds ? &it->second : nullptr;
 }
 
 // Threshold rounds from 512 points and 192 picks (64 beyond three dimensions), unless a pass
@@ -521,9 +532,11 @@ static bool passes_asked(Ctx &c, size_t n, size_t dim, int tie) {
 // and 686; eight dimensions, 4096 / 64 106 and 120, 65536 / 64 207 and 165, 2^20 / 64 456
 // and 251.
 int plan_call(Ctx &c, size_t n, size_t dim, int tie, size_t m, Plan &p) {
+  const Plan *shape = tuned_rounds(c, n, dim, tie);
   const bool serves = n >= 512 && m >= (dim <= 3 ? 192u : 64u);
-  if (!passes_asked(c, n, dim, tie) && (env_set("FPSX_ROUNDS") || serves) &&
-      plan_rounds(c, n, dim, tie, m, p) == FPSX_OK)
+  if (!passes_asked(c, n, dim, tie) && (env_set("FPSX_ROUNDS") || serves || shape) &&
+      plan_rounds(c, n, dim, tie, m, p, shape ? shape->k->ppt : 0,
+                  shape ? (int)shape->grid : 0) == FPSX_OK)
     return FPSX_OK;
   t_err.clear();
   return plan(c, n, dim, tie, m, p);
@@ -691,7 +704,7 @@ static std::vector<Plan> candidates(Ctx &c, size_t n, size_t dim, int tie, size_
   std::vector<Plan> out;
   Plan q;
   if (plan(c, n, dim, tie, m, q) == FPSX_OK) out.push_back(q);
-  if (plan_rounds(c, n, dim, tie, m, q) == FPSX_OK) out.push_back(q);
+  if (!passes_named() && plan_rounds(c, n, dim, tie, m, q) == FPSX_OK) out.push_back(q);
   q = Plan();
   size_t cnt;
   const KernelEntry *t = resident_table(&cnt);
@@ -1279,6 +1292,7 @@ static int report_plan(bool call, size_t n_points, size_t dim, int tie, size_t n
   Ctx &c = *cp;
   std::lock_guard<std::mutex> lk(c.mu);
   Plan p;
+  call = call || (tuned_rounds(c, n_points, dim, tie) && !passes_named());
   rc = call ? plan_call(c, n_points, dim, tie, n_samples, p)
             : plan(c, n_points, dim, tie, n_samples, p);
   if (rc) return rc;

@@ -73,7 +73,7 @@ void *fpsx_stream(void);
 /*
  * The pass kernel the planner picks for a cloud of n_points x dim and n_samples
  * picks under `tie` (what a call runs when it does not take the threshold
- * rounds, see fpsx_call_info): kind 0 = register-resident, 1 = HBM-streaming,
+ * rounds, see fpsx_call_info; a tuned plan is reported as it is): kind 0 = register-resident, 1 = HBM-streaming,
  * 2 = register-resident with spatial order and per-wave pruning,
  * 4 = HBM-streaming with spatial order and per-block pruning,
  * 5 = kind 2 settling up to two picks per cross-workgroup exchange (2..256
@@ -114,12 +114,14 @@ int fpsx_call_info(size_t n_points, size_t dim, int tie, size_t n_samples, int *
 /*
  * Autotuner: times every feasible plan for `passes` passes (0: 256; pass the
  * number of samples later calls will draw) on the given device cloud -- the
- * planner's own choice, every resident shape (threads per workgroup, points
+ * planner's own choice, the threshold rounds unless pass kernels are asked for
+ * by name, every resident shape (threads per workgroup, points
  * per thread, workgroups), for 3-D clouds every pruned and paired shape and
  * the streaming pruned plan, and the streaming kernel -- and keeps, among the
  * plans within 3% of the fastest, the one with the fewest workgroups, for
  * clouds of exactly this (n_points, dim, tie) on the current device; later
- * calls use it whatever their sample count.  The chosen shape is returned
+ * calls use it whatever their sample count (of threshold rounds the shape, what
+ * else they depend on follows the call's).  The chosen shape is returned
  * through the optional pointers (fpsx_plan_info reports its kind).  Without
  * tuning the planner uses its per-pass time model.
  */
