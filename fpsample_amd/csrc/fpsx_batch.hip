@@ -572,7 +572,7 @@ FPSX_EXPORT int fpsx_batch_create(const float *d_points, size_t ld, size_t dim,
     const char *v = std::getenv(name);
     if (v && *v && std::strcmp(v, "0") != 0) rounds = false;
   }
-  float rounds_ms = 0.0f;
+  float rounds_ms = 1e30f;
   if (rounds) {
     rc = batch_prepare_rounds(b.get());
     if (rc != FPSX_OK && rc != FPSX_ETOOBIG) return rc;
@@ -588,9 +588,12 @@ FPSX_EXPORT int fpsx_batch_create(const float *d_points, size_t ld, size_t dim,
     if (rc) return rc;
     HIP_TRY(hipEventRecord(e1, c.stream));
     HIP_TRY(hipEventSynchronize(e1));
-    HIP_TRY(hipEventElapsedTime(&rounds_ms, e0, e1));
+    float ms = 0.0f;
+    HIP_TRY(hipEventElapsedTime(&ms, e0, e1));
     (void)hipEventDestroy(e0);  // timing events only
     (void)hipEventDestroy(e1);
+    HIP_TRY(hipMemcpy(c.host_status, b->rounds.status(), sizeof(uint32_t), hipMemcpyDeviceToHost));
+    if (*c.host_status == 0) rounds_ms = ms;  // a run that gave up is not fast
   }
   if (dim == 3 && !(plain && plain[0] == '1')) {
     for (int ppt : {8, 16, 4}) {
@@ -623,7 +626,7 @@ FPSX_EXPORT int fpsx_batch_create(const float *d_points, size_t ld, size_t dim,
     hipEvent_t e0, e1;
     HIP_TRY(hipEventCreate(&e0));
     HIP_TRY(hipEventCreate(&e1));
-    float best = rounds ? rounds_ms : 1e30f;
+    float best = rounds_ms;
     for (const Cand &cd : cands) {
       const KernelEntry *k = cd.k;
       if (batch_prepare_kernel(b.get(), k, cd.pruned) != FPSX_OK) continue;

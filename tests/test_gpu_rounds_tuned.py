@@ -55,3 +55,25 @@ def test_tuner_leaves_the_rounds_out_when_asked(gpu, monkeypatch):
     D.autotune(soa, 1, n, n, d, passes=64)
     monkeypatch.delenv("FPSX_NO_ROUNDS")
     assert D.call_info(n, d, n_samples=500)["kind"] != "rounds"  # the tuned plan serves
+
+
+def test_batch_tuner_skips_rounds_that_gave_up(gpu):
+    # Exchanges that may not wait at all: the rounds' teams give up at once, which is fast; clouds
+    # that one workgroup holds need no exchange in the pass kernels.
+    from fpsample_amd import device as D
+    from fpsample_amd.batch import DeviceBatch
+
+    rng = np.random.default_rng(16)
+    clouds = [rng.random((16_000, 3)).astype(np.float32) for _ in range(2)]
+    ms = [2000, 1500]
+    D.exchange_timeout(1e-9)
+    try:
+        b = DeviceBatch(clouds, ms, [0, 0], autotune=True)
+    finally:
+        D.exchange_timeout(0)
+    print(f"tuned batch: {b.info()}", flush=True)
+    b.run()
+    b.status()
+    for i, (g, pc, m) in enumerate(zip(b.picks(), clouds, ms)):
+        np.testing.assert_array_equal(g, O.fps(pc, m, 0), err_msg=f"cloud {i}")
+    b.close()
