@@ -398,6 +398,7 @@ struct fpsx_batch {
   hipStream_t capture_stream = nullptr;
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
+  void *status_word() const { return use_rounds ? rounds.d_clear.p : run.d_status.p; }
 };
 
 static int validate_batch(const uint64_t *offsets, size_t n_clouds, const uint64_t *n_samples,
@@ -687,6 +688,9 @@ FPSX_EXPORT int fpsx_batch_create(const float *d_points, size_t ld, size_t dim,
     return FPSX_OK;
   }
   if (rc) return rc;
+  // The status until the first run.
+  const uint32_t ok = 0;
+  HIP_TRY(hipMemcpy(b->status_word(), &ok, sizeof(ok), hipMemcpyHostToDevice));
   if (flags & FPSX_BATCH_GRAPH) {
     HIP_TRY(hipStreamCreateWithFlags(&b->capture_stream, hipStreamNonBlocking));
     HIP_TRY(hipStreamBeginCapture(b->capture_stream, hipStreamCaptureModeThreadLocal));
@@ -747,9 +751,8 @@ FPSX_EXPORT int fpsx_batch_status(fpsx_batch *b, void *stream) {
   std::lock_guard<std::mutex> lk(c.mu);
   hipStream_t st = stream ? (hipStream_t)stream : c.stream;
   HIP_TRY(hipStreamSynchronize(st));
-  const void *word = b->use_rounds ? b->rounds.d_clear.p : b->run.d_status.p;
-  if (!word) return FPSX_OK;  // never run
-  HIP_TRY(hipMemcpy(c.host_status, word, sizeof(uint32_t), hipMemcpyDeviceToHost));
+  if (!b->status_word()) return FPSX_OK;  // never run
+  HIP_TRY(hipMemcpy(c.host_status, b->status_word(), sizeof(uint32_t), hipMemcpyDeviceToHost));
   return status_code(*c.host_status);
 }
 

@@ -27,3 +27,23 @@ def test_teams_and_a_queue_of_clouds(gpu):
         for i, (g, w) in enumerate(zip(b.picks(), want)):
             np.testing.assert_array_equal(g, w, err_msg=f"run {rep} cloud {i} n={sizes[i]}")
     b.close()
+
+
+@pytest.mark.parametrize("d", [2, 3])
+@pytest.mark.parametrize("passes", [False, True], ids=["rounds", "passes"])
+def test_status_before_the_first_run(gpu, monkeypatch, d, passes):
+    # On memory that held other values before: a batch that has not run has not failed.
+    from fpsample_amd import device as D
+    from fpsample_amd.batch import DeviceBatch
+
+    if passes:
+        monkeypatch.setenv("FPSX_NO_ROUNDS", "1")
+    rng = np.random.default_rng(21)
+    clouds = [rng.random((n, d)).astype(np.float32) for n in (5000, 300)]
+    for size in (4096, 16_384, 65_536, 1 << 18, 1 << 20, 1 << 22):
+        filled = [D.DeviceArray.from_numpy(np.full(size, 255, np.uint8)) for _ in range(4)]
+        for a in filled:
+            a.free()
+        b = DeviceBatch(clouds, [500, 100], [0, 0], graph=False)
+        b.status()
+        b.close()
