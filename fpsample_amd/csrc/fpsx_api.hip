@@ -73,10 +73,10 @@ hipError_t DevBuf::reserve(size_t bytes) {
   held = false;
   hipError_t e = hipMalloc(&p, want);
   if (e == hipErrorOutOfMemory && want > least) {
-    (void)hipGetLastError();  // (dealt with here)
     want = least;
     e = hipMalloc(&p, want);
   }
+  if (e == hipErrorOutOfMemory) (void)hipGetLastError();  // reported here, not by a later launch
   if (e == hipSuccess)
     cap = want;
   else
@@ -825,6 +825,14 @@ static bool rounds_spill(const Plan &p) {
   return p.k->dim && p.chunk > (uint32_t)(kRoundsThreads * p.k->ppt);
 }
 
+// Memory for the spatial order of a cloud.
+static int reserve_order(Ctx &c, size_t n, size_t dim) {
+  HIP_TRY(c.rec.reserve(n * sizeof(float4)));
+  if (dim > 3) HIP_TRY(c.rest.reserve(n * (dim - 3) * sizeof(float)));
+  if (!c.order) c.order = new_rounds_order_scratch();
+  return rounds_order_reserve(*c.order, (uint32_t)n);
+}
+
 int launch_fps(Ctx &c, const Plan &p, const float *d_pts, size_t sp, size_t ld, size_t n,
                size_t dim, size_t m, const uint64_t *d_starts, size_t n_starts, uint64_t *d_out,
                float *d_out_pts, float init, hipStream_t st) {
@@ -879,10 +887,16 @@ int launch_fps(Ctx &c, const Plan &p, const float *d_pts, size_t sp, size_t ld, 
         ra.rest = (const float *)c.rest.p;
       }
     }
-    if (p.order) {
-      HIP_TRY(c.rec.reserve(n * sizeof(float4)));
-      if (dim > 3) HIP_TRY(c.rest.reserve(n * (dim - 3) * sizeof(float)));
-      if (!c.order) c.order = new_rounds_order_scratch();
+    bool order = p.order;
+    if (order) {
+      // (without the memory for an order the points are taken as they lie)
+      rc = reserve_order(c, n, dim);
+      if (rc == FPSX_ENOMEM)
+        order = false;
+      else if (rc)
+        return rc;
+    }
+    if (order) {
       rc = rounds_order(d_pts, sp, ld, (uint32_t)n, (uint32_t)dim, (float4 *)c.rec.p,
                         (float *)c.rest.p, *c.order, st);
       if (rc) return rc;

@@ -398,6 +398,13 @@ struct fpsx_batch {
   hipStream_t capture_stream = nullptr;
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
+  // What the rounds took, where they do not serve.
+  void drop_rounds() {
+    for (DevBuf *m : {&rec, &rest, &state, &d_order, &rounds.d_tables, &rounds.d_clear}) m->free();
+    delete_rounds_order_scratch(rorder);
+    rorder = nullptr;
+    order_jobs = 0;
+  }
   void *status_word() const { return use_rounds ? rounds.d_clear.p : run.d_status.p; }
 };
 
@@ -543,7 +550,10 @@ FPSX_EXPORT int fpsx_batch_create(const float *d_points, size_t ld, size_t dim,
   *out = nullptr;
   if (dim == 0) return fail(FPSX_EBADDIM, "dim must be >= 1");
   if (!d_points || !d_out) return fail(FPSX_EINVAL, "null pointer argument");
-  std::unique_ptr<fpsx_batch> b(new fpsx_batch());
+  struct Destroy {
+    void operator()(fpsx_batch *p) const { fpsx_batch_destroy(p); }
+  };
+  std::unique_ptr<fpsx_batch, Destroy> b(new fpsx_batch());
   int rc = validate_batch(offsets, n_clouds, n_samples, start_idx, ld, b->specs);
   if (rc) return rc;
   if (ld < offsets[n_clouds]) return fail(FPSX_EINVAL, "ld must be >= the total point count");
@@ -576,8 +586,9 @@ FPSX_EXPORT int fpsx_batch_create(const float *d_points, size_t ld, size_t dim,
   float rounds_ms = 1e30f;
   if (rounds) {
     rc = batch_prepare_rounds(b.get());
-    if (rc != FPSX_OK && rc != FPSX_ETOOBIG) return rc;
+    if (rc != FPSX_OK && rc != FPSX_ETOOBIG && rc != FPSX_ENOMEM) return rc;
     rounds = rc == FPSX_OK;
+    if (!rounds) b->drop_rounds();
   }
   if (rounds && (flags & FPSX_BATCH_AUTOTUNE)) {
     hipEvent_t e0, e1;
@@ -776,11 +787,7 @@ FPSX_EXPORT void fpsx_batch_destroy(fpsx_batch *b) {
   if (b->capture_stream) (void)hipStreamDestroy(b->capture_stream);
   b->sorted.free();
   b->perm.free();
-  b->rec.free();
-  b->d_order.free();
-  b->rest.free();
-  b->state.free();
-  delete_rounds_order_scratch(b->rorder);
+  b->drop_rounds();
   delete_spatial_scratch(b->spatial);
   delete b;
 }
