@@ -94,7 +94,7 @@ __global__ void __launch_bounds__(kRoundsThreads) fps_rounds_any(RoundsParams) {
   uint32_t s = 0, np = 0;
   uint64_t T = ~0ull, Tg = ~0ull;
   uint64_t step = (uint64_t)1 << 51;
-  uint32_t e = 0, idle = 0;
+  uint32_t e = 0, empty = 0;
 
   // Coordinates of the point with tie word t into row r, by one wave.
   auto fetch = [&](uint32_t r, uint32_t t) {
@@ -113,7 +113,7 @@ __global__ void __launch_bounds__(kRoundsThreads) fps_rounds_any(RoundsParams) {
     s = uniform_u32(s);
     np = uniform_u32(np);
     e = uniform_u32(e);
-    idle = uniform_u32(idle);
+    empty = uniform_u32(empty);
     T = uniform_u64(T);
     Tg = uniform_u64(Tg);
     step = uniform_u64(step);
@@ -226,19 +226,27 @@ __global__ void __launch_bounds__(kRoundsThreads) fps_rounds_any(RoundsParams) {
     U = uniform_u64(U);
     C = (uint32_t)__builtin_amdgcn_readfirstlane((int)C);
     if (C > (uint32_t)LIST || C == 0) {
-      // No picks: a smaller step, or the exact bound (see fps_rounds.hip).
-      np = 0;
-      if (++idle > 1024) {
-        if (tid == 0) atomicOr(f.status, kStatusTimeout);
-        return;
+      // Too many candidates, or none: the best point of all is the pick (see fps_rounds.hip).
+      if (wave == 0) {
+        fetch(0, (uint32_t)U);
+        bool own = true;  // (a coordinate without a distance to itself leaves the point as it is)
+        for (uint32_t j = lane; j < dim; j += 64) own = own && rows[j] - rows[j] == 0.0f;
+        if (lane == 0) {
+          s_pp[0] = 0;
+          s_pt[0] = (uint32_t)U;
+        }
+        if (__ballot(!own) || !(0.0f < __int_as_float((int)(uint32_t)(U >> 32) - 1)))
+          if (lane == 0) S.stuck = 1;
       }
-      if (C) {
+      np = 1;
+      if (C)
         step = less_step(step, a.target, C);
-      } else {
-        T = U;
-      }
+      else if (empty)
+        step = next_step(step, a.target, 1);
+      empty = C == 0;
+      T = U;
       Tg = round_bound(T, step);
-      lds_barrier();
+      __syncthreads();
       continue;
     }
 
@@ -342,7 +350,7 @@ __global__ void __launch_bounds__(kRoundsThreads) fps_rounds_any(RoundsParams) {
       }
     }
     lds_barrier();
-    idle = 0;
+    empty = 0;
     np = uniform_u32(S.np[par]);
     step = uniform_u64(S.step);
     Tg = round_bound(T, step);

@@ -32,7 +32,7 @@ FPSX_BOUND uint64_t round_bound(uint64_t T, uint64_t step) {
 // The step after a round of C candidates: the square root damps it against the count's noise,
 // and it at most doubles, since a round with too many candidates for the list is lost (2^20
 // clustered points, 16384 picks: 205 rounds and 2118 us where it could grow fourfold and doubled
-// after a round without candidates too, 196 and 2035 so).
+// after every round without candidates too, 196 and 2035 so).
 FPSX_BOUND uint64_t next_step(uint64_t step, uint32_t target, uint32_t C) {
   double r = sqrt((double)target / (double)C);
   r = r > 2.0 ? 2.0 : r;
@@ -40,8 +40,7 @@ FPSX_BOUND uint64_t next_step(uint64_t step, uint32_t target, uint32_t C) {
   return ns < 1.0 ? 1 : (ns > 4.0e18 ? (uint64_t)1 << 61 : (uint64_t)ns);
 }
 
-// The step after a round of C candidates that were too many: from an exact bound every step has
-// a candidate, and halving ends at the best point alone.
+// The step after a round of C candidates that were too many.
 FPSX_BOUND uint64_t less_step(uint64_t step, uint32_t target, uint32_t C) {
   const uint64_t ns = (uint64_t)((double)step * sqrt((double)target / (double)C));
   return ns < 1 ? 1 : ns;

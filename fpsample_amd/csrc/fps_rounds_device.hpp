@@ -78,7 +78,7 @@ struct RoundsCounts {
 
 // The exchange of round e: own candidates (keys lk, coordinates lc) out, everybody's into ck and
 // cc in any order.  On return C is the number of all (more than LIST where they do not fit) and,
-// where it is 0, U the best key of all.  False when something did not arrive in time.  Entered
+// where it is that or 0, U the best key of all.  False when something did not arrive in time.  Entered
 // and left by all waves, with a barrier before it is left.
 // L lanes read one workgroup's header and its first L candidates at once, so most candidates
 // are here as soon as their header is; those beyond L follow, a memory round trip later (64
@@ -200,8 +200,8 @@ __device__ __forceinline__ bool rounds_exchange(uint64_t *xchg, uint64_t spin_ti
   C = S.sum[par];
   const uint32_t got = S.at[par];
   if (got != C || C > (uint32_t)LIST) C = max(C, (uint32_t)LIST + 1);  // some did not fit
-  if (C == 0) {
-    // Nobody has a candidate: the best key of all, read only now, is the exact bound.
+  if (C == 0 || C > (uint32_t)LIST) {
+    // No candidates to decide on: the best key of all, read only now, is the pick.
     uint64_t u = 0;
     for (uint32_t i = (uint32_t)tid; i < G; i += kRoundsThreads) {
       const uint64_t *h = buf + ((size_t)(g % kRoundsReplicas) * kRoundsHeadWords + 1) * hp + i;

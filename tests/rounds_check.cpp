@@ -72,7 +72,7 @@ static std::vector<uint32_t> rounds(const Cloud &c, uint32_t m, uint32_t start, 
   uint32_t end = std::min(m, 1 + part);
   bool stuck = false;
   uint64_t last = ~0ull;
-  int idle = 0;
+  bool empty = false;
   for (;;) {
     if (out.size() >= m) return out;
     const bool cut = out.size() >= end;
@@ -102,15 +102,22 @@ static std::vector<uint32_t> rounds(const Cloud &c, uint32_t m, uint32_t start, 
     }
     const uint32_t C = (uint32_t)ck.size();
     if (C == 0 || C > list) {
-      if (++idle > 1024) return {};
+      // the best point alone
+      const uint32_t i = lowest ? ~(uint32_t)U : (uint32_t)U;
+      stuck = !(sqdist(c, i, i) < dm[i]);
+      out.push_back(i);
+      np.push_back(i);
+      last = U;
       if (C)
         step = fpsx::less_step(step, target, C);
-      else
-        T = U;
+      else if (empty)
+        step = fpsx::next_step(step, target, 1);
+      empty = C == 0;
+      T = U;
       Tg = fpsx::round_bound(T, step);
       continue;
     }
-    idle = 0;
+    empty = false;
     std::sort(ck.rbegin(), ck.rend());
     const uint32_t F = std::min(C, cap);
     uint64_t te = C > cap ? ck[cap].first : 0;
