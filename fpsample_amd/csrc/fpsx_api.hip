@@ -524,17 +524,26 @@ static const Plan *tuned_rounds(Ctx &c, size_t n, size_t dim, int tie) {
   return it != c.tuned.end() && it->second.kind == PlanKind::Rounds ? &it->second : nullptr;
 }
 
-// Threshold rounds from 512 points and 192 picks (64 beyond three dimensions), unless a pass
-// plan is asked for by name or by the tuner: the first picks come one or two a round, at 5 to
-// 10 us, where a pass takes 0.6 to 3 us.  Passes against rounds, us a call: 512 points / 128
+// Threshold rounds from 512 points and 192 picks (64 beyond three dimensions, but 112 where a
+// pass takes one workgroup, in up to eight dimensions and 8192 points), unless a pass plan is
+// asked for by name or by the tuner: the first picks come one or two a round, at 5 to 10 us,
+// where a pass takes 0.6 to 3 us.  Passes against rounds, us a call: 512 points / 128
 // picks 88 and 85, 1024 / 128 96 and 121, 1024 / 256 181 and 151, 4096 / 128 122 and 136,
 // 4096 / 512 452 and 236, 65536 / 64 146 and 214, 65536 / 256 555 and 334, 2^20 / 256 847
 // and 686; eight dimensions, 4096 / 64 106 and 120, 65536 / 64 207 and 165, 2^20 / 64 456
-// and 251.
+// and 251.  Rounds by passes, the mean of uniform, spherical and normal clouds: 2500 points in
+// four dimensions 1.27, 1.10, 1.09, 1.02 and 0.93 at 64, 80, 96, 112 and 128 picks, in eight 1.01,
+// 0.95 and 0.85 at 64, 80 and 96, 1500 in six 1.08 and 0.97 at 64 and 112; 512 and 20000 points at
+// 64 picks 0.99 and 0.94 in four, 0.90 and 0.78 in six.
+static bool rounds_serve(size_t n, size_t dim, size_t m) {
+  const size_t least = dim <= 3 ? 192 : dim <= 8 && n > 512 && n <= 8192 ? 112 : 64;
+  return n >= 512 && m >= least;
+}
+
 int plan_call(Ctx &c, size_t n, size_t dim, int tie, size_t m, Plan &p) {
   const Plan *shape = tuned_rounds(c, n, dim, tie);
-  const bool serves = n >= 512 && m >= (dim <= 3 ? 192u : 64u);
-  if (!passes_asked(c, n, dim, tie) && (env_set("FPSX_ROUNDS") || serves || shape) &&
+  if (!passes_asked(c, n, dim, tie) &&
+      (env_set("FPSX_ROUNDS") || rounds_serve(n, dim, m) || shape) &&
       plan_rounds(c, n, dim, tie, m, p, shape ? shape->k->ppt : 0,
                   shape ? (int)shape->grid : 0) == FPSX_OK)
     return FPSX_OK;

@@ -77,3 +77,17 @@ def test_batch_tuner_skips_rounds_that_gave_up(gpu):
     for i, (g, pc, m) in enumerate(zip(b.picks(), clouds, ms)):
         np.testing.assert_array_equal(g, O.fps(pc, m, 0), err_msg=f"cloud {i}")
     b.close()
+
+
+@pytest.mark.parametrize("n,d,m,rounds", [
+    (511, 3, 192, False), (512, 3, 191, False), (512, 3, 192, True), (512, 4, 63, False),
+    (512, 4, 64, True), (513, 4, 111, False), (513, 8, 112, True), (8192, 6, 111, False),
+    (8192, 6, 112, True), (8193, 6, 64, True), (600, 9, 63, False), (600, 9, 64, True)])
+def test_which_calls_run_in_rounds(gpu, n, d, m, rounds):
+    # Both sides of each line of the rule: what runs, and its picks.
+    import fpsample_amd as F
+    from fpsample_amd import device as D
+
+    assert (D.call_info(n, d, n_samples=m)["kind"] == "rounds") is rounds
+    pc = np.random.default_rng(n + d).random((n, d)).astype(np.float32)
+    np.testing.assert_array_equal(F.fps_sampling(pc, m, start_idx=5), O.fps(pc, m, 5))
