@@ -542,6 +542,23 @@ static int batch_prepare_kernel(fpsx_batch *b, const KernelEntry *k, bool pruned
   return b->run.prepare(*b->ctx, k, jobs, mj, areas, b->d_pts, b->d_out, nullptr);
 }
 
+// An internal flag of fpsx_batch_create: the batch is run once.
+constexpr int kBatchOnce = 1 << 16;
+
+// Whether the pass kernels run a 3-D batch faster: the first picks of a cloud come one or two a
+// round.  Passes and rounds, us a run: 512 clouds of 1000 points 72 and 107 at 8 picks, 134 and
+// 157 at 32, 218 and 194 at 64; 64 of 16000 124 and 168 at 32, 180 and 205 at 64; 64 of 60000 358
+// and 439 at 64, 585 and 519 at 128.  Run once, with the order made for it, rounds are ahead from
+// 32 picks too (8 clouds of 16000 from host memory 1097 and 917).
+static bool few_picks(const std::vector<JobSpec> &specs) {
+  uint32_t m = 0, n = 0;
+  for (auto &s : specs) {
+    m = std::max(m, s.m);
+    n = std::max(n, s.n);
+  }
+  return m < (n > 8192 ? 96u : 64u);
+}
+
 FPSX_EXPORT int fpsx_batch_create(const float *d_points, size_t ld, size_t dim,
                                   const uint64_t *offsets, size_t n_clouds,
                                   const uint64_t *n_samples, const uint64_t *start_idx,
@@ -583,6 +600,7 @@ FPSX_EXPORT int fpsx_batch_create(const float *d_points, size_t ld, size_t dim,
     const char *v = std::getenv(name);
     if (v && *v && std::strcmp(v, "0") != 0) rounds = false;
   }
+  if (dim == 3 && !(flags & (FPSX_BATCH_AUTOTUNE | kBatchOnce)) && few_picks(b->specs)) rounds = false;
   float rounds_ms = 1e30f;
   if (rounds) {
     rc = batch_prepare_rounds(b.get());
@@ -820,7 +838,7 @@ FPSX_EXPORT int fpsx_fps_batch(const float *points, size_t dim, const uint64_t *
   }
   fpsx_batch *b = nullptr;
   rc = fpsx_batch_create((const float *)soa.p, total, dim, offsets, n_clouds, n_samples, start_idx,
-                         (uint64_t *)dout.p, 0, &b);
+                         (uint64_t *)dout.p, kBatchOnce, &b);
   if (rc == FPSX_OK) rc = fpsx_batch_run(b, nullptr);
   if (rc == FPSX_OK) rc = fpsx_batch_status(b, nullptr);
   if (rc == FPSX_OK) {

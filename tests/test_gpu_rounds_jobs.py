@@ -47,3 +47,24 @@ def test_status_before_the_first_run(gpu, monkeypatch, d, passes):
         b = DeviceBatch(clouds, [500, 100], [0, 0], graph=False)
         b.status()
         b.close()
+
+
+@pytest.mark.parametrize("n,m,rounds", [(5000, 63, False), (5000, 64, True), (8193, 95, False),
+                                        (8193, 96, True), (300, 8, False)])
+def test_batches_of_few_picks(gpu, n, m, rounds):
+    # Both sides of the line below which 3-D batches take the pass kernels (8 points a thread).
+    import fpsample_amd as F
+    from fpsample_amd.batch import DeviceBatch
+
+    rng = np.random.default_rng(n + m)
+    clouds = [rng.random((k, 3)).astype(np.float32) for k in (n, 200, n // 2)]
+    ms = [m, 7, m // 2]
+    want = [O.fps(pc, k, 1) for pc, k in zip(clouds, ms)]
+    b = DeviceBatch(clouds, ms, [1, 1, 1])
+    assert b.info()["ppt"] == (4 if rounds else 8)
+    b.run()
+    b.status()
+    for g, o, w in zip(b.picks(), F.fps_sampling_batch(clouds, ms, 1), want):
+        np.testing.assert_array_equal(g, w)
+        np.testing.assert_array_equal(o, w)
+    b.close()
