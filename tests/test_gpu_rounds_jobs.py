@@ -68,3 +68,54 @@ def test_batches_of_few_picks(gpu, n, m, rounds):
         np.testing.assert_array_equal(g, w)
         np.testing.assert_array_equal(o, w)
     b.close()
+
+
+def special_clouds():
+    """NaN, infinite and overflowing coordinates, and clouds whose last points are at distance 0,
+    so that a run ends on one point taken again and again."""
+    rng = np.random.default_rng(22)
+    for n in (200, 3000, 40_000):
+        sp = (rng.random((n, 3)) * 4e19).astype(np.float32)
+        sp[9] = np.inf
+        sp[10, 1] = -np.inf
+        yield sp, min(n, 300), 0
+        sp = sp.copy()
+        sp[[5, 70, n - 1]] = np.nan
+        yield sp, min(n, 300), 3
+        yield (rng.random((n, 3)) * 1e-21).astype(np.float32), min(n, 400), 1
+        yield np.ones((n, 3), np.float32), 77, n // 2
+        yield rng.integers(0, 4, (n, 3)).astype(np.float32), min(n, 103), 2  # 64 places
+        yield rng.integers(0, 30, (n, 3)).astype(np.float32), min(n, 1500), 2
+
+
+@pytest.mark.parametrize("chunk", [5, 64, 1 << 20])
+def test_special_values_on_the_serving_loop(gpu, chunk):
+    # In one part and in many: a run may end on one point in the middle of a part.
+    from fpsample_amd.serve import Server
+
+    clouds = list(special_clouds())
+    print(f"special values, serving loop, {chunk} picks a launch", flush=True)
+    with Server(hbm_budget_bytes=128 << 20, chunk_passes=chunk) as srv:
+        ids = [srv.submit(pc, m, s) for pc, m, s in clouds]
+        outs = [srv.wait(r)[0] for r in ids]
+    for i, (g, (pc, m, s)) in enumerate(zip(outs, clouds)):
+        np.testing.assert_array_equal(g, O.fps(pc, m, s), err_msg=f"request {i} n={len(pc)} m={m}")
+
+
+def test_special_values_in_a_batch(gpu):
+    # With enough small clouds beside them that the large ones get one workgroup each and keep
+    # their min-distances in memory, and alone, as teams.
+    from fpsample_amd.batch import DeviceBatch
+
+    special = list(special_clouds())
+    rng = np.random.default_rng(23)
+    many = special + [(rng.random((9000, 3)).astype(np.float32), 900, 0) for _ in range(400)]
+    for name, work in (("teams", special), ("one workgroup each", many)):
+        print(f"special values, batch, {name}", flush=True)
+        b = DeviceBatch([w[0] for w in work], [w[1] for w in work], [w[2] for w in work])
+        assert b.info()["ppt"] == 4
+        b.run()
+        b.status()
+        for i, (g, (pc, m, s)) in enumerate(zip(b.picks(), work)):
+            np.testing.assert_array_equal(g, O.fps(pc, m, s), err_msg=f"{name} cloud {i} n={len(pc)}")
+        b.close()
