@@ -3,10 +3,9 @@
 
 A step is one vanilla FPS run (fps_sampling semantics, src/lib.cpp:188-246)
 over one synthetic cloud already resident in HBM: one call of
-fpsx_fps_sampling_device, i.e. the exchange-area clear, for large 3-D clouds
-the spatial ordering of the points (bounding box, Hilbert codes, two radix
-sorts, gather), and the single persistent FPS launch that makes all M-1
-passes.  The kernel shape comes from the library's planner; --autotune on
+fpsx_fps_sampling_device, i.e. the exchange-area clear, for long runs the
+spatial ordering of the points (bounding box, count, scatter and sort by
+Hilbert codes), and the single persistent FPS launch that takes all M picks.  The kernel shape comes from the library's planner; --autotune on
 times every plan first (untimed) instead.  The npdu* workloads time
 fps_npdu_sampling (src/lib.cpp:272-340) the same way, through
 fpsx_fps_npdu_sampling_device on row-major device data.  The kdline*
@@ -29,8 +28,8 @@ start_idx = 0.  The same JSON line then carries the metric's second half:
 
 Prints one JSON line.  value = samples/s of the whole job (M x steps / wall
 time between two device synchronisations).  roofline: what bounds the
-kernel.  Multi-workgroup resident and pruned kernels are bound by the
-latency of their per-pass cross-workgroup exchange, not by HBM: the line
+kernel.  Multi-workgroup kernels are bound by the latency of their rounds or
+passes, each with a cross-workgroup exchange, not by HBM: the line
 reports exchanges per second against what the exchange alone sustains at
 the same grid and candidate size (fpsx_probe_exchange, measured in the same
 run), plus the measured HBM traffic and LDS bytes (committed rocprofv3
@@ -452,9 +451,9 @@ def roofline(workload: str, plan: dict, n: int, m: int, kernel_s: float, npdu: b
                us_per_exchange=round(kernel_s * 1e6 / exchanges, 4),
                floor_probe={"grid": grid, "words": words, "threads": 1024})
     if kind == "rounds":
-        out["note"] = ("threshold rounds: one exchange settles many picks, and a round's own work (the "
-                       "update, sorting the candidates, deciding the picks) takes longer than the "
-                       "exchange that the floor counts")
+        out["note"] = ("threshold rounds: one exchange settles many picks; the floor is an exchange of five "
+                       "words a workgroup, less than a round's headers and candidates, and a round's own "
+                       "work (the update, sorting the candidates, deciding the picks) takes longer")
         out["picks_per_exchange"] = round(m / exchanges, 1)
     if kind in ("spruned", "spair"):
         out["note"] = ("the floor is the exchange alone; a streamed round also waits for the memory "
@@ -652,7 +651,7 @@ def run_serve(args) -> dict:
         "metric": "p50/p99 latency, mixed FPS stream",
         "config": {"workload": "96 requests, N log-uniform [2^10, 2^20], uniform cube, "
                                "M = N*U{1/8,1/4,1/2}, start_idx=0, HBM budget 16 GiB, "
-                               f"{args.serve_chunk}-pass chunks, batch kernel 1024 x 16",
+                               f"{args.serve_chunk}-pass chunks, threshold rounds",
                    "total_samples": total_m, "qps": round(qps, 3)},
         "p50_ms": round(float(np.percentile(lat, 50)), 3),
         "p99_ms": round(float(np.percentile(lat, 99)), 3),
