@@ -20,8 +20,8 @@
 // of equal distances.
 //
 // What bounds it: a round's serial chain, not bytes (2^20 clustered points, 16384 picks, 128
-// workgroups: 181 rounds of 11 us, the paired pass kernel 8203 exchanges of 3.4 us).  Of a
-// round (50 K points, 64 workgroups, 65 rounds of 9.7 us): update 2.2 us with the wait for the
+// workgroups: 165 rounds of 11.6 us, the paired pass kernel 8203 exchanges of 3.4 us).  Of a
+// round (50 K points, 64 workgroups, 64 rounds of 9.7 us): update 2.2 us with the wait for the
 // slowest wave, exchange 3.0, sorting 0.9, rows 1.4, settling 0.4, the bound and the picks 0.6.
 // Settling the candidates one by one instead took 450 ns a pick.  A block per wave in
 // registers, the candidates loaded beside the headers and the best 256 taken from up to 512

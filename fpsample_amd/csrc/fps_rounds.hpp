@@ -60,8 +60,8 @@ constexpr uint32_t kRoundsReplicas = 4;    // copies of the headers
 inline uint32_t rounds_target(size_t m) {
   return m >= 16384 ? 224 : m >= 1280 ? 160 : m <= 512 ? 64 : (uint32_t)(m / 8);
 }
-// Candidates one workgroup may publish: a round in which one has more is lost, which clustered
-// clouds do to small limits, and larger areas cost their clearing and the candidates' way (us a
+// Candidates one workgroup may publish: a round in which one has more takes one pick, as clustered
+// clouds do with small limits, and larger areas cost their clearing and the candidates' way (us a
 // run and rounds at 64 / 32 for up to 64 and more workgroups, at 128 / 64 and at 256 / 128: 2^24
 // lattice points, 2048 picks 3608 (220), 3321 (168), 3305 (147); 2^20 clustered points, 16384
 // picks 2035 (196), 1989 (181), 2027 (171); 2^22 / 4096 1999, 1983, 2040).

@@ -30,7 +30,7 @@ FPSX_BOUND uint64_t round_bound(uint64_t T, uint64_t step) {
 }
 
 // The step after a round of C candidates: the square root damps it against the count's noise,
-// and it at most doubles, since a round with too many candidates for the list is lost (2^20
+// and it at most doubles, since a round with too many candidates for the list takes one pick (2^20
 // clustered points, 16384 picks: 205 rounds and 2118 us where it could grow fourfold and doubled
 // after every round without candidates too, 196 and 2035 so).
 FPSX_BOUND uint64_t next_step(uint64_t step, uint32_t target, uint32_t C) {
